@@ -69,6 +69,7 @@ struct SweepArgs {
   int p_lo, p_hi;       // pencils swept (the third index)
   int w_ilo, w_ihi, w_plo, w_phi;  // cells written to the output (plus s in 1..m)
   int H, nrb, npencil, nistrips;
+  int inplace;          // qin == qout: a workgroup holds all the runs of its strip
   const T* qin;
   T* qout;
   const T* comp_in;
@@ -212,17 +213,34 @@ __device__ __forceinline__ long long cell_off(const Geom& g, int i, int s, int p
   return (long long)(i - 1 + g.g) + (long long)(j - 1 + g.g) * g.rs + (long long)(k - 1 + g.g) * g.ss;
 }
 
+// A wavefront marches H rows of a 64-column strip of one pencil plane.  The next
+// row is loaded one iteration before its use, the compensation of the row being
+// stored at the top of its iteration.
+//
+// In place (a.inplace, the 3D y-sweep), the 4 wavefronts of a workgroup take the
+// 4 consecutive runs of rows of the same strip: each reads the two rows past its
+// run (the next run's, which that wavefront overwrites) and the two before it
+// ahead of the workgroup's barrier, so nobody reads a row already swept.  One
+// wavefront a pencil left 768 of them on 1024 SIMDs at 210x170x190.  With the
+// runs, the row loaded ahead and one Courant-number atomic per workgroup the
+// split step takes 1.04 instead of 1.33 ms there (FP64) and 4.13 instead of
+// 5.24 ms at 384^3 (FP32 + Kahan).
 template <class RS, typename T, bool KAHAN, int AXIS, bool HALF_IN_SUM>
 __global__ void __launch_bounds__(256) k_march(const SweepArgs<T> a) {
   constexpr int ME = RS::meqn, MW = RS::mwaves;
   constexpr int IXY = AXIS;   // Riemann direction: 2 = y, 3 = z
   using Roe = typename RS::Roe;
   const int lane = threadIdx.x & 63;
-  const int wid = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  if (wid >= a.nistrips * a.npencil * a.nrb) return;
+  const int wave = threadIdx.x >> 6;
+  const bool inplace = a.inplace;
+  // out of place: wavefronts run over (strip, pencil, run); in place: workgroups
+  // over (strip, pencil), their wavefronts over the runs.  Wavefronts past the
+  // last run do no work but reach the workgroup's barriers.
+  const int wid = inplace ? (int)blockIdx.x : (int)(blockIdx.x * (blockDim.x >> 6)) + wave;
   const int istrip = wid % a.nistrips;
   const int rest = wid / a.nistrips;
-  const int pidx = rest % a.npencil, rb = rest / a.npencil;
+  const int pidx = rest % a.npencil, rb = inplace ? wave : rest / a.npencil;
+  const bool run = rb < a.nrb;   // uniform per wavefront
   const int i = a.i_lo + istrip * 64 + lane;
   const int p = a.p_lo + pidx;
   const bool live = i <= a.i_hi;
@@ -252,114 +270,160 @@ __global__ void __launch_bounds__(256) k_march(const SweepArgs<T> a) {
   };
 
   T Qm[ME], Q0[ME], Q1[ME], Am[MA], A0[MA], A1[MA];
-  load(j0 - 2, Qm);
-  load(j0 - 1, Q0);
-  load(j0, Q1);
-  load_aux(j0 - 2, Am);
-  load_aux(j0 - 1, A0);
-  load_aux(j0, A1);
-  T Wt[MW][ME], st[MW], amt[ME], apt[ME], dotl[MW];
-  Roe roet;
-  {
-    T Wp[MW][ME], sp[MW], amp[ME], app[ME];
-    Roe roep;
-    rpn_call<RS, IXY>(a.rp, Qm, Q0, Am, A0, Wp, sp, amp, app, roep);
-    if (j0 - 1 >= 1) {
-#pragma unroll
-      for (int w = 0; w < MW; w++) smax = cfl_term(smax, fabs(sp[w]));
-    }
-    rpn_call<RS, IXY>(a.rp, Q0, Q1, A0, A1, Wt, st, amt, apt, roet);
-#pragma unroll
-    for (int w = 0; w < MW; w++) smax = cfl_term(smax, fabs(st[w]));
-    wave_dots<ME, MW>(Wp, Wt, dotl);
+  T Qn[ME];            // row t+1 of the coming iteration, loaded one ahead
+  T U0[ME], U1[ME];    // in place: rows jend and jend+1 as they were
+  if (run) {
+    load(j0 - 2, Qm);
+    load(j0 - 1, Q0);
+    load(j0, Q1);
+    load(j0 + 1, Qn);
   }
-  T qold_prev[ME], qadd_p[ME], F_p[ME];
+  if (inplace) {   // uniform over the launch
+    if (run) {
+      load(jend, U0);
+      load(jend + 1, U1);
+      // the values are in registers (not merely on their way) before the barrier
 #pragma unroll
-  for (int m = 0; m < ME; m++) { Q0[m] = Q1[m]; qold_prev[m] = T(0); qadd_p[m] = T(0); F_p[m] = T(0); }
-#pragma unroll
-  for (int m = 0; m < MA; m++) A0[m] = A1[m];
-
-  for (int t = j0; t <= jend; t++) {
-    load(t + 1, Q1);
-    load_aux(t + 1, A1);
-    T Wn[MW][ME], sn[MW], amn[ME], apn[ME], dotn[MW];
-    Roe roen;
-    rpn_call<RS, IXY>(a.rp, Q0, Q1, A0, A1, Wn, sn, amn, apn, roen);
-    if (t + 1 <= m_ax + 1) {
-#pragma unroll
-      for (int w = 0; w < MW; w++) smax = cfl_term(smax, fabs(sn[w]));
+      for (int m = 0; m < ME; m++)
+        asm volatile("" : "+v"(Qm[m]), "+v"(Q0[m]), "+v"(Q1[m]), "+v"(Qn[m]), "+v"(U0[m]),
+                          "+v"(U1[m]));
     }
-    T F[ME];
+    __syncthreads();
+  }
+  if (run) {
+    load_aux(j0 - 2, Am);
+    load_aux(j0 - 1, A0);
+    load_aux(j0, A1);
+    T Wt[MW][ME], st[MW], amt[ME], apt[ME], dotl[MW];
+    Roe roet;
+    {
+      T Wp[MW][ME], sp[MW], amp[ME], app[ME];
+      Roe roep;
+      rpn_call<RS, IXY>(a.rp, Qm, Q0, Am, A0, Wp, sp, amp, app, roep);
+      if (j0 - 1 >= 1) {
 #pragma unroll
-    for (int m = 0; m < ME; m++) F[m] = T(0);
-#pragma unroll
-    for (int w = 0; w < MW; w++) dotn[w] = T(0);
-    if (a.order != 1) {
-      wave_dots<ME, MW>(Wt, Wn, dotn);
-      limit_waves<ME, MW>(Wt, st, dotl, dotn, a.mthlim);
-      corr_flux<ME, MW, HALF_IN_SUM>(Wt, st, dtdx, F, a.rp.fwave);
-    }
-    if (t > j0 && wcol) {
-      // cell t-1: apdq of interface t-1 (carried), amdq of interface t
-      const int s = t - 1;
-      T* po = a.qout + cell_off<AXIS>(a.gout, ic, s, p);
-      if (KAHAN) {
-        const T* pci = a.comp_in + cell_off<AXIS>(a.gin, ic, s, p);
-        T* pco = a.comp_out + cell_off<AXIS>(a.gout, ic, s, p);
-#pragma unroll
-        for (int m = 0; m < ME; m++) {
-          T qadd = qadd_p[m] - dtdx * amt[m];
-          T d = qadd - dtdx * (F[m] - F_p[m]);
-          T y = d - pci[(long long)m * a.gin.fs];
-          T tq = qold_prev[m] + y;
-          pco[(long long)m * a.gout.fs] = (tq - qold_prev[m]) - y;
-          po[(long long)m * a.gout.fs] = tq;
-        }
-      } else {
-#pragma unroll
-        for (int m = 0; m < ME; m++) {
-          T qadd = qadd_p[m] - dtdx * amt[m];
-          po[(long long)m * a.gout.fs] = (qold_prev[m] + qadd) - dtdx * (F[m] - F_p[m]);
-        }
+        for (int w = 0; w < MW; w++) smax = cfl_term(smax, fabs(sp[w]));
       }
-    }
+      rpn_call<RS, IXY>(a.rp, Q0, Q1, A0, A1, Wt, st, amt, apt, roet);
 #pragma unroll
-    for (int m = 0; m < ME; m++) {
-      qadd_p[m] = T(0) - dtdx * apt[m];
-      F_p[m] = F[m];
-      amt[m] = amn[m];
-      apt[m] = apn[m];
-      qold_prev[m] = Q0[m];
-      Q0[m] = Q1[m];
+      for (int w = 0; w < MW; w++) smax = cfl_term(smax, fabs(st[w]));
+      wave_dots<ME, MW>(Wp, Wt, dotl);
     }
+    T qold_prev[ME], qadd_p[ME], F_p[ME];
+#pragma unroll
+    for (int m = 0; m < ME; m++) { Q0[m] = Q1[m]; qold_prev[m] = T(0); qadd_p[m] = T(0); F_p[m] = T(0); }
 #pragma unroll
     for (int m = 0; m < MA; m++) A0[m] = A1[m];
+
+    for (int t = j0; t <= jend; t++) {
 #pragma unroll
-    for (int w = 0; w < MW; w++) {
-      st[w] = sn[w];
-      dotl[w] = dotn[w];
+      for (int m = 0; m < ME; m++) Q1[m] = Qn[m];
+      if (inplace && t + 2 >= jend) {   // rows jend, jend+1 belong to the next run
 #pragma unroll
-      for (int m = 0; m < ME; m++) Wt[w][m] = Wn[w][m];
+        for (int m = 0; m < ME; m++) Qn[m] = t + 2 == jend ? U0[m] : U1[m];
+      } else if (t < jend) {
+        load(t + 2, Qn);
+      }
+      T ci[ME];
+      const bool store = t > j0 && wcol;
+      if (KAHAN && store) {
+        const T* pci = a.comp_in + cell_off<AXIS>(a.gin, ic, t - 1, p);
+#pragma unroll
+        for (int m = 0; m < ME; m++) ci[m] = pci[(long long)m * a.gin.fs];
+      }
+      load_aux(t + 1, A1);
+      T Wn[MW][ME], sn[MW], amn[ME], apn[ME], dotn[MW];
+      Roe roen;
+      rpn_call<RS, IXY>(a.rp, Q0, Q1, A0, A1, Wn, sn, amn, apn, roen);
+      if (t + 1 <= m_ax + 1) {
+#pragma unroll
+        for (int w = 0; w < MW; w++) smax = cfl_term(smax, fabs(sn[w]));
+      }
+      T F[ME];
+#pragma unroll
+      for (int m = 0; m < ME; m++) F[m] = T(0);
+#pragma unroll
+      for (int w = 0; w < MW; w++) dotn[w] = T(0);
+      if (a.order != 1) {
+        wave_dots<ME, MW>(Wt, Wn, dotn);
+        limit_waves<ME, MW>(Wt, st, dotl, dotn, a.mthlim);
+        corr_flux<ME, MW, HALF_IN_SUM>(Wt, st, dtdx, F, a.rp.fwave);
+      }
+      if (store) {
+        // cell t-1: apdq of interface t-1 (carried), amdq of interface t
+        const int s = t - 1;
+        T* po = a.qout + cell_off<AXIS>(a.gout, ic, s, p);
+        if (KAHAN) {
+          T* pco = a.comp_out + cell_off<AXIS>(a.gout, ic, s, p);
+#pragma unroll
+          for (int m = 0; m < ME; m++) {
+            T qadd = qadd_p[m] - dtdx * amt[m];
+            T d = qadd - dtdx * (F[m] - F_p[m]);
+            T y = d - ci[m];
+            T tq = qold_prev[m] + y;
+            pco[(long long)m * a.gout.fs] = (tq - qold_prev[m]) - y;
+            po[(long long)m * a.gout.fs] = tq;
+          }
+        } else {
+#pragma unroll
+          for (int m = 0; m < ME; m++) {
+            T qadd = qadd_p[m] - dtdx * amt[m];
+            po[(long long)m * a.gout.fs] = (qold_prev[m] + qadd) - dtdx * (F[m] - F_p[m]);
+          }
+        }
+      }
+#pragma unroll
+      for (int m = 0; m < ME; m++) {
+        qadd_p[m] = T(0) - dtdx * apt[m];
+        F_p[m] = F[m];
+        amt[m] = amn[m];
+        apt[m] = apn[m];
+        qold_prev[m] = Q0[m];
+        Q0[m] = Q1[m];
+      }
+#pragma unroll
+      for (int m = 0; m < MA; m++) A0[m] = A1[m];
+#pragma unroll
+      for (int w = 0; w < MW; w++) {
+        st[w] = sn[w];
+        dotl[w] = dotn[w];
+#pragma unroll
+        for (int m = 0; m < ME; m++) Wt[w][m] = Wn[w][m];
+      }
+      roet = roen;
     }
-    roet = roen;
   }
-  double cfl = live ? (double)a.dtdx * (double)smax : 0.0;
-  wave_atomic_max(cfl, a.cfl_bits);
+  block_atomic_max(run && live ? (double)a.dtdx * (double)smax : 0.0, a.cfl_bits);
 }
 
 // ---------------------------------------------------------------- launchers
 namespace {
-constexpr int kMarchRows = 32;
-
-// Rows per wavefront of an out-of-place y/z sweep: kMarchRows, or
-// CLAWHIP_SPLIT_ROWS (tuning sweeps).  In-place sweeps march whole pencils
-// (launch_march).
-int march_rows_split() {
+// Rows per wavefront of an out-of-place y/z sweep, or CLAWHIP_SPLIT_ROWS (tuning
+// sweeps).  A run of H rows solves H + 3 interfaces; with R wavefronts resident,
+// k rounds hold k * R / columns runs of a column of strips, and the k with the
+// smallest k * (H + 3) is taken (H >= 3; ties: the longer run).  A fixed 32 rows
+// left 128 wavefronts on 1024 SIMDs at 501x487: the FP64 shallow-water step there
+// takes 77 us with this rule, 134 us with the 32 rows.
+template <class Kernel>
+int march_rows_split(Kernel kernel, int per_simd, long long columns, int m_ax) {
   if (const char* env = getenv("CLAWHIP_SPLIT_ROWS")) {
     const int h = atoi(env);
     if (h >= 1 && h <= 65536) return h;
   }
-  return kMarchRows;
+  const long long resident = resident_waves((const void*)kernel, per_simd);
+  if (resident == 0) return 32;
+  long long best = m_ax, best_cost = -1;
+  for (long long k = (columns + resident - 1) / resident; best_cost < 0 || k * 6 < best_cost;
+       k++) {
+    const long long runs = k * resident / columns;
+    long long h = (m_ax + runs - 1) / runs;
+    if (h < 3) h = 3;
+    if (best_cost < 0 || k * (h + 3) < best_cost) {
+      best = h;
+      best_cost = k * (h + 3);
+    }
+  }
+  return (int)best;
 }
 
 template <typename T>
@@ -379,7 +443,7 @@ SweepArgs<T> base_args(const clawhip_rp& rp, const Geom& gin, const Geom& gout, 
   a.cfl_bits = cfl;
   a.nstrips = 0; a.xrows = 1; a.axis = 0; a.i_lo = a.i_hi = a.p_lo = a.p_hi = 0;
   a.w_ilo = a.w_ihi = a.w_plo = a.w_phi = 0;
-  a.H = march_rows_split(); a.nrb = a.npencil = a.nistrips = 0;
+  a.H = a.nrb = a.npencil = a.nistrips = a.inplace = 0;
   a.aux = nullptr;
   a.gaux = gout;
   a.bcaux = a.bc;
@@ -423,15 +487,23 @@ template <class RS, typename T, bool KAHAN, int AXIS, bool HALF>
 int launch_march(SweepArgs<T> a, hipStream_t stream) {
   const int m_ax = AXIS == 2 ? a.gin.my : a.gin.mz;
   a.axis = AXIS;
-  // An in-place sweep must march whole pencils: a block's halo rows would
-  // otherwise be rewritten by the next block of the same pencil.
-  if ((const void*)a.qin == (const void*)a.qout) a.H = m_ax;
   a.nistrips = (a.i_hi - a.i_lo + 1 + 63) / 64;
   a.npencil = a.p_hi - a.p_lo + 1;
-  a.nrb = (m_ax + a.H - 1) / a.H;
-  long long waves = (long long)a.nistrips * a.npencil * a.nrb;
-  hipLaunchKernelGGL((k_march<RS, T, KAHAN, AXIS, HALF>), dim3((unsigned)((waves + 3) / 4)),
-                     dim3(256), 0, stream, a);
+  a.inplace = (const void*)a.qin == (const void*)a.qout;
+  const long long columns = (long long)a.nistrips * a.npencil;
+  unsigned blocks;
+  if (a.inplace) {   // 4 runs of rows to a pencil, one workgroup
+    a.H = (m_ax + 3) / 4;
+    a.nrb = (m_ax + a.H - 1) / a.H;
+    blocks = (unsigned)columns;
+  } else {
+    // FP64 is bound by its issue from two wavefronts a SIMD on
+    a.H = march_rows_split(k_march<RS, T, KAHAN, AXIS, HALF>, sizeof(T) == 8 ? 2 : 0, columns,
+                           m_ax);
+    a.nrb = (m_ax + a.H - 1) / a.H;
+    blocks = (unsigned)((columns * a.nrb + 3) / 4);
+  }
+  hipLaunchKernelGGL((k_march<RS, T, KAHAN, AXIS, HALF>), dim3(blocks), dim3(256), 0, stream, a);
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : (int)e;
 }

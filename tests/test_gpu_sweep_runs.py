@@ -1,0 +1,71 @@
+"""The y and z sweeps of the dimension-split steps cut a pencil into runs of rows
+(classic_split.hip k_march): in place, four runs to a workgroup, each reading its
+neighbours' rows before they are rewritten; out of place, runs sized to fill the
+device.  Lengths around the runs' edges, bit for bit against the oracle's
+step2ds / step3ds (FP64)."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as O
+from tests._cases import seeded_state
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("my", [2, 3, 4, 5, 7, 8, 9, 16, 17, 33])
+def test_split3_runs_bit_exact(my):
+    from pyclaw_amd import kernels as K
+    from pyclaw_amd.device import q_from_device, q_to_device
+    mx, mz, ng = 67, my + 2, 2
+    print("split3 runs", (mx, my, mz), flush=True)
+    bcl, bcu = [1, 1, 1], [1, 1, 1]
+    q = seeded_state(np.random.default_rng(my), O.EULER3, (mx, my, mz))
+    meth = O.method_array(dimensional_split=True)
+    dx, dy, dz = 1.0 / mx, 0.9 / my, 1.1 / mz
+    dt = 0.2 * min(dx, dy, dz)
+    qbc = O.with_ghosts(q, ng)
+    O.bc3(qbc, ng, bcl, bcu)
+    qold = qbc.copy(order="F")
+    rp = O.make_rp(O.EULER3)
+    cs = [O.step3ds(rp, src, qbc, ng, dx, dy, dz, dt, meth, [4] * 3, k)
+          for k, src in ((1, qold), (2, qbc), (3, qbc))]
+    qi = q_to_device(q)
+    qo = torch.empty_like(qi)
+    cfl = torch.zeros(1, dtype=torch.float64, device="cuda")
+    K.step3_split(K.make_rp(5, {"gamma": 1.4}), qi, qo, cfl, bcl, bcu, [1, 2, 3], meth, [4] * 3,
+                  dx, dy, dz, dt)
+    torch.cuda.synchronize()
+    assert np.array_equal(q_from_device(qo), O.interior(qbc, ng))
+    assert float(cfl.item()) == max(cs)
+
+
+@pytest.mark.parametrize("mx,my", [(3, 2), (64, 2), (61, 3), (200, 37), (5, 130), (130, 1030)])
+def test_split2_runs_bit_exact(mx, my):
+    """Both forms of the 2D y sweep: out of place, and in place on a whole qbc."""
+    from pyclaw_amd import kernels as K
+    from pyclaw_amd.device import q_from_device, q_to_device
+    ng, bcl, bcu = 2, [1, 1], [1, 1]
+    print("split2 runs", (mx, my), flush=True)
+    q = seeded_state(np.random.default_rng(mx + my), O.SHALLOW, (mx, my))
+    meth = O.method_array(dimensional_split=True)
+    dx, dy = 1.0 / mx, 0.8 / my
+    dt = 0.2 * min(dx, dy)
+    qbc = O.with_ghosts(q, ng)
+    O.bc2(qbc, ng, bcl, bcu)
+    start = qbc.copy(order="F")
+    ref = qbc.copy(order="F")
+    rp = O.make_rp(O.SHALLOW)
+    c = max(O.step2(rp, qbc, ref, ng, dx, dy, dt, meth, [4] * 3, ids=1),
+            O.step2(rp, ref.copy(order="F"), ref, ng, dx, dy, dt, meth, [4] * 3, ids=2))
+    krp = K.make_rp(3, {"grav": 1.0})
+    for whole in (False, True):
+        qi = q_to_device(start if whole else q)
+        qo = torch.empty_like(qi)
+        cfl = torch.zeros(1, dtype=torch.float64, device="cuda")
+        codes = ([4, 4], [4, 4]) if whole else (bcl, bcu)
+        K.step2_split(krp, qi, qo, cfl, *codes, [1, 2], meth, [4] * 3, dx, dy, dt, whole=whole)
+        torch.cuda.synchronize()
+        out = q_from_device(qo)
+        assert np.array_equal(O.interior(out, ng) if whole else out, O.interior(ref, ng))
+        assert float(cfl.item()) == c
