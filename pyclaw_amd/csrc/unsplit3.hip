@@ -5,19 +5,26 @@
 // around it: 9 x-slices (k outer, j inner), 9 y-slices (k outer, i inner), 9
 // z-slices (j outer, i inner) (step3.f90:120-580).  Every slice reads the old
 // state, so the slices are independent; the order only matters for the sums.
-// Two kernels per step:
-//   k_flux3<DIR> (one per direction): for every slice of that direction, the
-//     flux3 results of each cell along it -- qadd, fadd at its left interface,
-//     and the transverse modifications gadd(m, 1:2, -1:1) and hadd -- into a
-//     work array; one wavefront per 64-cell strip of a slice, lane l at cell
-//     c = base + l, neighbours' values by DPP lane shifts as in the split sweeps.
-//   k_apply3: one thread per cell, qnew = qold plus the 27 slices' terms in the
-//     reference's order and parenthesisation (bitwise equal to the oracle, whose
-//     step3 equals the reference's own Fortran on every qbc cell).
-// Work: 14 * meqn doubles per cell and direction.  Bound: HBM, by the work
-// array's write and its 27-fold gather (about 3.4 KB per cell-step for
-// euler_3D against 80 B algorithmic); the path exists for parity with
-// ClawSolver3D's unsplit default, the split step is the fast 3D path.
+// Two kernels per direction:
+//   k_flux3<DIR>: for every slice of that direction, the flux3 results of each
+//     cell along it -- qadd, fadd at its left interface, and the transverse
+//     modifications gadd(m, 1:2, -1:1) and hadd -- into a work array.  The
+//     slices' cells with their ghosts (n + 4 each) are laid end to end and a
+//     wavefront takes 64 consecutive ones and owns the middle 60, so a slice
+//     of any length fills the lanes (one strip a slice left 47 % of them idle
+//     at n = 64); neighbours' values by DPP lane shifts as in the split sweeps.
+//   k_apply3<DIR>: adds a direction's 9 slices to each cell, in the reference's
+//     order and parenthesisation (bitwise equal to the oracle, whose step3 equals
+//     the reference's own Fortran on every qbc cell).  A pass per direction lets
+//     the lanes run along the slices, as the work array is laid out: with lanes
+//     along x throughout, the y- and z-slices' 270 of a cell's 405 loads per
+//     field touched a cache line each: at 96x64x80 one such pass took 1.23 ms,
+//     the three take 0.28, and the step 0.73 instead of 1.86 ms (k_flux3
+//     0.60 -> 0.42).
+// Work: 14 * meqn doubles per cell and direction; x, then y, then z use the same
+// array, so that a direction's results are read while they are cached.  Bound:
+// HBM, by the work array's write and its 27-fold gather; the path exists for
+// parity with ClawSolver3D's unsplit default, the split step is the fast 3D path.
 #include <type_traits>
 
 #include "launch.hpp"
@@ -34,9 +41,10 @@ struct Step3Args {
   T dtdx, dtdy, dtdz;
   const T* qin;
   T* qout;           // compact output (k_apply3)
-  T* work[3];        // per direction: component-major slice results
-  long long wstride[3];   // elements per component
-  int nstrips;       // k_flux3
+  T* work;           // the direction's component-major slice results
+  long long wstride; // elements per component
+  const T* qsum;     // k_apply3: what the direction's slices are added to, and its
+  Geom gsum;         //   geometry (the old state, then qout)
   unsigned long long* cfl_bits;
 };
 
@@ -49,10 +57,23 @@ __device__ __host__ __forceinline__ void dir_extents(const Geom& g, int& n, int&
   else { n = g.mz; na = g.mx; nb = g.my; }
 }
 
-// Work index of (component, slice (a, b), position p = 1..n+1).
-__device__ __forceinline__ long long widx(int comp, long long stride, int a, int b, int p,
-                                          int n, int na) {
-  return comp * stride + ((long long)b * (na + 2) + a) * (n + 1) + (p - 1);
+// Slices are numbered so that consecutive ones lie next to each other in x (in y
+// for the x-slices): the strided q rows of neighbouring slices share lines.
+template <int DIR>
+__device__ __forceinline__ void slice_ab(long long sl, int na, int nb, int& sa, int& sb) {
+  if (DIR == 2) { sb = (int)(sl % (nb + 2)); sa = (int)(sl / (nb + 2)); }
+  else { sa = (int)(sl % (na + 2)); sb = (int)(sl / (na + 2)); }
+}
+template <int DIR>
+__device__ __forceinline__ long long slice_no(int a, int b, int na, int nb) {
+  return DIR == 2 ? (long long)a * (nb + 2) + b : (long long)b * (na + 2) + a;
+}
+
+// Each XCD takes a contiguous range of the blocks (the dispatcher deals them out
+// in turn over 8 XCDs), so that neighbouring slices meet in one L2.
+__device__ __forceinline__ long long xcd_block() {
+  const unsigned n = gridDim.x, b = blockIdx.x, per = n / 8, rest = n % 8, x = b % 8, i = b / 8;
+  return (long long)x * per + min(x, rest) + i;
 }
 
 // component slots: 0..ME-1 qadd, ME..2ME-1 fadd, then gadd / hadd as
@@ -71,19 +92,26 @@ __global__ void __launch_bounds__(256) k_flux3(const Step3Args<double> a) {
   constexpr int ME = RS::meqn, MW = RS::mwaves;
   using WL = W3<ME>;
   const int lane = threadIdx.x & 63;
-  const int wid = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  const long long wid = xcd_block() * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int n, na, nb;
   dir_extents<DIR>(a.g, n, na, nb);
-  const long long slices = (long long)(na + 2) * (nb + 2);
-  // wavefronts past the last slice skip the work but reach the workgroup's
+  const long long slices = (long long)(na + 2) * (nb + 2), cells = slices * (n + 4);
+  // wavefronts past the last cell skip the work but reach the workgroup's
   // Courant-number reduction (a barrier): one atomic per workgroup
-  const bool live = wid < a.nstrips * slices;   // uniform per wavefront
+  const bool live = wid * 60 < cells;   // uniform per wavefront
   double cfl_wave = 0.0;
   if (live) {
-    const int strip = wid % a.nstrips;
-    const long long sl = wid / a.nstrips;
-    const int sa = (int)(sl % (na + 2)), sb = (int)(sl / (na + 2));   // 0..na+1, 0..nb+1
-    const int c = 1 + strip * 60 - 2 + lane;
+    // the lane's place in the row of slices: cell c = -1..n+2 of slice (sa, sb);
+    // lanes outside the row take its first or last cell and own nothing
+    const long long first = wid * 60 / (n + 4);
+    const int at = (int)(wid * 60 - first * (n + 4)) + lane - 2;
+    const int hop = at < 0 ? 0 : at / (n + 4);
+    const bool inside = (at >= 0 || first > 0) && first + hop < slices;
+    // at < 0: the last cells of the slice before
+    const long long sl = !inside ? (at < 0 ? 0 : slices - 1) : at < 0 ? first - 1 : first + hop;
+    const int c = (!inside ? (at < 0 ? 0 : n + 3) : at < 0 ? at + n + 4 : at - hop * (n + 4)) - 1;
+    int sa, sb;   // 0..na+1, 0..nb+1
+    slice_ab<DIR>(sl, na, nb, sa, sb);
     const T dtn = DIR == 1 ? a.dtdx : (DIR == 2 ? a.dtdy : a.dtdz);
     // flux3's dtdy / dtdz: the first / second transverse direction's dt/d
     const T dt1 = DIR == 1 ? a.dtdy : (DIR == 2 ? a.dtdz : a.dtdx);
@@ -100,7 +128,7 @@ __global__ void __launch_bounds__(256) k_flux3(const Step3Args<double> a) {
     RS::template rpn<DIR>(a.rp, QL, Q, W, s, am, ap, roe);
     // Courant number over interfaces 1..n+1 (flux3.f90:214-221)
     T smax = T(0);
-    if (lane >= 1 && c >= 1 && c <= n + 1) {
+    if (lane >= 1 && inside && c >= 1 && c <= n + 1) {
   #pragma unroll
       for (int w = 0; w < MW; w++) smax = cfl_term(smax, fabs(s[w]));
     }
@@ -138,17 +166,17 @@ __global__ void __launch_bounds__(256) k_flux3(const Step3Args<double> a) {
     for (int m = 0; m < ME; m++) fadd[m] = T(0) + cq[m];
 
     // stores of this lane's cell c (cells 1..n; fadd at interfaces 1..n+1)
-    const bool own = lane >= 2 && lane < 62 && c >= 1;
+    const bool own = lane >= 2 && lane < 62 && inside && c >= 1;
     const bool own_cell = own && c <= n;
-    T* wk = a.work[DIR - 1];
-    const long long st = a.wstride[DIR - 1];
+    const long long st = a.wstride;
+    T* wk = a.work + slice_no<DIR>(sa, sb, na, nb) * (n + 1) + (c - 1);
     if (own && c <= n + 1) {
   #pragma unroll
-      for (int m = 0; m < ME; m++) wk[widx(WL::FA + m, st, sa, sb, c, n, na)] = fadd[m];
+      for (int m = 0; m < ME; m++) wk[(WL::FA + m) * st] = fadd[m];
     }
     if (own_cell) {
   #pragma unroll
-      for (int m = 0; m < ME; m++) wk[widx(WL::QA + m, st, sa, sb, c, n, na)] = qadd[m];
+      for (int m = 0; m < ME; m++) wk[(WL::QA + m) * st] = qadd[m];
     }
     const int m3 = a.m3, m4 = a.m4;
     T bmam[ME], bpam[ME], bmap[ME], bpap[ME], cmam[ME], cpam[ME], cmap[ME], cpap[ME];
@@ -249,7 +277,7 @@ __global__ void __launch_bounds__(256) k_flux3(const Step3Args<double> a) {
           for (int sd = 0; sd < 2; sd++)
   #pragma unroll
             for (int o = 0; o < 3; o++)
-              wk[widx(WL::gh(base, m, sd + 1, o - 1), st, sa, sb, c, n, na)] = v[sd][o];
+              wk[WL::gh(base, m, sd + 1, o - 1) * st] = v[sd][o];
         }
       }
     };
@@ -262,78 +290,103 @@ __global__ void __launch_bounds__(256) k_flux3(const Step3Args<double> a) {
   block_atomic_max(cfl_wave, a.cfl_bits);
 }
 
-// One slice's update of a cell at transverse offsets (da, db) from the slice
-// (step3.f90:189-225 and the y / z equivalents): v is the cell's running value.
-template <int ME>
-__device__ __forceinline__ double term3(double v, const double* wk, long long st, int sa, int sb,
-                                        int p, int n, int na, int m, int da, int db, double dtn,
-                                        double dt1, double dt2) {
+// One slice's update of a cell at transverse offsets (DA, DB) from the slice
+// (step3.f90:189-225 and the y / z equivalents): v is the cell's running value,
+// wk field m's qadd of the slice (uniform), at the cell's byte offset in it (32
+// bits: a component of a work array that fits in memory is under 4 GB).
+template <int ME, int DA, int DB>
+__device__ __forceinline__ double term3(double v, const double* wk, long long st, unsigned at,
+                                        double dtn, double dt1, double dt2) {
   using WL = W3<ME>;
-  auto G = [&](int side, int off) { return wk[widx(WL::gh(WL::G, m, side, off), st, sa, sb, p, n, na)]; };
-  auto H = [&](int side, int off) { return wk[widx(WL::gh(WL::H, m, side, off), st, sa, sb, p, n, na)]; };
-  if (da == 0 && db == 0) {
-    const double qa = wk[widx(WL::QA + m, st, sa, sb, p, n, na)];
-    const double f0 = wk[widx(WL::FA + m, st, sa, sb, p, n, na)];
-    const double f1 = wk[widx(WL::FA + m, st, sa, sb, p + 1, n, na)];
+  auto W = [&](long long comp) {
+    return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(wk + comp * st) + at);
+  };
+  auto G = [&](int side, int off) { return W(WL::gh(WL::G, 0, side, off)); };
+  auto H = [&](int side, int off) { return W(WL::gh(WL::H, 0, side, off)); };
+  if constexpr (DA == 0 && DB == 0) {
+    const double qa = W(WL::QA);
+    const double f0 = W(WL::FA);
+    const double f1 =
+        *reinterpret_cast<const double*>(reinterpret_cast<const char*>(wk + WL::FA * st + 1) + at);
     return v + qa - dtn * (f1 - f0) - dt1 * (G(2, 0) - G(1, 0)) - dt2 * (H(2, 0) - H(1, 0));
   }
-  if (da == -1 && db == 0) return v - dt1 * G(1, 0) - dt2 * (H(2, -1) - H(1, -1));
-  if (da == -1 && db == -1) return v - dt1 * G(1, -1) - dt2 * H(1, -1);
-  if (da == 0 && db == -1) return v - dt1 * (G(2, -1) - G(1, -1)) - dt2 * H(1, 0);
-  if (da == 1 && db == -1) return v + dt1 * G(2, -1) - dt2 * H(1, 1);
-  if (da == 1 && db == 0) return v + dt1 * G(2, 0) - dt2 * (H(2, 1) - H(1, 1));
-  if (da == 1 && db == 1) return v + dt1 * G(2, 1) + dt2 * H(2, 1);
-  if (da == 0 && db == 1) return v - dt1 * (G(2, 1) - G(1, 1)) + dt2 * H(2, 0);
+  if constexpr (DA == -1 && DB == 0) return v - dt1 * G(1, 0) - dt2 * (H(2, -1) - H(1, -1));
+  if constexpr (DA == -1 && DB == -1) return v - dt1 * G(1, -1) - dt2 * H(1, -1);
+  if constexpr (DA == 0 && DB == -1) return v - dt1 * (G(2, -1) - G(1, -1)) - dt2 * H(1, 0);
+  if constexpr (DA == 1 && DB == -1) return v + dt1 * G(2, -1) - dt2 * H(1, 1);
+  if constexpr (DA == 1 && DB == 0) return v + dt1 * G(2, 0) - dt2 * (H(2, 1) - H(1, 1));
+  if constexpr (DA == 1 && DB == 1) return v + dt1 * G(2, 1) + dt2 * H(2, 1);
+  if constexpr (DA == 0 && DB == 1) return v - dt1 * (G(2, 1) - G(1, 1)) + dt2 * H(2, 0);
   return v - dt1 * G(1, 1) + dt2 * H(2, -1);   // (-1, 1)
 }
 
-template <class RS>
+// A thread per cell, numbered along the slices (consecutive lanes: consecutive
+// cells of a slice), then as the slices are.
+template <class RS, int DIR>
 __global__ void __launch_bounds__(256) k_apply3(const Step3Args<double> a) {
   constexpr int ME = RS::meqn;
   const Geom& g = a.g;
-  const long long cell = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  const long long ncell = (long long)g.mx * g.my * g.mz;
-  if (cell >= ncell) return;
-  const int i = 1 + (int)(cell % g.mx);
-  const int j = 1 + (int)((cell / g.mx) % g.my);
-  const int k = 1 + (int)(cell / ((long long)g.mx * g.my));
-  const double* pin = cell_ptr3(a.qin, g, i, j, k);
+  int n, na, nb;
+  dir_extents<DIR>(g, n, na, nb);
+  const long long cell = xcd_block() * 256 + threadIdx.x;
+  if (cell >= (long long)n * na * nb) return;
+  const int p = 1 + (int)(cell % n);
+  const long long rest = cell / n;
+  const int sa = 1 + (int)(DIR == 2 ? rest / nb : rest % na);
+  const int sb = 1 + (int)(DIR == 2 ? rest % nb : rest / na);
+  int i, j, k;
+  if (DIR == 1) { i = p; j = sa; k = sb; }
+  else if (DIR == 2) { j = p; k = sa; i = sb; }
+  else { k = p; i = sa; j = sb; }
+  const double* pin = cell_ptr3(a.qsum, a.gsum, i, j, k);
   Geom go = g;
   go.g = 0; go.rs = g.mx; go.ss = (long long)g.mx * g.my; go.fs = go.ss * g.mz;
   double* pout = cell_ptr3(a.qout, go, i, j, k);
+  const double dtn = DIR == 1 ? a.dtdx : (DIR == 2 ? a.dtdy : a.dtdz);
+  const double dt1 = DIR == 1 ? a.dtdy : (DIR == 2 ? a.dtdz : a.dtdx);
+  const double dt2 = DIR == 1 ? a.dtdz : (DIR == 2 ? a.dtdx : a.dtdy);
+  // elements from a slice to the next in a and in b
+  const long long ea = (DIR == 2 ? nb + 2 : 1) * (long long)(n + 1);
+  const long long eb = (DIR == 2 ? 1 : na + 2) * (long long)(n + 1);
+  // byte offset of (p, slice (sa-1, sb-1)), the first of the 9
+  const unsigned at =
+      (unsigned)((slice_no<DIR>(sa - 1, sb - 1, na, nb) * (n + 1) + (p - 1)) * (long long)sizeof(double));
+  const long long st = a.wstride;
 #pragma unroll 1
   for (int m = 0; m < ME; m++) {
-    double v = pin[(long long)m * g.fs];
-    // x-slices (a = j', b = k'): k' outer, j' inner
-    for (int bb = k - 1; bb <= k + 1; bb++)
-      for (int aa = j - 1; aa <= j + 1; aa++)
-        v = term3<ME>(v, a.work[0], a.wstride[0], aa, bb, i, g.mx, g.my, m, j - aa, k - bb,
-                      a.dtdx, a.dtdy, a.dtdz);
-    // y-slices (a = k', b = i'): k' outer, i' inner
-    for (int aa = k - 1; aa <= k + 1; aa++)
-      for (int bb = i - 1; bb <= i + 1; bb++)
-        v = term3<ME>(v, a.work[1], a.wstride[1], aa, bb, j, g.my, g.mz, m, k - aa, i - bb,
-                      a.dtdy, a.dtdz, a.dtdx);
-    // z-slices (a = i', b = j'): j' outer, i' inner
-    for (int bb = j - 1; bb <= j + 1; bb++)
-      for (int aa = i - 1; aa <= i + 1; aa++)
-        v = term3<ME>(v, a.work[2], a.wstride[2], aa, bb, k, g.mz, g.mx, m, i - aa, j - bb,
-                      a.dtdz, a.dtdx, a.dtdy);
+    const double* w = a.work + m * st;
+    double v = pin[(long long)m * a.gsum.fs];
+#define TERM(AA, BB) \
+  v = term3<ME, -(AA), -(BB)>(v, w + ((AA) + 1) * ea + ((BB) + 1) * eb, st, at, dtn, dt1, dt2)
+    if constexpr (DIR == 2) {   // y-slices (a = k', b = i'): k' outer, i' inner
+      TERM(-1, -1); TERM(-1, 0); TERM(-1, 1);
+      TERM(0, -1); TERM(0, 0); TERM(0, 1);
+      TERM(1, -1); TERM(1, 0); TERM(1, 1);
+    } else {   // x-slices (a = j', b = k'): k' outer; z-slices (a = i', b = j'): j' outer
+      TERM(-1, -1); TERM(0, -1); TERM(1, -1);
+      TERM(-1, 0); TERM(0, 0); TERM(1, 0);
+      TERM(-1, 1); TERM(0, 1); TERM(1, 1);
+    }
+#undef TERM
     pout[(long long)m * go.fs] = v;
   }
 }
 
 namespace {
 template <class RS, int DIR>
-int launch_flux3(Step3Args<double> a, hipStream_t stream) {
+void launch_flux3(const Step3Args<double>& a, hipStream_t stream) {
   int n, na, nb;
   dir_extents<DIR>(a.g, n, na, nb);
-  a.nstrips = (n + 1 + 59) / 60;
-  const long long waves = (long long)a.nstrips * (na + 2) * (nb + 2);
-  hipLaunchKernelGGL((k_flux3<RS, DIR>), dim3((unsigned)((waves + 3) / 4)), dim3(256), 0,
+  const long long cells = (long long)(na + 2) * (nb + 2) * (n + 4);
+  hipLaunchKernelGGL((k_flux3<RS, DIR>), dim3((unsigned)((cells + 239) / 240)), dim3(256), 0,
                      stream, a);
-  hipError_t e = hipGetLastError();
-  return e == hipSuccess ? 0 : (int)e;
+}
+
+template <class RS, int DIR>
+void launch_apply3(const Step3Args<double>& a, hipStream_t stream) {
+  const long long ncell = (long long)a.g.mx * a.g.my * a.g.mz;
+  hipLaunchKernelGGL((k_apply3<RS, DIR>), dim3((unsigned)((ncell + 255) / 256)), dim3(256), 0,
+                     stream, a);
 }
 }  // namespace
 
@@ -362,21 +415,28 @@ int launch_step3(const clawhip_rp& rp, const void* q_in, const Geom& gin, void* 
   a.qin = (const double*)q_in;
   a.qout = (double*)q_out;
   a.cfl_bits = cfl;
-  const int mx = gin.mx, my = gin.my, mz = gin.mz, ME = RS::meqn;
+  const int mx = gin.mx, my = gin.my, mz = gin.mz;
   const long long s1 = (long long)(mx + 1) * (my + 2) * (mz + 2);
   const long long s2 = (long long)(my + 1) * (mz + 2) * (mx + 2);
   const long long s3 = (long long)(mz + 1) * (mx + 2) * (my + 2);
-  double* w = (double*)work;
-  a.work[0] = w; a.wstride[0] = s1;
-  a.work[1] = w + 14LL * ME * s1; a.wstride[1] = s2;
-  a.work[2] = a.work[1] + 14LL * ME * s2; a.wstride[2] = s3;
-  int rc = launch_flux3<RS, 1>(a, stream);
-  if (!rc) rc = launch_flux3<RS, 2>(a, stream);
-  if (!rc) rc = launch_flux3<RS, 3>(a, stream);
-  if (rc) return rc;
-  const long long ncell = (long long)mx * my * mz;
-  hipLaunchKernelGGL((k_apply3<RS>), dim3((unsigned)((ncell + 255) / 256)), dim3(256), 0,
-                     stream, a);
+  // the directions share the work array (the entry point refuses q_out == q_in,
+  // so all of them read the old state); each adds its slices to the sum so far
+  const long long stride[3] = {s1, s2, s3};
+  Geom go = gin;
+  go.g = 0; go.rs = mx; go.ss = (long long)mx * my; go.fs = go.ss * mz;
+  Step3Args<double> d[3] = {a, a, a};
+  for (int k = 0; k < 3; k++) {
+    d[k].work = (double*)work;
+    d[k].wstride = stride[k];
+    d[k].qsum = k == 0 ? a.qin : a.qout;
+    d[k].gsum = k == 0 ? gin : go;
+  }
+  launch_flux3<RS, 1>(d[0], stream);
+  launch_apply3<RS, 1>(d[0], stream);
+  launch_flux3<RS, 2>(d[1], stream);
+  launch_apply3<RS, 2>(d[1], stream);
+  launch_flux3<RS, 3>(d[2], stream);
+  launch_apply3<RS, 3>(d[2], stream);
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : (int)e;
 }
