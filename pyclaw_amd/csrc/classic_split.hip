@@ -108,11 +108,12 @@ __global__ void __launch_bounds__(256) k_xsweep(const SweepArgs<T> a) {
     j = 1 - ng + row % nrows_j;
     k = DIM == 3 ? 1 - ng + row / nrows_j : 1;
   };
+  const Column col = make_column(a.gin, a.bc, ng, c);
   auto load_row = [&](int row, T (&Q)[ME]) {
     int j, k;
     row_jk(row, j, k);
-    if (DIM == 2) load_cell2<ME>(a.qin, a.gin, a.bc, ng, c, j, Q);
-    else load_cell3<ME>(a.qin, a.gin, a.bc, ng, c, j, k, Q);
+    if (DIM == 2) load_row2<ME>(a.qin, a.gin, a.bc, ng, col, j, Q);
+    else load_row3<ME>(a.qin, a.gin, a.bc, ng, col, j, k, Q);
   };
   double cfl = 0.0;
   T Qn[ME];
@@ -225,8 +226,18 @@ __device__ __forceinline__ long long cell_off(const Geom& g, int i, int s, int p
 // runs, the row loaded ahead and one Courant-number atomic per workgroup the
 // split step takes 1.04 instead of 1.33 ms there (FP64) and 4.13 instead of
 // 5.24 ms at 384^3 (FP32 + Kahan).
+// Wavefronts per SIMD a march is compiled for, where that differs from the
+// compiler's choice: FP64 euler_3D sits 4 registers above the 256 of 2 per SIMD
+// and fits them without spills (210x170x190 step 1.07 -> 0.95 ms).  FP32 + Kahan
+// euler_3D (141, 15 spilled at the 128 of 4 per SIMD) loses 4 % there.
+template <class RS>
+struct SplitMarchWaves { static constexpr int value = 1; };
+template <>
+struct SplitMarchWaves<Euler3<double>> { static constexpr int value = 2; };
+
 template <class RS, typename T, bool KAHAN, int AXIS, bool HALF_IN_SUM>
-__global__ void __launch_bounds__(256) k_march(const SweepArgs<T> a) {
+__global__ void __launch_bounds__(256)
+    __attribute__((amdgpu_waves_per_eu(SplitMarchWaves<RS>::value))) k_march(const SweepArgs<T> a) {
   constexpr int ME = RS::meqn, MW = RS::mwaves;
   constexpr int IXY = AXIS;   // Riemann direction: 2 = y, 3 = z
   using Roe = typename RS::Roe;

@@ -375,55 +375,86 @@ __device__ __forceinline__ void load_store_in(const SharpArgs<T>& a, const Stage
   const T* pa = (om == OUT_DQDT || om == OUT_ADD6 || om == OUT_D) ? nullptr : v.A;
   const T* pb = om == OUT_F32_S2 ? a.B : om == OUT_F32_S3 ? a.aux_in : nullptr;
   const T* pc = om == OUT_F32_S3 ? v.comp_in : nullptr;
+  auto take = [&](const T* p, T (&x)[ME]) __attribute__((always_inline)) {
+    if (p) {
 #pragma unroll
-  for (int m = 0; m < ME; m++) {
-    si.pa[m] = pa ? pa[off + m * fs] : T(0);
-    si.pb[m] = pb ? pb[off + m * fs] : T(0);
-    si.pc[m] = pc ? pc[off + m * fs] : T(0);
+      for (int m = 0; m < ME; m++) x[m] = p[off + m * fs];
+    } else {
+#pragma unroll
+      for (int m = 0; m < ME; m++) x[m] = T(0);
+    }
+  };
+  take(pa, si.pa);
+  if constexpr (sizeof(T) == 4) {   // the FP32 stages' inputs
+    take(pb, si.pb);
+    take(pc, si.pc);
   }
 }
 
-// Stage combination of cell offset `off`, field m (SharpClawSolver.step,
+// Stage combination of cell offset `off` into o and memory (SharpClawSolver.step,
 // sharpclaw/solver.py:312-323, 400-430; the FP32 stages keep a compensated sum).
+// One (uniform) choice of the mode for all fields.
 template <int ME, typename T>
-__device__ __forceinline__ T stage_store(const SharpArgs<T>& a, const StageView<T>& v,
-                                         const StoreIn<ME, T>& si, long long off, int m, T D,
-                                         T yv) {
+__device__ __forceinline__ void stage_store(const SharpArgs<T>& a, const StageView<T>& v,
+                                            const StoreIn<ME, T>& si, long long off, T (&D)[ME],
+                                            const T (&yv)[ME], T (&o)[ME]) {
   const long long fs = a.g.fs;
   // dq = dq_hyperbolic + dq_src (sharpclaw/solver.py:537-540)
-  if (a.src) D = D + a.src[off + m * fs];
-  const int om = a.omode;
-  T o;
-  if (om == OUT_DQDT) {
-    if constexpr (sizeof(T) == 4) o = D * v.rdt;
-    else o = D / v.dt;
-  } else if (om == OUT_SSP33_2) {
-    o = T(0.75) * si.pa[m] + T(0.25) * (yv + D);
-  } else if (om == OUT_SSP33_3) {
-    o = T(1. / 3.) * si.pa[m] + T(2. / 3.) * (yv + D);
-  } else if (om == OUT_ADD6) {
-    o = yv + D / T(6);
-  } else if (om == OUT_SSP104_FIN) {
-    o = si.pa[m] + (T(0.6) * yv + T(0.1) * D);
-  } else if (om == OUT_D) {
-    o = D;
-  } else if (om == OUT_SSP22) {
-    o = T(0.5) * ((si.pa[m] + yv) + D);
-  } else if (om == OUT_F32_S2) {
-    T e1 = v.s * si.pb[m];
-    T inc = e1 + D;
-    o = si.pa[m] + T(0.25) * inc;
-    a.aux_out[off + m * fs] = inc * T(1. / 6.);
-  } else {   // OUT_F32_S3
-    T delta = si.pb[m] + T(2. / 3.) * D;
-    T qa = si.pa[m];
-    T yk = delta - si.pc[m];
-    T tq = qa + yk;
-    v.comp_out[off + m * fs] = (tq - qa) - yk;
-    o = tq;
+  if (a.src) {
+#pragma unroll
+    for (int m = 0; m < ME; m++) D[m] = D[m] + a.src[off + m * fs];
   }
-  v.out[off + m * fs] = o;
-  return o;
+  auto each = [&](auto f) __attribute__((always_inline)) {
+#pragma unroll
+    for (int m = 0; m < ME; m++) o[m] = f(m);
+  };
+  switch (a.omode) {
+    case OUT_DQDT:
+      each([&](int m) {
+        if constexpr (sizeof(T) == 4) return D[m] * v.rdt;
+        else return D[m] / v.dt;
+      });
+      break;
+    case OUT_SSP33_2:
+      each([&](int m) { return T(0.75) * si.pa[m] + T(0.25) * (yv[m] + D[m]); });
+      break;
+    case OUT_SSP33_3:
+      each([&](int m) { return T(1. / 3.) * si.pa[m] + T(2. / 3.) * (yv[m] + D[m]); });
+      break;
+    case OUT_ADD6:
+      each([&](int m) { return yv[m] + D[m] / T(6); });
+      break;
+    case OUT_SSP104_FIN:
+      each([&](int m) { return si.pa[m] + (T(0.6) * yv[m] + T(0.1) * D[m]); });
+      break;
+    case OUT_D:
+      each([&](int m) { return D[m]; });
+      break;
+    case OUT_SSP22:
+      each([&](int m) { return T(0.5) * ((si.pa[m] + yv[m]) + D[m]); });
+      break;
+    case OUT_F32_S2:
+      if constexpr (sizeof(T) == 4)
+        each([&](int m) {
+          const T e1 = v.s * si.pb[m];
+          const T inc = e1 + D[m];
+          a.aux_out[off + m * fs] = inc * T(1. / 6.);
+          return si.pa[m] + T(0.25) * inc;
+        });
+      break;
+    default:   // OUT_F32_S3
+      if constexpr (sizeof(T) == 4)
+        each([&](int m) {
+          const T delta = si.pb[m] + T(2. / 3.) * D[m];
+          const T qa = si.pa[m];
+          const T yk = delta - si.pc[m];
+          const T tq = qa + yk;
+          v.comp_out[off + m * fs] = (tq - qa) - yk;
+          return tq;
+        });
+  }
+#pragma unroll
+  for (int m = 0; m < ME; m++) v.out[off + m * fs] = o[m];
 }
 
 // The stage input Y of cell (c, r): P, P + s*Q or P + (s*Q)/6 (y_mode), with the
@@ -713,19 +744,23 @@ __global__ void __launch_bounds__(256) k_sharp_march(const MarchArgs<T> ma) {
     const bool ycfl_lane = c >= 0 && c <= mx + 1;
     const RPParams<T>& rp = a.rp;
 
-    auto load_y = [&](int r, T (&y)[ME]) { stage_input<ME>(a, v, c, r, y); };
+    const Column col = make_column(a.gin, a.bc, a.ng, c);
     // a window row in two parts: its loads (issued one iteration ahead) and the
     // stage-input combination stage_input applies (the same expression)
     auto load_raw = [&](int r, T (&p)[ME], T (&q)[ME]) {
-      load_cell2<ME>(v.P, a.gin, a.bc, a.ng, c, r, p);
-      if (a.ymode != Y_ARRAY) load_cell2<ME>(a.Q, a.gin, a.bc, a.ng, c, r, q);
+      load_row2<ME>(v.P, a.gin, a.bc, a.ng, col, r, p);
+      if (a.ymode != Y_ARRAY) load_row2<ME>(a.Q, a.gin, a.bc, a.ng, col, r, q);
     };
     auto combine = [&](const T (&p)[ME], const T (&q)[ME], T (&y)[ME]) {
+      if (a.ymode == Y_ARRAY) {
   #pragma unroll
-      for (int m = 0; m < ME; m++) {
-        y[m] = p[m];
-        if (a.ymode != Y_ARRAY)
-          y[m] = a.ymode == Y_AXPY ? y[m] + v.s * q[m] : y[m] + (v.s * q[m]) / T(6);
+        for (int m = 0; m < ME; m++) y[m] = p[m];
+      } else if (a.ymode == Y_AXPY) {
+  #pragma unroll
+        for (int m = 0; m < ME; m++) y[m] = p[m] + v.s * q[m];
+      } else {
+  #pragma unroll
+        for (int m = 0; m < ME; m++) y[m] = p[m] + (v.s * q[m]) / T(6);
       }
     };
     auto load_a = [&](int r, T (&A)[MA]) {
@@ -807,9 +842,16 @@ __global__ void __launch_bounds__(256) k_sharp_march(const MarchArgs<T> ma) {
     };
 
     // ---- window rows r0-3 .. r0+2; y-interface r0; aux of rows t-1 (Alo), t (Ahi)
-    T win[6][ME];
+    T win[6][ME], raw[6][ME];
   #pragma unroll
-    for (int k = 0; k < 6; k++) load_y(r0 - 3 + k, win[k]);
+    for (int k = 0; k < 6; k++) load_raw(r0 - 3 + k, win[k], raw[k]);
+  #pragma unroll
+    for (int k = 0; k < 6; k++) {
+      T y[ME];
+      combine(win[k], raw[k], y);
+  #pragma unroll
+      for (int m = 0; m < ME; m++) win[k][m] = y[m];
+    }
     T Alo[MA], Ahi[MA];
     load_a(r0 - 1, Alo);
     load_a(r0, Ahi);
@@ -892,13 +934,17 @@ __global__ void __launch_bounds__(256) k_sharp_march(const MarchArgs<T> ma) {
       T dqx[ME];
       x_cell(win[2], Alo, t - 1, xlisted(xb), dqx);
       if (out_lane) {
-        bool bad = false;
+        T D[ME], o[ME];
   #pragma unroll
-        for (int m = 0; m < ME; m++) {
-          const T o = stage_store<ME>(a, v, si, off, m, (T(0) + dqx[m]) + dqy[m], win[2][m]);
-          bad = bad || (((a.pos_mask >> m) & 1u) && (!(o > T(0)) || !isfinite(o)));
+        for (int m = 0; m < ME; m++) D[m] = (T(0) + dqx[m]) + dqy[m];
+        stage_store<ME>(a, v, si, off, D, win[2], o);
+        if (a.pos_mask) {
+          bool lost = false;
+  #pragma unroll
+          for (int m = 0; m < ME; m++)
+            lost = lost || (((a.pos_mask >> m) & 1u) && (!(o[m] > T(0)) || !isfinite(o[m])));
+          nbad += lost ? 1 : 0;
         }
-        nbad += bad ? 1 : 0;
       }
   #pragma unroll
       for (int m = 0; m < ME; m++) { qlY[m] = qlR[m]; apY[m] = ap[m]; }

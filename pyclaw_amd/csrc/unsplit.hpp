@@ -248,9 +248,10 @@ __device__ __forceinline__ double unsplit_body(const UnsplitArgs<T>& a, int wid)
   T Am[NA], A0[NA], A1[NA];   // aux rows t-1, t, t+1 (AUX)
   XRow<ME, T> xr;
   // ---- warm-up: rows j0-2, j0-1, j0; x-pass of row j0-1; y-interfaces j0-1, j0
-  load_cell2<ME>(a.qin, a.gin, a.bc, a.ng, c, j0 - 2, Qm);
-  load_cell2<ME>(a.qin, a.gin, a.bc, a.ng, c, j0 - 1, Q0);
-  load_cell2<ME>(a.qin, a.gin, a.bc, a.ng, c, j0, Q1);
+  const Column col = make_column(a.gin, a.bc, a.ng, c);
+  load_row2<ME>(a.qin, a.gin, a.bc, a.ng, col, j0 - 2, Qm);
+  load_row2<ME>(a.qin, a.gin, a.bc, a.ng, col, j0 - 1, Q0);
+  load_row2<ME>(a.qin, a.gin, a.bc, a.ng, col, j0, Q1);
   load_aux<AUX>(a, c, j0 - 2, Am);
   load_aux<AUX>(a, c, j0 - 1, A0);
   load_aux<AUX>(a, c, j0, A1);
@@ -284,7 +285,7 @@ __device__ __forceinline__ double unsplit_body(const UnsplitArgs<T>& a, int wid)
   for (int m = 0; m < ME; m++) { qaddy_p[m] = T(0); hbm_p[m] = T(0); hbp_p[m] = T(0); Fy_p[m] = T(0); }
 
   for (int t = j0; t <= jend; t++) {
-    load_cell2<ME>(a.qin, a.gin, a.bc, a.ng, c, t + 1, Q1);
+    load_row2<ME>(a.qin, a.gin, a.bc, a.ng, col, t + 1, Q1);
     load_aux<AUX>(a, c, t + 1, A1);
     // ---- x-slice t
     xpass<RS, AUX, CAPA>(a, Q0, Am, A0, A1, cflx_col && t <= my + 1, smx, xr);
