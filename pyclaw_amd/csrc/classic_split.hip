@@ -141,7 +141,10 @@ __global__ void __launch_bounds__(256) k_xsweep(const SweepArgs<T> a) {
       from_left(Q, QL);
       T W[MW][ME], s[MW], am[ME], ap[ME];
       typename RS::Roe roe;
-      rpn_call<RS, 1>(a.rp, QL, Q, AL, A, W, s, am, ap, roe);
+      Watch<RS, T> seen;
+      seen.see(Q);
+      const bool wide = watched<RS, T>() && (a.rp.wide || !seen.all_tame());
+      rpn_either<RS, 1>(a.rp, wide, QL, Q, AL, A, W, s, am, ap, roe);
       T smax = T(0);
       if (lane >= 1 && c >= 1 && c <= mx + 1) {
 #pragma unroll
@@ -305,17 +308,21 @@ __global__ void __launch_bounds__(256)
     load_aux(j0 - 2, Am);
     load_aux(j0 - 1, A0);
     load_aux(j0, A1);
+    // uniform: a value read so far needs the plain division (see Divided)
+    Watch<RS, T> seen;
+    seen.see(Qm); seen.see(Q0); seen.see(Q1);
+    bool wide = watched<RS, T>() && (a.rp.wide || !seen.all_tame());
     T Wt[MW][ME], st[MW], amt[ME], apt[ME], dotl[MW];
     Roe roet;
     {
       T Wp[MW][ME], sp[MW], amp[ME], app[ME];
       Roe roep;
-      rpn_call<RS, IXY>(a.rp, Qm, Q0, Am, A0, Wp, sp, amp, app, roep);
+      rpn_either<RS, IXY>(a.rp, wide, Qm, Q0, Am, A0, Wp, sp, amp, app, roep);
       if (j0 - 1 >= 1) {
 #pragma unroll
         for (int w = 0; w < MW; w++) smax = cfl_term(smax, fabs(sp[w]));
       }
-      rpn_call<RS, IXY>(a.rp, Q0, Q1, A0, A1, Wt, st, amt, apt, roet);
+      rpn_either<RS, IXY>(a.rp, wide, Q0, Q1, A0, A1, Wt, st, amt, apt, roet);
 #pragma unroll
       for (int w = 0; w < MW; w++) smax = cfl_term(smax, fabs(st[w]));
       wave_dots<ME, MW>(Wp, Wt, dotl);
@@ -329,6 +336,8 @@ __global__ void __launch_bounds__(256)
     for (int t = j0; t <= jend; t++) {
 #pragma unroll
       for (int m = 0; m < ME; m++) Q1[m] = Qn[m];
+      seen.see(Q1);
+      if (watched<RS, T>()) wide = wide || !seen.all_tame();   // to the run's end
       if (inplace && t + 2 >= jend) {   // rows jend, jend+1 belong to the next run
 #pragma unroll
         for (int m = 0; m < ME; m++) Qn[m] = t + 2 == jend ? U0[m] : U1[m];
@@ -345,7 +354,7 @@ __global__ void __launch_bounds__(256)
       load_aux(t + 1, A1);
       T Wn[MW][ME], sn[MW], amn[ME], apn[ME], dotn[MW];
       Roe roen;
-      rpn_call<RS, IXY>(a.rp, Q0, Q1, A0, A1, Wn, sn, amn, apn, roen);
+      rpn_either<RS, IXY>(a.rp, wide, Q0, Q1, A0, A1, Wn, sn, amn, apn, roen);
       if (t + 1 <= m_ax + 1) {
 #pragma unroll
         for (int w = 0; w < MW; w++) smax = cfl_term(smax, fabs(sn[w]));

@@ -47,6 +47,11 @@ inline RPParams<T> to_params(const clawhip_rp& r) {
   p.gamma = T(r.gamma); p.gamma1 = T(r.gamma - 1.0);
   p.grav = T(r.grav); p.u = T(r.u); p.v = T(r.v); p.efix = r.efix;
   p.dry_tolerance = T(r.dry_tolerance); p.fwave = r.fwave;
+  p.wide = 0;
+  for (double v : {r.gamma, r.gamma - 1.0, r.grav}) {
+    const double m = v < 0 ? -v : v;
+    if (!(m == 0.0 || (m > 0x1p-200 && m < 0x1p200))) p.wide = 1;
+  }
   return p;
 }
 

@@ -32,6 +32,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #ifndef CLAW_FAST
 #define CLAW_FAST 0
 #endif
@@ -51,6 +53,97 @@ struct RPParams {
   T dry_tolerance;       // shallow water with bathymetry
   int efix;
   int fwave;             // the solver returns f-waves (step2's use_fwave)
+  int wide;              // a parameter is beyond 2^+-200: see Divided
+};
+
+// ---- several quotients over one denominator, square roots
+// The compiler's FP64 division is: scale both operands if an exponent is extreme;
+// r = rcp(d) improved twice by Newton; q = a r, q + (a - d q) r; special cases
+// patched (div_fixup).  Divided<double, false> is that sequence with r computed
+// once for all numerators and without the scaling, so a / Divided(d) equals a / d
+// bit for bit (zeros, infinities and NaN too) unless an operand or quotient lies
+// beyond about 2^+-960.  Likewise root<false>(x) is the compiler's sqrt without
+// the scaling of x < 2^-767.  A division takes 57 cycles of a SIMD, a further
+// quotient over the same denominator 18, sqrt 86 and root 62; the FP64 Roe solves
+// spent half their cycles on them (1024^2 Euler step 128 -> 119 us, 2048^2 shallow-
+// water WENO5 stage 465 -> 398, 210x170x190 euler_3D step 0.99 -> 0.82 ms).
+// WIDE = true, and every type but double: the plain division and sqrt.  The
+// reference-equal FP64 kernels take it where a state has a value beyond 2^200 or
+// a nonzero one below 2^-700 (Watch; decaying tails reach denormals): a
+// march with several solves a row starts again at that row with the plain division
+// (march_both), the split sweeps go on with it.
+template <typename T, bool WIDE>
+struct Divided {
+  T d;
+  __device__ __forceinline__ explicit Divided(T den) : d(den) {}
+  __device__ __forceinline__ Divided(T den, T) : d(den) {}
+  __device__ __forceinline__ T reciprocal() const { return T(0); }   // not used
+  __device__ __forceinline__ friend T operator/(T a, const Divided& o) { return a / o.d; }
+};
+template <>
+struct Divided<double, false> {
+  double d, r;
+  __device__ __forceinline__ explicit Divided(double den) : d(den) {
+    r = __builtin_amdgcn_rcp(den);
+    r = __builtin_fma(r, __builtin_fma(-den, r, 1.0), r);
+    r = __builtin_fma(r, __builtin_fma(-den, r, 1.0), r);
+  }
+  // a reciprocal known beforehand
+  __device__ __forceinline__ Divided(double den, double rec) : d(den), r(rec) {}
+  __device__ __forceinline__ double reciprocal() const { return r; }
+  __device__ __forceinline__ friend double operator/(double a, const Divided& o) {
+    const double q = a * o.r;
+    return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-o.d, q, a), o.r, q), o.d, a);
+  }
+};
+template <bool WIDE, typename T>
+__device__ __forceinline__ T root(T x) {
+  if constexpr (sizeof(T) == 8 && !WIDE) {
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = y * 0.5;
+    const double e = __builtin_fma(-h, g, 0.5);
+    g = __builtin_fma(g, e, g);
+    h = __builtin_fma(h, e, h);
+    g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+    g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+    return __builtin_amdgcn_class(x, 0x260) ? x : g;   // +-0 and +infinity
+  } else {
+    return sqrt(x);
+  }
+}
+
+// Whether a solver's kernels watch for values that need WIDE (see above): the
+// reference-equal FP64 build.  The contracted build is held to tolerances.
+template <class RS, typename T>
+constexpr bool watched() { return RS::shares && sizeof(T) == 8 && CLAW_FAST == 0; }
+
+// The magnitudes of the values a lane has met: tame() while all are zero or in
+// [2^-700, 2^200) (not NaN).  Kept as the smallest and largest of the words that
+// hold a value's exponent and leading digits (doubled, which drops the sign; a
+// zero, less one, is the largest), so that watching costs no branch.
+template <class RS, typename T>
+struct Watch {
+  unsigned least = ~0u, most = 0u;
+  template <int ME>
+  __device__ __forceinline__ void see(const T (&q)[ME]) {
+    if constexpr (watched<RS, T>()) {
+#pragma unroll
+      for (int m = 0; m < ME; m++) {
+        const unsigned long long b = __builtin_bit_cast(unsigned long long, q[m]);
+        const unsigned low = (unsigned)b;
+        const unsigned u = ((unsigned)(b >> 32) << 1) | (low < 1u ? low : 1u);
+        least = least < u - 1u ? least : u - 1u;
+        most = most > u ? most : u;
+      }
+    }
+  }
+  // uniform over the wavefront
+  __device__ __forceinline__ bool all_tame() const {
+    return !watched<RS, T>() || __ballot(!tame()) == 0ull;
+  }
+  __device__ __forceinline__ bool tame() const {
+    return least >= 2u * 0x14300000u && most < 2u * 0x4c700000u;
+  }
 };
 
 template <typename T>
@@ -62,6 +155,9 @@ __device__ __forceinline__ T dmin(T a, T b) { return a < b ? a : b; }
 template <typename T>
 struct Acoustics {
   static constexpr int meqn = 3, mwaves = 2, maux = 0;
+  // divides plainly: its divisions are few, and watching the values for shared
+  // reciprocals costs a 256^2 step 5 % where it gains 4 % at 4096^2
+  static constexpr bool shares = false;
   struct Roe {};
   template <int IXY>
   __device__ static __forceinline__ void rpn(const RPParams<T>& p, const T* qL, const T* qR,
@@ -110,7 +206,8 @@ struct Acoustics {
 template <typename T, int TR>
 struct EulerT {
   static constexpr int meqn = 4 + TR, mwaves = 4 + TR, maux = 0;
-  struct Roe { T u, v, enth, u2v2, a, g1a2, euv; };
+  static constexpr bool shares = true;   // shared denominators: rpn and rpt take WIDE
+  struct Roe { T u, v, enth, u2v2, a, g1a2, euv, a2r; };   // a2r: reciprocal of 2 a (Divided)
   // normal flux; the Roe linearisation gives amdq + apdq = flux(qR) - flux(qL)
   template <int IXY>
   __device__ static __forceinline__ void flux(const RPParams<T>& p, const T* q, T (&f)[meqn]) {
@@ -133,14 +230,14 @@ struct EulerT {
 
   // The fast variant's Roe average: 1/rho per side (also 1/sqrt(rho) =
   // sqrt(rho)/rho), 1/(sqrt(rhoL) + sqrt(rhoR)) and 1/a^2 once each.
-  template <int IXY>
+  template <int IXY, bool WIDE>
   __device__ static __forceinline__ Roe roe_avg_shared(T gamma1, const T* qL, const T* qR,
                                                        T& irl, T& irr, T& ia2) {
     constexpr int mu = IXY == 1 ? 1 : 2, mv = IXY == 1 ? 2 : 1;
     Roe r;
     irl = T(1) / qL[0];
     irr = T(1) / qR[0];
-    const T rhsqrtl = sqrt(qL[0]), rhsqrtr = sqrt(qR[0]);
+    const T rhsqrtl = root<WIDE>(qL[0]), rhsqrtr = root<WIDE>(qR[0]);
     const T isl = rhsqrtl * irl, isr = rhsqrtr * irr;
     const T pl = gamma1 * (qL[3] - T(0.5) * (qL[1] * qL[1] + qL[2] * qL[2]) * irl);
     const T pr = gamma1 * (qR[3] - T(0.5) * (qR[1] * qR[1] + qR[2] * qR[2]) * irr);
@@ -150,42 +247,45 @@ struct EulerT {
     r.enth = ((qL[3] + pl) * isl + (qR[3] + pr) * isr) * irq;
     r.u2v2 = r.u * r.u + r.v * r.v;
     const T a2 = gamma1 * (r.enth - T(.5) * r.u2v2);
-    r.a = sqrt(a2);
+    r.a = root<WIDE>(a2);
+    r.a2r = Divided<T, WIDE>(T(2) * r.a).reciprocal();
     ia2 = T(1) / a2;
     r.g1a2 = gamma1 * ia2;
     r.euv = r.enth - r.u2v2;
     return r;
   }
 
-  template <int IXY>
-  __device__ static __forceinline__ Roe roe_avg(T gamma1, const T* qL, const T* qR) {
+  template <int IXY, bool WIDE>
+  __device__ static __forceinline__ Roe roe_avg(T gamma1, const T* qL, const T* qR,
+                                                const Divided<T, WIDE>& rhol, const Divided<T, WIDE>& rhor) {
     constexpr int mu = IXY == 1 ? 1 : 2, mv = IXY == 1 ? 2 : 1;
     Roe r;
-    T rhsqrtl = sqrt(qL[0]);
-    T rhsqrtr = sqrt(qR[0]);
-    T pl = gamma1 * (qL[3] - T(0.5) * (qL[1] * qL[1] + qL[2] * qL[2]) / qL[0]);
-    T pr = gamma1 * (qR[3] - T(0.5) * (qR[1] * qR[1] + qR[2] * qR[2]) / qR[0]);
-    T rhsq2 = rhsqrtl + rhsqrtr;
+    const T rootl = root<WIDE>(qL[0]), rootr = root<WIDE>(qR[0]);
+    T pl = gamma1 * (qL[3] - T(0.5) * (qL[1] * qL[1] + qL[2] * qL[2]) / rhol);
+    T pr = gamma1 * (qR[3] - T(0.5) * (qR[1] * qR[1] + qR[2] * qR[2]) / rhor);
+    const Divided<T, WIDE> rhsqrtl(rootl), rhsqrtr(rootr), rhsq2(rootl + rootr);
     r.u = (qL[mu] / rhsqrtl + qR[mu] / rhsqrtr) / rhsq2;
     r.v = (qL[mv] / rhsqrtl + qR[mv] / rhsqrtr) / rhsq2;
     r.enth = (((qL[3] + pl) / rhsqrtl + (qR[3] + pr) / rhsqrtr)) / rhsq2;
     r.u2v2 = r.u * r.u + r.v * r.v;
     T a2 = gamma1 * (r.enth - T(.5) * r.u2v2);
-    r.a = sqrt(a2);
+    r.a = root<WIDE>(a2);
+    r.a2r = Divided<T, WIDE>(T(2) * r.a).reciprocal();
     r.g1a2 = gamma1 / a2;
     r.euv = r.enth - r.u2v2;
     return r;
   }
 
-  template <int IXY>
+  template <int IXY, bool WIDE>
   __device__ static __forceinline__ void rpn(const RPParams<T>& p, const T* qL, const T* qR,
                                              T (&wave)[mwaves][meqn], T (&s)[mwaves],
                                              T (&amdq)[meqn], T (&apdq)[meqn], Roe& r) {
     constexpr int mu = IXY == 1 ? 1 : 2, mv = IXY == 1 ? 2 : 1;
     const T gamma = p.gamma, gamma1 = p.gamma1;
     T irl = T(0), irr = T(0), ia2 = T(0);   // shared reciprocals (fast variant)
-    if constexpr (kSharedReciprocals) r = roe_avg_shared<IXY>(gamma1, qL, qR, irl, irr, ia2);
-    else r = roe_avg<IXY>(gamma1, qL, qR);
+    const Divided<T, WIDE> rhol(qL[0]), rhor(qR[0]);
+    if constexpr (kSharedReciprocals) r = roe_avg_shared<IXY, WIDE>(gamma1, qL, qR, irl, irr, ia2);
+    else r = roe_avg<IXY, WIDE>(gamma1, qL, qR, rhol, rhor);
     T d0 = qR[0] - qL[0], d1 = qR[mu] - qL[mu], d2 = qR[mv] - qL[mv], d3 = qR[3] - qL[3];
     T a3 = r.g1a2 * (r.euv * d0 + r.u * d1 + r.v * d2 - d3);
     T a2 = d2 - r.v * d0;
@@ -193,7 +293,7 @@ struct EulerT {
     if constexpr (kSharedReciprocals)   // 1/(2a) = a/(2a^2)
       a4 = (d1 + (r.a - r.u) * d0 - r.a * a3) * (T(0.5) * r.a * ia2);
     else
-      a4 = (d1 + (r.a - r.u) * d0 - r.a * a3) / (T(2) * r.a);
+      a4 = (d1 + (r.a - r.u) * d0 - r.a * a3) / Divided<T, WIDE>(T(2) * r.a, r.a2r);
     T a1 = d0 - a3 - a4;
     wave[0][0] = a1; wave[0][mu] = a1 * (r.u - r.a); wave[0][mv] = a1 * r.v;
     wave[0][3] = a1 * (r.enth - r.u * r.a); s[0] = r.u - r.a;
@@ -221,16 +321,15 @@ struct EulerT {
       return;
     }
     do {
-      T rhoim1 = qL[0];
       T pim1, cim1, s0;
       if constexpr (kSharedReciprocals) {
         pim1 = gamma1 * (qL[3] - T(0.5) * (qL[mu] * qL[mu] + qL[mv] * qL[mv]) * irl);
-        cim1 = sqrt(gamma * pim1 * irl);
+        cim1 = root<WIDE>(gamma * pim1 * irl);
         s0 = qL[mu] * irl - cim1;
       } else {
-        pim1 = gamma1 * (qL[3] - T(0.5) * (qL[mu] * qL[mu] + qL[mv] * qL[mv]) / rhoim1);
-        cim1 = sqrt(gamma * pim1 / rhoim1);
-        s0 = qL[mu] / rhoim1 - cim1;
+        pim1 = gamma1 * (qL[3] - T(0.5) * (qL[mu] * qL[mu] + qL[mv] * qL[mv]) / rhol);
+        cim1 = root<WIDE>(gamma * pim1 / rhol);
+        s0 = qL[mu] / rhol - cim1;
       }
       if (s0 >= T(0) && s[0] > T(0)) {
 #pragma unroll
@@ -245,12 +344,13 @@ struct EulerT {
       if constexpr (kSharedReciprocals) {
         const T ir1 = T(1) / rho1;
         p1 = gamma1 * (en1 - T(0.5) * (rhou1 * rhou1 + rhov1 * rhov1) * ir1);
-        c1 = sqrt(gamma * p1 * ir1);
+        c1 = root<WIDE>(gamma * p1 * ir1);
         s1 = rhou1 * ir1 - c1;
       } else {
-        p1 = gamma1 * (en1 - T(0.5) * (rhou1 * rhou1 + rhov1 * rhov1) / rho1);
-        c1 = sqrt(gamma * p1 / rho1);
-        s1 = rhou1 / rho1 - c1;
+        const Divided<T, WIDE> drho1(rho1);
+        p1 = gamma1 * (en1 - T(0.5) * (rhou1 * rhou1 + rhov1 * rhov1) / drho1);
+        c1 = root<WIDE>(gamma * p1 / drho1);
+        s1 = rhou1 / drho1 - c1;
       }
       T sfract;
       if (s0 < T(0) && s1 > T(0)) sfract = s0 * (s1 - s[0]) / (s1 - s0);
@@ -265,16 +365,15 @@ struct EulerT {
         amdq[m] = amdq[m] + s[2] * wave[2][m];
         if constexpr (TR) amdq[m] = amdq[m] + s[4] * wave[4][m];
       }
-      T rhoi = qR[0];
       T pi, ci, s3;
       if constexpr (kSharedReciprocals) {
         pi = gamma1 * (qR[3] - T(0.5) * (qR[mu] * qR[mu] + qR[mv] * qR[mv]) * irr);
-        ci = sqrt(gamma * pi * irr);
+        ci = root<WIDE>(gamma * pi * irr);
         s3 = qR[mu] * irr + ci;
       } else {
-        pi = gamma1 * (qR[3] - T(0.5) * (qR[mu] * qR[mu] + qR[mv] * qR[mv]) / rhoi);
-        ci = sqrt(gamma * pi / rhoi);
-        s3 = qR[mu] / rhoi + ci;
+        pi = gamma1 * (qR[3] - T(0.5) * (qR[mu] * qR[mu] + qR[mv] * qR[mv]) / rhor);
+        ci = root<WIDE>(gamma * pi / rhor);
+        s3 = qR[mu] / rhor + ci;
       }
       T rho2 = qR[0] - wave[3][0];
       T rhou2 = qR[mu] - wave[3][mu];
@@ -284,12 +383,13 @@ struct EulerT {
       if constexpr (kSharedReciprocals) {
         const T ir2 = T(1) / rho2;
         p2 = gamma1 * (en2 - T(0.5) * (rhou2 * rhou2 + rhov2 * rhov2) * ir2);
-        c2 = sqrt(gamma * p2 * ir2);
+        c2 = root<WIDE>(gamma * p2 * ir2);
         s2 = rhou2 * ir2 + c2;
       } else {
-        p2 = gamma1 * (en2 - T(0.5) * (rhou2 * rhou2 + rhov2 * rhov2) / rho2);
-        c2 = sqrt(gamma * p2 / rho2);
-        s2 = rhou2 / rho2 + c2;
+        const Divided<T, WIDE> drho2(rho2);
+        p2 = gamma1 * (en2 - T(0.5) * (rhou2 * rhou2 + rhov2 * rhov2) / drho2);
+        c2 = root<WIDE>(gamma * p2 / drho2);
+        s2 = rhou2 / drho2 + c2;
       }
       if (s2 < T(0) && s3 > T(0)) sfract = s2 * (s3 - s[3]) / (s3 - s2);
       else if (s[3] < T(0)) sfract = s[3];
@@ -306,13 +406,13 @@ struct EulerT {
     }
   }
 
-  template <int IXY>
+  template <int IXY, bool WIDE>
   __device__ static __forceinline__ void rpt(const RPParams<T>&, const Roe& r, const T (&asdq)[meqn],
                                              T (&bm)[meqn], T (&bp)[meqn]) {
     constexpr int mu = IXY == 1 ? 1 : 2, mv = IXY == 1 ? 2 : 1;
     T a3 = r.g1a2 * (r.euv * asdq[0] + r.u * asdq[mu] + r.v * asdq[mv] - asdq[3]);
     T a2 = asdq[mu] - r.u * asdq[0];
-    T a4 = (asdq[mv] + (r.a - r.v) * asdq[0] - r.a * a3) / (T(2) * r.a);
+    T a4 = (asdq[mv] + (r.a - r.v) * asdq[0] - r.a * a3) / Divided<T, WIDE>(T(2) * r.a, r.a2r);
     T a1 = asdq[0] - a3 - a4;
     T wb[3 + TR][meqn], sb[3 + TR];
     wb[0][0] = a1; wb[0][mu] = a1 * r.u; wb[0][mv] = a1 * (r.v - r.a);
@@ -345,6 +445,7 @@ template <typename T> using Euler5 = EulerT<T, 1>;
 template <typename T>
 struct Shallow {
   static constexpr int meqn = 3, mwaves = 3, maux = 0;
+  static constexpr bool shares = true;
   struct Roe { T u, v, a; };
   // normal flux; the Roe linearisation gives amdq + apdq = flux(qR) - flux(qL)
   template <int IXY>
@@ -356,19 +457,18 @@ struct Shallow {
     f[mv] = q[mv] * un;
   }
 
-  template <int IXY>
+  template <int IXY, bool WIDE>
   __device__ static __forceinline__ void rpn(const RPParams<T>& p, const T* qL, const T* qR,
                                              T (&wave)[mwaves][meqn], T (&s)[mwaves],
                                              T (&amdq)[meqn], T (&apdq)[meqn], Roe& r) {
     constexpr int mu = IXY == 1 ? 1 : 2, mv = IXY == 1 ? 2 : 1;
     const T grav = p.grav;
     T h = (qL[0] + qR[0]) * T(0.50);
-    T hsqrtl = sqrt(qL[0]);
-    T hsqrtr = sqrt(qR[0]);
-    T hsq2 = hsqrtl + hsqrtr;
+    const T rootl = root<WIDE>(qL[0]), rootr = root<WIDE>(qR[0]);
+    const Divided<T, WIDE> hsqrtl(rootl), hsqrtr(rootr), hsq2(rootl + rootr);
     T u = (qL[mu] / hsqrtl + qR[mu] / hsqrtr) / hsq2;
     T v = (qL[mv] / hsqrtl + qR[mv] / hsqrtr) / hsq2;
-    T a = sqrt(grav * h);
+    T a = root<WIDE>(grav * h);
     r.u = u; r.v = v; r.a = a;
     T delta0 = qR[0] - qL[0];
     T delta1 = qR[mu] - qL[mu];
@@ -393,7 +493,7 @@ struct Shallow {
     }
     do {
       T him1 = qL[0];
-      T s0 = qL[mu] / him1 - sqrt(grav * him1);
+      T s0 = qL[mu] / him1 - root<WIDE>(grav * him1);
       if (s0 >= T(0) && s[0] > T(0)) {
 #pragma unroll
         for (int m = 0; m < meqn; m++) amdq[m] = T(0);
@@ -401,7 +501,7 @@ struct Shallow {
       }
       T h1 = qL[0] + wave[0][0];
       T hu1 = qL[mu] + wave[0][mu];
-      T s1 = hu1 / h1 - sqrt(grav * h1);
+      T s1 = hu1 / h1 - root<WIDE>(grav * h1);
       T sfract;
       if (s0 < T(0) && s1 > T(0)) sfract = s0 * (s1 - s[0]) / (s1 - s0);
       else if (s[0] < T(0)) sfract = s[0];
@@ -412,10 +512,10 @@ struct Shallow {
 #pragma unroll
       for (int m = 0; m < meqn; m++) amdq[m] = amdq[m] + s[1] * wave[1][m];
       T hi = qR[0];
-      T s03 = qR[mu] / hi + sqrt(grav * hi);
+      T s03 = qR[mu] / hi + root<WIDE>(grav * hi);
       T h3 = qR[0] - wave[2][0];
       T hu3 = qR[mu] - wave[2][mu];
-      T s3 = hu3 / h3 + sqrt(grav * h3);
+      T s3 = hu3 / h3 + root<WIDE>(grav * h3);
       if (s3 < T(0) && s03 > T(0)) sfract = s3 * (s03 - s[2]) / (s03 - s3);
       else if (s[2] < T(0)) sfract = s[2];
       else break;
@@ -433,7 +533,7 @@ struct Shallow {
 
   // The transverse split recomputes the Roe average with the same operations as
   // rpn except that the wave speed uses the mean depth; it is carried in `r`.
-  template <int IXY>
+  template <int IXY, bool WIDE>
   __device__ static __forceinline__ void rpt(const RPParams<T>&, const Roe& r, const T (&asdq)[meqn],
                                              T (&bm)[meqn], T (&bp)[meqn]) {
     constexpr int mu = IXY == 1 ? 1 : 2, mv = IXY == 1 ? 2 : 1;
@@ -461,6 +561,7 @@ struct Shallow {
 template <typename T>
 struct Advection {
   static constexpr int meqn = 1, mwaves = 1, maux = 0;
+  static constexpr bool shares = false;
   struct Roe {};
   template <int IXY>
   __device__ static __forceinline__ void rpn(const RPParams<T>& p, const T* qL, const T* qR,
@@ -488,11 +589,12 @@ struct Advection {
 template <typename T>
 struct Euler3 {
   static constexpr int meqn = 5, mwaves = 3, maux = 0;
+  static constexpr bool shares = true;
   // the interface's Roe averages, kept for the transverse splits (u is the
   // normal velocity, v and w the next two in the cycle x -> y -> z)
-  struct Roe { T u, v, w, enth, a, g1a2, euv, u2v2w2; };
+  struct Roe { T u, v, w, enth, a, g1a2, euv, u2v2w2, a2r; };   // a2r: reciprocal of 2 a (Divided)
   // IXY = 1, 2, 3 selects x, y, z as the normal direction.
-  template <int IXY>
+  template <int IXY, bool WIDE>
   __device__ static __forceinline__ void rpn(const RPParams<T>& p, const T* qL, const T* qR,
                                              T (&wave)[mwaves][meqn], T (&s)[mwaves],
                                              T (&amdq)[meqn], T (&apdq)[meqn], Roe& roe) {
@@ -500,8 +602,8 @@ struct Euler3 {
     constexpr int mv = IXY == 1 ? 2 : (IXY == 2 ? 3 : 1);
     constexpr int mw = IXY == 1 ? 3 : (IXY == 2 ? 1 : 2);
     const T gamma = p.gamma, gamma1 = p.gamma1;
-    T rhsqrtl = sqrt(qL[0]);
-    T rhsqrtr = sqrt(qR[0]);
+    const T rootl = root<WIDE>(qL[0]), rootr = root<WIDE>(qR[0]);
+    const Divided<T, WIDE> rhol(qL[0]), rhor(qR[0]);
     // the fast variant's shared reciprocals (kSharedReciprocals): 1/rho per side
     // (and 1/sqrt(rho) = sqrt(rho)/rho), the Roe denominator, 1/a^2
     T irl = T(0), irr = T(0), ia2 = T(0);
@@ -509,18 +611,18 @@ struct Euler3 {
     if constexpr (kSharedReciprocals) {
       irl = T(1) / qL[0];
       irr = T(1) / qR[0];
-      const T isl = rhsqrtl * irl, isr = rhsqrtr * irr;
+      const T isl = rootl * irl, isr = rootr * irr;
       pl = gamma1 * (qL[4] - T(0.5) * (qL[1] * qL[1] + qL[2] * qL[2] + qL[3] * qL[3]) * irl);
       pr = gamma1 * (qR[4] - T(0.5) * (qR[1] * qR[1] + qR[2] * qR[2] + qR[3] * qR[3]) * irr);
-      const T irq = T(1) / (rhsqrtl + rhsqrtr);
+      const T irq = T(1) / (rootl + rootr);
       u = (qL[mu] * isl + qR[mu] * isr) * irq;
       v = (qL[mv] * isl + qR[mv] * isr) * irq;
       w = (qL[mw] * isl + qR[mw] * isr) * irq;
       enth = ((qL[4] + pl) * isl + (qR[4] + pr) * isr) * irq;
     } else {
-      pl = gamma1 * (qL[4] - T(0.5) * (qL[1] * qL[1] + qL[2] * qL[2] + qL[3] * qL[3]) / qL[0]);
-      pr = gamma1 * (qR[4] - T(0.5) * (qR[1] * qR[1] + qR[2] * qR[2] + qR[3] * qR[3]) / qR[0]);
-      T rhsq2 = rhsqrtl + rhsqrtr;
+      pl = gamma1 * (qL[4] - T(0.5) * (qL[1] * qL[1] + qL[2] * qL[2] + qL[3] * qL[3]) / rhol);
+      pr = gamma1 * (qR[4] - T(0.5) * (qR[1] * qR[1] + qR[2] * qR[2] + qR[3] * qR[3]) / rhor);
+      const Divided<T, WIDE> rhsqrtl(rootl), rhsqrtr(rootr), rhsq2(rootl + rootr);
       u = (qL[mu] / rhsqrtl + qR[mu] / rhsqrtr) / rhsq2;
       v = (qL[mv] / rhsqrtl + qR[mv] / rhsqrtr) / rhsq2;
       w = (qL[mw] / rhsqrtl + qR[mw] / rhsqrtr) / rhsq2;
@@ -528,7 +630,8 @@ struct Euler3 {
     }
     T u2v2w2 = u * u + v * v + w * w;
     T a2 = gamma1 * (enth - T(.5) * u2v2w2);
-    T a = sqrt(a2);
+    T a = root<WIDE>(a2);
+    roe.a2r = Divided<T, WIDE>(T(2) * a).reciprocal();
     T g1a2;
     if constexpr (kSharedReciprocals) {
       ia2 = T(1) / a2;
@@ -548,7 +651,7 @@ struct Euler3 {
     if constexpr (kSharedReciprocals)   // 1/(2a) = a/(2a^2)
       a5 = (d1 + (a - u) * d0 - a * a4) * (T(0.5) * a * ia2);
     else
-      a5 = (d1 + (a - u) * d0 - a * a4) / (T(2) * a);
+      a5 = (d1 + (a - u) * d0 - a * a4) / Divided<T, WIDE>(T(2) * a, roe.a2r);
     T a1 = d0 - a4 - a5;
     wave[0][0] = a1; wave[0][mu] = a1 * (u - a); wave[0][mv] = a1 * v; wave[0][mw] = a1 * w;
     wave[0][4] = a1 * (enth - u * a); s[0] = u - a;
@@ -569,16 +672,15 @@ struct Euler3 {
       return;
     }
     do {
-      T rhoim1 = qL[0];
       T pim1, cim1, s0;
       if constexpr (kSharedReciprocals) {
         pim1 = gamma1 * (qL[4] - T(0.5) * (qL[mu] * qL[mu] + qL[mv] * qL[mv] + qL[mw] * qL[mw]) * irl);
-        cim1 = sqrt(gamma * pim1 * irl);
+        cim1 = root<WIDE>(gamma * pim1 * irl);
         s0 = qL[mu] * irl - cim1;
       } else {
-        pim1 = gamma1 * (qL[4] - T(0.5) * (qL[mu] * qL[mu] + qL[mv] * qL[mv] + qL[mw] * qL[mw]) / rhoim1);
-        cim1 = sqrt(gamma * pim1 / rhoim1);
-        s0 = qL[mu] / rhoim1 - cim1;
+        pim1 = gamma1 * (qL[4] - T(0.5) * (qL[mu] * qL[mu] + qL[mv] * qL[mv] + qL[mw] * qL[mw]) / rhol);
+        cim1 = root<WIDE>(gamma * pim1 / rhol);
+        s0 = qL[mu] / rhol - cim1;
       }
       if (s0 >= T(0) && s[0] > T(0)) {
 #pragma unroll
@@ -594,12 +696,13 @@ struct Euler3 {
       if constexpr (kSharedReciprocals) {
         const T ir1 = T(1) / rho1;
         p1 = gamma1 * (en1 - T(0.5) * (rhou1 * rhou1 + rhov1 * rhov1 + rhow1 * rhow1) * ir1);
-        c1 = sqrt(gamma * p1 * ir1);
+        c1 = root<WIDE>(gamma * p1 * ir1);
         s1 = rhou1 * ir1 - c1;
       } else {
-        p1 = gamma1 * (en1 - T(0.5) * (rhou1 * rhou1 + rhov1 * rhov1 + rhow1 * rhow1) / rho1);
-        c1 = sqrt(gamma * p1 / rho1);
-        s1 = rhou1 / rho1 - c1;
+        const Divided<T, WIDE> drho1(rho1);
+        p1 = gamma1 * (en1 - T(0.5) * (rhou1 * rhou1 + rhov1 * rhov1 + rhow1 * rhow1) / drho1);
+        c1 = root<WIDE>(gamma * p1 / drho1);
+        s1 = rhou1 / drho1 - c1;
       }
       T sfract;
       if (s0 < T(0) && s1 > T(0)) sfract = s0 * (s1 - s[0]) / (s1 - s0);
@@ -610,16 +713,15 @@ struct Euler3 {
       if (s[1] >= T(0)) break;
 #pragma unroll
       for (int m = 0; m < meqn; m++) amdq[m] = amdq[m] + s[1] * wave[1][m];
-      T rhoi = qR[0];
       T pi, ci, s3;
       if constexpr (kSharedReciprocals) {
         pi = gamma1 * (qR[4] - T(0.5) * (qR[mu] * qR[mu] + qR[mv] * qR[mv] + qR[mw] * qR[mw]) * irr);
-        ci = sqrt(gamma * pi * irr);
+        ci = root<WIDE>(gamma * pi * irr);
         s3 = qR[mu] * irr + ci;
       } else {
-        pi = gamma1 * (qR[4] - T(0.5) * (qR[mu] * qR[mu] + qR[mv] * qR[mv] + qR[mw] * qR[mw]) / rhoi);
-        ci = sqrt(gamma * pi / rhoi);
-        s3 = qR[mu] / rhoi + ci;
+        pi = gamma1 * (qR[4] - T(0.5) * (qR[mu] * qR[mu] + qR[mv] * qR[mv] + qR[mw] * qR[mw]) / rhor);
+        ci = root<WIDE>(gamma * pi / rhor);
+        s3 = qR[mu] / rhor + ci;
       }
       T rho2 = qR[0] - wave[2][0];
       T rhou2 = qR[mu] - wave[2][mu];
@@ -630,12 +732,13 @@ struct Euler3 {
       if constexpr (kSharedReciprocals) {
         const T ir2 = T(1) / rho2;
         p2 = gamma1 * (en2 - T(0.5) * (rhou2 * rhou2 + rhov2 * rhov2 + rhow2 * rhow2) * ir2);
-        c2 = sqrt(gamma * p2 * ir2);
+        c2 = root<WIDE>(gamma * p2 * ir2);
         s2 = rhou2 * ir2 + c2;
       } else {
-        p2 = gamma1 * (en2 - T(0.5) * (rhou2 * rhou2 + rhov2 * rhov2 + rhow2 * rhow2) / rho2);
-        c2 = sqrt(gamma * p2 / rho2);
-        s2 = rhou2 / rho2 + c2;
+        const Divided<T, WIDE> drho2(rho2);
+        p2 = gamma1 * (en2 - T(0.5) * (rhou2 * rhou2 + rhov2 * rhov2 + rhow2 * rhow2) / drho2);
+        c2 = root<WIDE>(gamma * p2 / drho2);
+        s2 = rhou2 / drho2 + c2;
       }
       if (s2 < T(0) && s3 > T(0)) sfract = s2 * (s3 - s[2]) / (s3 - s2);
       else if (s[2] < T(0)) sfract = s[2];
@@ -651,7 +754,7 @@ struct Euler3 {
       apdq[m] = df - amdq[m];
     }
   }
-  template <int IXY>
+  template <int IXY, bool WIDE>
   __device__ static __forceinline__ void rpt(const RPParams<T>&, const Roe&, const T (&)[meqn],
                                              T (&bm)[meqn], T (&bp)[meqn]) {
 #pragma unroll
@@ -662,7 +765,7 @@ struct Euler3 {
   // direction after IXY in the cycle, momentum mv; 3: the next, mw) with the
   // interface's Roe averages; three waves at vt - a, vt, vt + a with the shear
   // parts lumped into the middle one; bm / bp take the negative / positive speeds.
-  template <int IXY, int ICOOR>
+  template <int IXY, int ICOOR, bool WIDE>
   __device__ static __forceinline__ void rpt3(const Roe& r, const T (&asdq)[meqn],
                                               T (&bm)[meqn], T (&bp)[meqn]) {
     constexpr int mu = IXY == 1 ? 1 : (IXY == 2 ? 2 : 3);
@@ -674,7 +777,7 @@ struct Euler3 {
     T a4 = r.g1a2 * (r.euv * asdq[0] + u * asdq[mu] + v * asdq[mv] + w * asdq[mw] - asdq[4]);
     T b1 = asdq[m1] - c1 * asdq[0];
     T b2 = asdq[m2] - c2 * asdq[0];
-    T a5 = (asdq[mt] + (a - vt) * asdq[0] - a * a4) / (T(2) * a);
+    T a5 = (asdq[mt] + (a - vt) * asdq[0] - a * a4) / Divided<T, WIDE>(T(2) * a, r.a2r);
     T a1 = asdq[0] - a4 - a5;
     T wv[3][meqn], sb[3];
     wv[0][0] = a1; wv[0][m1] = a1 * c1; wv[0][mt] = a1 * (vt - a); wv[0][m2] = a1 * c2;
@@ -708,13 +811,14 @@ struct Euler3 {
 template <typename T>
 struct ShallowHLLE {
   static constexpr int meqn = 3, mwaves = 2, maux = 0;
+  static constexpr bool shares = true;
   struct Roe {};
   // normal flux; the HLL waves give amdq + apdq = flux(qR) - flux(qL)
   template <int IXY>
   __device__ static __forceinline__ void flux(const RPParams<T>& p, const T* q, T (&f)[meqn]) {
     Shallow<T>::template flux<IXY>(p, q, f);
   }
-  template <int IXY>
+  template <int IXY, bool WIDE>
   __device__ static __forceinline__ void rpn(const RPParams<T>& p, const T* qL, const T* qR,
                                              T (&wave)[mwaves][meqn], T (&s)[mwaves],
                                              T (&amdq)[meqn], T (&apdq)[meqn], Roe&) {
@@ -722,16 +826,17 @@ struct ShallowHLLE {
     const T grav = p.grav;
     const T h_l = qL[0], h_r = qR[0];
     const T u_l = qL[mu] / qL[0], u_r = qR[mu] / qR[0];
-    const T hsqrt_l = sqrt(qL[0]), hsqrt_r = sqrt(qR[0]);
+    const T hsqrt_l = root<WIDE>(qL[0]), hsqrt_r = root<WIDE>(qR[0]);
     const T hsq2 = hsqrt_l + hsqrt_r;
     const T ubar = (u_l * hsqrt_l + u_r * hsqrt_r) / hsq2;
-    const T cbar = sqrt(T(0.5) * grav * (h_l + h_r));
-    const T s1 = dmin(u_l - sqrt(grav * h_l), ubar - cbar);
-    const T s2 = dmax(u_r + sqrt(grav * h_r), ubar + cbar);
-    const T hm = (qR[mu] - qL[mu] - s2 * qR[0] + s1 * qL[0]) / (s1 - s2);
+    const T cbar = root<WIDE>(T(0.5) * grav * (h_l + h_r));
+    const T s1 = dmin(u_l - root<WIDE>(grav * h_l), ubar - cbar);
+    const T s2 = dmax(u_r + root<WIDE>(grav * h_r), ubar + cbar);
+    const Divided<T, WIDE> ds(s1 - s2);
+    const T hm = (qR[mu] - qL[mu] - s2 * qR[0] + s1 * qL[0]) / ds;
     const T hum = (qR[mu] * u_r - qL[mu] * u_l + T(0.5) * grav * (h_r * h_r - h_l * h_l) -
-                   s2 * qR[mu] + s1 * qL[mu]) / (s1 - s2);
-    const T hvm = (qR[mv] * u_r - qL[mv] * u_l - s2 * qR[mv] + s1 * qL[mv]) / (s1 - s2);
+                   s2 * qR[mu] + s1 * qL[mu]) / ds;
+    const T hvm = (qR[mv] * u_r - qL[mv] * u_l - s2 * qR[mv] + s1 * qL[mv]) / ds;
     wave[0][0] = hm - h_l;
     wave[0][mu] = hum - qL[mu];
     wave[0][mv] = hvm - qL[mv];
@@ -752,7 +857,7 @@ struct ShallowHLLE {
     }
   }
   // Not reached: the entry points refuse transverse_waves > 0 for this solver.
-  template <int IXY>
+  template <int IXY, bool WIDE>
   __device__ static __forceinline__ void rpt(const RPParams<T>&, const Roe&, const T (&)[meqn],
                                              T (&bm)[meqn], T (&bp)[meqn]) {
 #pragma unroll
@@ -781,6 +886,7 @@ struct ShallowHLLE {
 template <typename T, int ME>
 struct VCAdvection {
   static constexpr int meqn = ME, mwaves = 1, maux = 2;
+  static constexpr bool shares = false;
   struct Roe {};
   template <int IXY>
   __device__ static __forceinline__ void rpn_aux(const RPParams<T>&, const T* qL, const T* qR,
@@ -833,6 +939,7 @@ template <typename T> using VCAdvection4 = VCAdvection<T, 4>;
 template <typename T>
 struct VCAcoustics {
   static constexpr int meqn = 3, mwaves = 2, maux = 2;
+  static constexpr bool shares = false;
   struct Roe {};
   template <int IXY>
   __device__ static __forceinline__ void rpn_aux(const RPParams<T>&, const T* qL, const T* qR,
@@ -895,6 +1002,7 @@ struct VCAcoustics {
 template <typename T>
 struct ShallowFwave {
   static constexpr int meqn = 3, mwaves = 3, maux = 1;
+  static constexpr bool shares = false;
   struct Roe {};
   template <int IXY>
   __device__ static __forceinline__ void rpn_aux(const RPParams<T>& p, const T* qL, const T* qR,
@@ -955,7 +1063,7 @@ struct ShallowFwave {
 
 // The normal solve with the aux values of the left and right cells; solvers
 // without aux fields take the plain call.
-template <class RS, int IXY, typename T>
+template <class RS, int IXY, bool WIDE, typename T>
 __device__ __forceinline__ void rpn_call(const RPParams<T>& p, const T* qL, const T* qR,
                                          const T* auxL, const T* auxR,
                                          T (&wave)[RS::mwaves][RS::meqn], T (&s)[RS::mwaves],
@@ -965,13 +1073,16 @@ __device__ __forceinline__ void rpn_call(const RPParams<T>& p, const T* qL, cons
     RS::template rpn_aux<IXY>(p, qL, qR, auxL, auxR, wave, s, amdq, apdq, roe);
   } else {
     (void)auxL; (void)auxR;
-    RS::template rpn<IXY>(p, qL, qR, wave, s, amdq, apdq, roe);
+    if constexpr (RS::shares)
+      RS::template rpn<IXY, WIDE>(p, qL, qR, wave, s, amdq, apdq, roe);
+    else
+      RS::template rpn<IXY>(p, qL, qR, wave, s, amdq, apdq, roe);
   }
 }
 
 // The transverse split with the aux values of cell i1 in the three slices
 // (previous, this, next); solvers without aux fields take the plain call.
-template <class RS, int IXY, typename T>
+template <class RS, int IXY, bool WIDE, typename T>
 __device__ __forceinline__ void rpt_call(const RPParams<T>& p, const typename RS::Roe& roe,
                                          const T* a1, const T* a2, const T* a3,
                                          const T (&asdq)[RS::meqn], T (&bm)[RS::meqn],
@@ -980,8 +1091,46 @@ __device__ __forceinline__ void rpt_call(const RPParams<T>& p, const typename RS
     RS::template rpt_aux<IXY>(p, roe, a1, a2, a3, asdq, bm, bp);
   } else {
     (void)a1; (void)a2; (void)a3;
-    RS::template rpt<IXY>(p, roe, asdq, bm, bp);
+    if constexpr (RS::shares)
+      RS::template rpt<IXY, WIDE>(p, roe, asdq, bm, bp);
+    else
+      RS::template rpt<IXY>(p, roe, asdq, bm, bp);
   }
+}
+
+// march(WIDE, first) is a wavefront's out-of-place work from row `first` on (its
+// beginning included); it returns the row it ended at because that row and the
+// following ones need the plain division, or kMarched.  With shared denominators
+// as far as they go, then plainly: the second march warms up anew and rewrites the
+// row the first stopped in.  (A branch at each of a row's solves keeps the
+// scheduler from interleaving them, and two forms of a row iteration in one march
+// cost registers; carrying the first march's values into the second does too.)
+constexpr int kMarched = 0x7fffffff;
+template <class RS, typename T, class March>
+__device__ __forceinline__ void march_both(bool wide, int first, March march) {
+  if constexpr (watched<RS, T>()) {
+    int row = wide ? first : march(std::false_type(), first);
+    if (__builtin_expect(row != kMarched, 0)) {
+      asm volatile("" : "+v"(row));   // nothing of it is worked out ahead
+      march(std::true_type(), __builtin_amdgcn_readfirstlane(row));
+    }
+  } else {
+    (void)wide;
+    march(std::integral_constant<bool, !RS::shares>(), first);
+  }
+}
+
+// One normal solve with the wavefront's kind of division.
+template <class RS, int IXY, typename T>
+__device__ __forceinline__ void rpn_either(const RPParams<T>& p, bool wide, const T* qL,
+                                           const T* qR, const T* auxL, const T* auxR,
+                                           T (&wave)[RS::mwaves][RS::meqn], T (&s)[RS::mwaves],
+                                           T (&amdq)[RS::meqn], T (&apdq)[RS::meqn],
+                                           typename RS::Roe& roe) {
+  if (watched<RS, T>() && __builtin_expect(wide, 0))
+    rpn_call<RS, IXY, true>(p, qL, qR, auxL, auxR, wave, s, amdq, apdq, roe);
+  else
+    rpn_call<RS, IXY, false>(p, qL, qR, auxL, auxR, wave, s, amdq, apdq, roe);
 }
 
 }  // namespace claw

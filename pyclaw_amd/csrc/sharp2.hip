@@ -106,7 +106,7 @@ struct SharpArgs {
 // ---------------------------------------------------------------- WENO5
 // weno.f90:32-79 for one cell: ql = left edge (fs0), qr = right edge (fs1).
 // `v` holds cells i-2..i+2.
-template <typename T>
+template <bool WIDE, typename T>
 __device__ __forceinline__ void weno5_cell(const T (&v)[5], T& fs0, T& fs1) {
   const T qm2 = v[0], qm1 = v[1], q0 = v[2], qp1 = v[3], qp2 = v[4];
   const T eps = weno_eps<T>();
@@ -129,12 +129,13 @@ __device__ __forceinline__ void weno5_cell(const T (&v)[5], T& fs0, T& fs1) {
              T(6.3333333333333333333333333333333333) * qm1 * qm2 +
              T(1.3333333333333333333333333333333333) * (qm2 * qm2);
   T d0 = eps + sigma0, d1 = eps + sigma1, d2 = eps + sigma2;
-  T omega0 = T(0.1) / (d0 * d0);
-  T omega1 = T(0.6) / (d1 * d1);
-  T omega2 = T(0.3) / (d2 * d2);
-  T omega3 = T(0.3) / (d0 * d0);
-  T omega4 = T(0.6) / (d1 * d1);
-  T omega5 = T(0.1) / (d2 * d2);
+  const Divided<T, WIDE> s0(d0 * d0), s1(d1 * d1), s2(d2 * d2);
+  T omega0 = T(0.1) / s0;
+  T omega1 = T(0.6) / s1;
+  T omega2 = T(0.3) / s2;
+  T omega3 = T(0.3) / s0;
+  T omega4 = omega1;
+  T omega5 = T(0.1) / s2;
   T fr0 = T(1.8333333333333333333333333333333333) * q0 -
           T(1.1666666666666666666666666666666667) * qp1 +
           T(0.33333333333333333333333333333333333) * qp2;
@@ -158,7 +159,7 @@ __device__ __forceinline__ void weno5_cell(const T (&v)[5], T& fs0, T& fs1) {
 }
 
 // reconstruct.f90:264-284 for one side: hh(-2..2) -> uu.
-template <typename T>
+template <bool WIDE, typename T>
 __device__ __forceinline__ T weno_char_side(T hm2, T hm1, T h0, T hp1, T hp2, int im) {
   // im = +1: (intwo, inone, ione) = (-2, -1, +1); im = -1: (2, 1, -1)
   T a2 = im == 1 ? hm2 : hp2;   // hh(intwo)
@@ -193,25 +194,25 @@ __device__ __forceinline__ T weno_char_side(T hm2, T hm1, T h0, T hp1, T hp2, in
     s1 = s1 * t0;
     s3 = s3 * t0;
   }
-  return (s1 * (t2 - t1) + (T(0.5) * s3 - T(0.25)) * (t3 - t2)) / T(3);
+  return (s1 * (t2 - t1) + (T(0.5) * s3 - T(0.25)) * (t3 - t2)) / Divided<T, WIDE>(T(3), T(1. / 3.));
 }
 
 // Eigenvectors at the Roe average of (qL, qR) in direction IXY (the same
 // formulas as the oracle's evec).  evl[ip][m] = row ip of R^-1, evr[m][ip].
-template <class RS, int IXY, typename T>
+template <class RS, int IXY, typename T, bool WIDE>
 struct Evec;
 
-template <int IXY, typename T>
-struct Evec<Shallow<T>, IXY, T> {
+template <int IXY, typename T, bool WIDE>
+struct Evec<Shallow<T>, IXY, T, WIDE> {
   __device__ static __forceinline__ void get(const RPParams<T>& p, const T* qL, const T* qR,
                                              T (&evl)[3][3], T (&evr)[3][3]) {
     constexpr int mu = IXY == 1 ? 1 : 2, mv = IXY == 1 ? 2 : 1;
     T h = (qL[0] + qR[0]) * T(0.50);
-    T hsqrtl = sqrt(qL[0]), hsqrtr = sqrt(qR[0]);
-    T hsq2 = hsqrtl + hsqrtr;
+    const T rootl = root<WIDE>(qL[0]), rootr = root<WIDE>(qR[0]);
+    const Divided<T, WIDE> hsqrtl(rootl), hsqrtr(rootr), hsq2(rootl + rootr);
     T u = (qL[mu] / hsqrtl + qR[mu] / hsqrtr) / hsq2;
     T v = (qL[mv] / hsqrtl + qR[mv] / hsqrtr) / hsq2;
-    T c = sqrt(p.grav * h);
+    T c = root<WIDE>(p.grav * h);
     evr[0][0] = T(1); evr[mu][0] = u - c; evr[mv][0] = v;
     evr[0][1] = T(0); evr[mu][1] = T(0); evr[mv][1] = T(1);
     evr[0][2] = T(1); evr[mu][2] = u + c; evr[mv][2] = v;
@@ -223,16 +224,16 @@ struct Evec<Shallow<T>, IXY, T> {
 };
 
 // The shallow-water eigenvectors do not depend on the Riemann solver.
-template <int IXY, typename T>
-struct Evec<ShallowHLLE<T>, IXY, T> : Evec<Shallow<T>, IXY, T> {};
+template <int IXY, typename T, bool WIDE>
+struct Evec<ShallowHLLE<T>, IXY, T, WIDE> : Evec<Shallow<T>, IXY, T, WIDE> {};
 
-template <int IXY, typename T>
-struct Evec<Euler<T>, IXY, T> {
+template <int IXY, typename T, bool WIDE>
+struct Evec<Euler<T>, IXY, T, WIDE> {
   __device__ static __forceinline__ void get(const RPParams<T>& p, const T* qL, const T* qR,
                                              T (&evl)[4][4], T (&evr)[4][4]) {
     constexpr int mu = IXY == 1 ? 1 : 2, mv = IXY == 1 ? 2 : 1;
     const T gamma1 = p.gamma1;
-    auto r = Euler<T>::template roe_avg<IXY>(gamma1, qL, qR);
+    auto r = Euler<T>::template roe_avg<IXY, WIDE>(gamma1, qL, qR, Divided<T, WIDE>(qL[0]), Divided<T, WIDE>(qR[0]));
     T u = r.u, v = r.v, c = r.a, H = r.enth;
     T q2 = T(0.5) * r.u2v2;
     evr[0][0] = T(1); evr[mu][0] = u - c; evr[mv][0] = v; evr[3][0] = H - u * c;
@@ -266,7 +267,7 @@ __device__ __forceinline__ void recon_linear(const T (&st)[6][ME], T (&qrL)[ME],
 
 // Reconstruct both sides of the interface between stencil cells 2 and 3 of
 // st[0..5] (cells c-3..c+2): qrL = right edge of cell c-1, qlR = left edge of c.
-template <class RS, int IXY, typename T, bool CHAR>
+template <class RS, int IXY, typename T, bool CHAR, bool WIDE>
 __device__ __forceinline__ void recon_interface(const RPParams<T>& p,
                                                 const T (&st)[6][RS::meqn],
                                                 T (&qrL)[RS::meqn], T (&qlR)[RS::meqn]) {
@@ -277,14 +278,14 @@ __device__ __forceinline__ void recon_interface(const RPParams<T>& p,
       T a[5] = {st[0][m], st[1][m], st[2][m], st[3][m], st[4][m]};
       T b[5] = {st[1][m], st[2][m], st[3][m], st[4][m], st[5][m]};
       T f0, f1;
-      weno5_cell(a, f0, f1);
+      weno5_cell<WIDE>(a, f0, f1);
       qrL[m] = f1;
-      weno5_cell(b, f0, f1);
+      weno5_cell<WIDE>(b, f0, f1);
       qlR[m] = f0;
     }
   } else {
     T evl[ME][ME], evr[ME][ME];
-    Evec<RS, IXY, T>::get(p, st[2], st[3], evl, evr);
+    Evec<RS, IXY, T, WIDE>::get(p, st[2], st[3], evl, evr);
     T dq[5][ME];   // dq(m, c+m2) = q(c+m2) - q(c+m2-1), m2 = -2..2
 #pragma unroll
     for (int k = 0; k < 5; k++)
@@ -292,7 +293,8 @@ __device__ __forceinline__ void recon_interface(const RPParams<T>& p,
       for (int m = 0; m < ME; m++) dq[k][m] = st[k + 1][m] - st[k][m];
 #pragma unroll
     for (int m = 0; m < ME; m++) {
-      T lin = (-st[1][m] + T(7) * (st[2][m] + st[3][m]) - st[4][m]) / T(12);
+      T lin = (-st[1][m] + T(7) * (st[2][m] + st[3][m]) - st[4][m]) /
+              Divided<T, WIDE>(T(12), T(1. / 12.));
       qrL[m] = lin;
       qlR[m] = lin;
     }
@@ -305,8 +307,8 @@ __device__ __forceinline__ void recon_interface(const RPParams<T>& p,
 #pragma unroll
         for (int m = 0; m < ME; m++) hh[k] = hh[k] + evl[ip][m] * dq[k][m];
       }
-      T uu1 = weno_char_side(hh[0], hh[1], hh[2], hh[3], hh[4], 1);
-      T uu2 = weno_char_side(hh[0], hh[1], hh[2], hh[3], hh[4], -1);
+      T uu1 = weno_char_side<WIDE>(hh[0], hh[1], hh[2], hh[3], hh[4], 1);
+      T uu2 = weno_char_side<WIDE>(hh[0], hh[1], hh[2], hh[3], hh[4], -1);
 #pragma unroll
       for (int m = 0; m < ME; m++) {
         qrL[m] = qrL[m] + evr[m][ip] * uu1;
@@ -658,13 +660,13 @@ __global__ void __launch_bounds__(256) k_weno_flagged(const SharpArgs<T> a) {
       const int c = 1 + (int)(id % (mx + 1)), r = 1 + (int)(id / (mx + 1));
 #pragma unroll
       for (int k = 0; k < 6; k++) stage_input<ME>(a, v, c - 3 + k, r, st[k]);
-      recon_interface<RS, 1, T, CHAR>(a.rp, st, qrL, qlR);
+      recon_interface<RS, 1, T, CHAR, true>(a.rp, st, qrL, qlR);
     } else {
       const long long j = id - nx;
       const int c = 1 + (int)(j % mx), t = 1 + (int)(j / mx);
 #pragma unroll
       for (int k = 0; k < 6; k++) stage_input<ME>(a, v, c, t - 3 + k, st[k]);
-      recon_interface<RS, 2, T, CHAR>(a.rp, st, qrL, qlR);
+      recon_interface<RS, 2, T, CHAR, true>(a.rp, st, qrL, qlR);
     }
     T* out = a.recon + id * (2 * ME);
 #pragma unroll
@@ -732,13 +734,15 @@ __global__ void __launch_bounds__(256) k_sharp_march(const MarchArgs<T> ma) {
   const bool live = wid < ma.nstrips * ma.nrb;   // uniform per wavefront
   T smax_x = T(0), smax_y = T(0);
   int nbad = 0;   // stored cells that lost positivity (count_bad)
-  if (live) {
-    const int strip = wid % ma.nstrips, rb = wid / ma.nstrips;
+  const int strip = wid % ma.nstrips, rb = wid / ma.nstrips;
+  // the wavefront's march from row `first` on (see march_both)
+  auto march = [&](auto kind, int first) __attribute__((always_inline)) {
+    constexpr bool WIDE = decltype(kind)::value;
     const int mx = a.g.mx, my = a.g.my;
     const int c0 = 1 + strip * 58;
     const int c = c0 - 3 + lane;                 // this lane's column
-    const int r0 = 1 + rb * ma.H;
-    const int rend = min(r0 + ma.H - 1, my);     // last output row
+    const int r0 = first;
+    const int rend = min((rb + 1) * ma.H, my);   // last output row
     const bool out_lane = lane >= 3 && lane <= 60 && c >= 1 && c <= mx;
     const bool xint_lane = lane >= 3 && lane <= 61 && c >= 1 && c <= mx + 1;
     const bool ycfl_lane = c >= 0 && c <= mx + 1;
@@ -770,7 +774,8 @@ __global__ void __launch_bounds__(256) k_sharp_march(const MarchArgs<T> ma) {
     // x-slice of row r (aux Ar of this lane's cell): interface c (left of this
     // lane's cell) -> qlR, qrL, am, ap
     auto x_interface = [&](const T (&row)[ME], const T (&Ar)[MA], int r, bool flagged,
-                           T (&qrL)[ME], T (&qlR)[ME], T (&am)[ME], T (&ap)[ME]) {
+                           T (&qrL)[ME], T (&qlR)[ME], T (&am)[ME], T (&ap)[ME])
+        __attribute__((always_inline)) {
       // st[k] = the row value of lane l + k - 3 (chained one-lane moves)
       T st[6][ME];
   #pragma unroll
@@ -788,13 +793,13 @@ __global__ void __launch_bounds__(256) k_sharp_march(const MarchArgs<T> ma) {
         recon_linear<ME>(st, qrL, qlR);
         if (flagged) load_recon<ME>(a.recon + xface_id(mx, c, r) * (2 * ME), qrL, qlR);
       } else {
-        recon_interface<RS, 1, T, CHAR>(rp, st, qrL, qlR);
+        recon_interface<RS, 1, T, CHAR, WIDE>(rp, st, qrL, qlR);
       }
       T W[MW][ME], sp[MW];
       typename RS::Roe roe;
       T AL[MA];
       if constexpr (AUX) from_left<MA>(Ar, AL);
-      rpn_call<RS, 1>(rp, qrL, qlR, AL, Ar, W, sp, am, ap, roe);
+      rpn_call<RS, 1, WIDE>(rp, qrL, qlR, AL, Ar, W, sp, am, ap, roe);
       if (xint_lane) {
   #pragma unroll
         for (int w = 0; w < MW; w++) smax_x = cfl_term(smax_x, (T)fabs(sp[w]));
@@ -803,23 +808,25 @@ __global__ void __launch_bounds__(256) k_sharp_march(const MarchArgs<T> ma) {
     // y-interface t (rows t-1 | t, aux Alo | Ahi) of this lane's column from the
     // window win[0..5] = rows t-3..t+2
     auto y_interface = [&](const T (&win)[6][ME], const T (&Alo)[MA], const T (&Ahi)[MA], int t,
-                           bool flagged, T (&qrL)[ME], T (&qlR)[ME], T (&am)[ME], T (&ap)[ME]) {
+                           bool flagged, T (&qrL)[ME], T (&qlR)[ME], T (&am)[ME], T (&ap)[ME])
+        __attribute__((always_inline)) {
       if (FLAGS) {
         recon_linear<ME>(win, qrL, qlR);
         if (flagged) load_recon<ME>(a.recon + yface_id(mx, my, c, t) * (2 * ME), qrL, qlR);
       } else {
-        recon_interface<RS, 2, T, CHAR>(rp, win, qrL, qlR);
+        recon_interface<RS, 2, T, CHAR, WIDE>(rp, win, qrL, qlR);
       }
       T W[MW][ME], sp[MW];
       typename RS::Roe roe;
-      rpn_call<RS, 2>(rp, qrL, qlR, Alo, Ahi, W, sp, am, ap, roe);
+      rpn_call<RS, 2, WIDE>(rp, qrL, qlR, Alo, Ahi, W, sp, am, ap, roe);
       if (ycfl_lane && t <= my + 1) {
   #pragma unroll
         for (int w = 0; w < MW; w++) smax_y = cfl_term(smax_y, (T)fabs(sp[w]));
       }
     };
     // x contribution of this lane's cell in row r (a whole x-slice pass)
-    auto x_cell = [&](const T (&row)[ME], const T (&Ar)[MA], int r, bool flagged, T (&dqx)[ME]) {
+    auto x_cell = [&](const T (&row)[ME], const T (&Ar)[MA], int r, bool flagged,
+                      T (&dqx)[ME]) __attribute__((always_inline)) {
       T qrL[ME], qlR[ME], am[ME], ap[ME];
       x_interface(row, Ar, r, flagged, qrL, qlR, am, ap);
       T qr[ME], amn[ME];
@@ -834,7 +841,7 @@ __global__ void __launch_bounds__(256) k_sharp_march(const MarchArgs<T> ma) {
       } else {
         T W[MW][ME], sp[MW], am2[ME], ap2[ME];
         typename RS::Roe roe;
-        rpn_call<RS, 1>(rp, qlR, qr, Ar, Ar, W, sp, am2, ap2, roe);
+        rpn_call<RS, 1, WIDE>(rp, qlR, qr, Ar, Ar, W, sp, am2, ap2, roe);
   #pragma unroll
         for (int m = 0; m < ME; m++)
           dqx[m] = T(0) - v.dtdx * (((amn[m] + ap[m]) + am2[m]) + ap2[m]);
@@ -842,6 +849,7 @@ __global__ void __launch_bounds__(256) k_sharp_march(const MarchArgs<T> ma) {
     };
 
     // ---- window rows r0-3 .. r0+2; y-interface r0; aux of rows t-1 (Alo), t (Ahi)
+    Watch<RS, T> seen;
     T win[6][ME], raw[6][ME];
   #pragma unroll
     for (int k = 0; k < 6; k++) load_raw(r0 - 3 + k, win[k], raw[k]);
@@ -851,7 +859,9 @@ __global__ void __launch_bounds__(256) k_sharp_march(const MarchArgs<T> ma) {
       combine(win[k], raw[k], y);
   #pragma unroll
       for (int m = 0; m < ME; m++) win[k][m] = y[m];
+      if (!WIDE) seen.see(win[k]);
     }
+    if (!WIDE && !seen.all_tame()) return r0;
     T Alo[MA], Ahi[MA];
     load_a(r0 - 1, Alo);
     load_a(r0, Ahi);
@@ -901,6 +911,10 @@ __global__ void __launch_bounds__(256) k_sharp_march(const MarchArgs<T> ma) {
   #pragma unroll
         for (int m = 0; m < ME; m++) win[k][m] = win[k + 1][m];
       combine(pf_p, pf_q, win[5]);
+      if (!WIDE) {
+        seen.see(win[5]);
+        if (!seen.all_tame()) return t - 1;
+      }
       if (t <= rend) load_raw(t + 3, pf_p, pf_q);
       // the store-time inputs of row t-1
       StoreIn<ME, T> si;
@@ -912,10 +926,10 @@ __global__ void __launch_bounds__(256) k_sharp_march(const MarchArgs<T> ma) {
       // the flag bytes of the next iteration (y-row t+1, x-row t)
       const int y_next = t <= rend ? ybyte(t + 1) : 0;
       const int x_next = t <= rend ? xbyte(t) : 0;
-      // y-interface t closes row t-1
-      T qrL[ME], qlR[ME], am[ME], ap[ME];
+      // y-interface t closes row t-1, then the x-slice of row t-1
+      T qlR[ME], ap[ME], dqx[ME], dqy[ME];
+      T qrL[ME], am[ME];
       y_interface(win, Alo, Ahi, t, (ym2 | ym1 | y0) != 0, qrL, qlR, am, ap);
-      T dqy[ME];
       if constexpr (TFLUCT) {
         T fl[ME], fr[ME];
         RS::template flux<2>(rp, qlY, fl);
@@ -925,13 +939,11 @@ __global__ void __launch_bounds__(256) k_sharp_march(const MarchArgs<T> ma) {
       } else {
         T W[MW][ME], sp[MW], am2[ME], ap2[ME];
         typename RS::Roe roe;
-        rpn_call<RS, 2>(rp, qlY, qrL, Alo, Alo, W, sp, am2, ap2, roe);
+        rpn_call<RS, 2, WIDE>(rp, qlY, qrL, Alo, Alo, W, sp, am2, ap2, roe);
   #pragma unroll
         for (int m = 0; m < ME; m++)
           dqy[m] = T(0) - v.dtdy * (((am[m] + apY[m]) + am2[m]) + ap2[m]);
       }
-      // x-slice of row t-1
-      T dqx[ME];
       x_cell(win[2], Alo, t - 1, xlisted(xb), dqx);
       if (out_lane) {
         T D[ME], o[ME];
@@ -957,7 +969,9 @@ __global__ void __launch_bounds__(256) k_sharp_march(const MarchArgs<T> ma) {
       T d[ME];
       x_cell(win[3], Ahi, my + 1, false, d);
     }
-  }
+    return kMarched;
+  };
+  if (live) march_both<RS, T>(a.rp.wide, 1 + rb * ma.H, march);
   double cx = (double)v.dtdx * (double)smax_x;
   double cy = (double)v.dtdy * (double)smax_y;
   block_atomic_max(cx > cy ? cx : cy, a.cfl_bits);

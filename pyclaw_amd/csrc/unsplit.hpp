@@ -89,7 +89,7 @@ struct XRow {
 // Am, A0, A1: aux of this lane's cell in rows t-1, t, t+1 (AUX kernels).
 // smax collects max |s| (dtdx applied at the end), or with CAPA the Courant
 // numbers themselves.
-template <class RS, bool AUX, bool CAPA, typename T>
+template <class RS, bool AUX, bool CAPA, bool WIDE, typename T>
 __device__ __forceinline__ void xpass(const UnsplitArgs<T>& a, const T (&Qc)[RS::meqn],
                                       const T (&Am)[UNSPLIT_MAX_AUX],
                                       const T (&A0)[UNSPLIT_MAX_AUX],
@@ -108,7 +108,7 @@ __device__ __forceinline__ void xpass(const UnsplitArgs<T>& a, const T (&Qc)[RS:
   }
   T W[MW][ME], s[MW], am[ME], ap[ME];
   typename RS::Roe roe;
-  rpn_call<RS, 1>(a.rp, QL, Qc, AL, A0, W, s, am, ap, roe);
+  rpn_call<RS, 1, WIDE>(a.rp, QL, Qc, AL, A0, W, s, am, ap, roe);
   if (cfl_ok) {
 #pragma unroll
     for (int w = 0; w < MW; w++) {
@@ -155,8 +155,8 @@ __device__ __forceinline__ void xpass(const UnsplitArgs<T>& a, const T (&Qc)[RS:
       from_left(Am, AmL);
       from_left(A1, A1L);
     }
-    rpt_call<RS, 1>(a.rp, roe, AmL, AL, A1L, amm, bmA, bpA);
-    rpt_call<RS, 1>(a.rp, roe, Am, A0, A1, apm, bmP, bpP);
+    rpt_call<RS, 1, WIDE>(a.rp, roe, AmL, AL, A1L, amm, bmA, bpA);
+    rpt_call<RS, 1, WIDE>(a.rp, roe, Am, A0, A1, apm, bmP, bpP);
     T bmAn[ME], bpAn[ME];
     from_right(bmA, bmAn);
     from_right(bpA, bpAn);
@@ -222,27 +222,24 @@ constexpr int unsplit_waves() {
   return (AUX || CAPA) ? 1 : UnsplitWaves<RS, T>::value;
 }
 
-// `wid`: this wavefront's index among the a.nstrips * a.nrb of the launch.
-// Returns this lane's Courant number (0 past the last strip); the kernel adds it
-// to *a.cfl_bits (one atomic per workgroup where every wavefront of the
-// workgroup reaches that point, else one per wavefront).
-template <class RS, typename T, bool KAHAN, bool AUX = false, bool CAPA = false>
-__device__ __forceinline__ double unsplit_body(const UnsplitArgs<T>& a, int wid) {
+// The march of wavefront `wid` from row `first` on, its Courant numbers' maxima
+// added to smx, smy; returns as march_both wants it.
+template <class RS, typename T, bool KAHAN, bool AUX, bool CAPA, bool WIDE>
+__device__ __forceinline__ int unsplit_march(const UnsplitArgs<T>& a, int wid, int first, T& smx,
+                                             T& smy) {
   constexpr int ME = RS::meqn, MW = RS::mwaves, NA = UNSPLIT_MAX_AUX;
   static_assert(AUX || (RS::maux == 0 && !CAPA), "aux solvers and capacity need the aux window");
   using Roe = typename RS::Roe;
   const int lane = threadIdx.x & 63;
-  if (wid >= a.nstrips * a.nrb) return 0.0;   // uniform per wavefront
   const int strip = wid % a.nstrips, rb = wid / a.nstrips;
   const int mx = a.gout.mx, my = a.gout.my;
   const int c = 1 + strip * 60 - 2 + lane;
-  const int j0 = 1 + rb * a.H;
-  const int jend = min(j0 + a.H, my + 1);
+  const int j0 = first;
+  const int jend = min(1 + (rb + 1) * a.H, my + 1);
   const bool out_col = lane >= 2 && lane < 62 && c >= 1 && c <= mx;
   const bool cflx_col = lane >= 1 && c >= 1 && c <= mx + 1;   // lane 0 has no left state
   const bool cfly_col = c >= 0 && c <= mx + 1;
   const T dtdx = a.dtdx, dtdy = a.dtdy, hy = T(0.5) * a.dtdy;
-  T smx = T(0), smy = T(0);
 
   T Qm[ME], Q0[ME], Q1[ME];
   T Am[NA], A0[NA], A1[NA];   // aux rows t-1, t, t+1 (AUX)
@@ -255,7 +252,25 @@ __device__ __forceinline__ double unsplit_body(const UnsplitArgs<T>& a, int wid)
   load_aux<AUX>(a, c, j0 - 2, Am);
   load_aux<AUX>(a, c, j0 - 1, A0);
   load_aux<AUX>(a, c, j0, A1);
-  xpass<RS, AUX, CAPA>(a, Q0, Am, A0, A1, cflx_col && j0 - 1 >= 0, smx, xr);
+  Watch<RS, T> seen;
+  if (!WIDE) {
+    seen.see(Qm);
+    seen.see(Q0);
+    seen.see(Q1);
+    if (!seen.all_tame()) return j0;
+  }
+  T Wt[MW][ME], st[MW], amt[ME], apt[ME], dotl[MW];
+  Roe roet;
+  {
+    xpass<RS, AUX, CAPA, WIDE>(a, Q0, Am, A0, A1, cflx_col && j0 - 1 >= 0, smx, xr);
+    T Wp[MW][ME], sp[MW], amp[ME], app[ME];
+    Roe roep;
+    rpn_call<RS, 2, WIDE>(a.rp, Qm, Q0, Am, A0, Wp, sp, amp, app, roep);
+    if (cfly_col && j0 - 1 >= 1) cfl_y<CAPA>(a, smy, sp, Am, A0);
+    rpn_call<RS, 2, WIDE>(a.rp, Q0, Q1, A0, A1, Wt, st, amt, apt, roet);
+    if (cfly_col && j0 <= my + 1) cfl_y<CAPA>(a, smy, st, A0, A1);
+    wave_dots<ME, MW>(Wp, Wt, dotl);
+  }
   T acc_prev[ME], acc_cur[ME], qold_prev[ME], qold_cur[ME];
 #pragma unroll
   for (int m = 0; m < ME; m++) {
@@ -264,17 +279,6 @@ __device__ __forceinline__ double unsplit_body(const UnsplitArgs<T>& a, int wid)
     qold_cur[m] = Q1[m];
     acc_prev[m] = T(0);
     qold_prev[m] = T(0);
-  }
-  T Wt[MW][ME], st[MW], amt[ME], apt[ME], dotl[MW];
-  Roe roet;
-  {
-    T Wp[MW][ME], sp[MW], amp[ME], app[ME];
-    Roe roep;
-    rpn_call<RS, 2>(a.rp, Qm, Q0, Am, A0, Wp, sp, amp, app, roep);
-    if (cfly_col && j0 - 1 >= 1) cfl_y<CAPA>(a, smy, sp, Am, A0);
-    rpn_call<RS, 2>(a.rp, Q0, Q1, A0, A1, Wt, st, amt, apt, roet);
-    if (cfly_col && j0 <= my + 1) cfl_y<CAPA>(a, smy, st, A0, A1);
-    wave_dots<ME, MW>(Wp, Wt, dotl);
   }
 #pragma unroll
   for (int m = 0; m < ME; m++) Q0[m] = Q1[m];
@@ -288,7 +292,7 @@ __device__ __forceinline__ double unsplit_body(const UnsplitArgs<T>& a, int wid)
     load_row2<ME>(a.qin, a.gin, a.bc, a.ng, col, t + 1, Q1);
     load_aux<AUX>(a, c, t + 1, A1);
     // ---- x-slice t
-    xpass<RS, AUX, CAPA>(a, Q0, Am, A0, A1, cflx_col && t <= my + 1, smx, xr);
+    xpass<RS, AUX, CAPA, WIDE>(a, Q0, Am, A0, A1, cflx_col && t <= my + 1, smx, xr);
     T acc_next[ME];
     if constexpr (CAPA) {
       const T km = capa_of(a, Am), k0 = capa_of(a, A0), k1 = capa_of(a, A1);
@@ -308,9 +312,11 @@ __device__ __forceinline__ double unsplit_body(const UnsplitArgs<T>& a, int wid)
       }
     }
     // ---- y-interface t+1 (rows t, t+1); limit interface t
+    const T smy_before = smy;
+    if (!WIDE) seen.see(Q1);
     T Wn[MW][ME], sn[MW], amn[ME], apn[ME], dotn[MW];
     Roe roen;
-    rpn_call<RS, 2>(a.rp, Q0, Q1, A0, A1, Wn, sn, amn, apn, roen);
+    rpn_call<RS, 2, WIDE>(a.rp, Q0, Q1, A0, A1, Wn, sn, amn, apn, roen);
     if (cfly_col && t + 1 <= my + 1) cfl_y<CAPA>(a, smy, sn, A0, A1);
     // dtdy1d of rows t-1 (imp = 1 side of interface t) and t (imp = 2 side)
     const T dyA = dy1d<CAPA>(a, Am), dyP = dy1d<CAPA>(a, A0);
@@ -343,8 +349,8 @@ __device__ __forceinline__ double unsplit_body(const UnsplitArgs<T>& a, int wid)
         from_left(A0, A0L);
         from_right(A0, A0R);
       }
-      rpt_call<RS, 2>(a.rp, roet, AmL, Am, AmR, amm, bmA, bpA);
-      rpt_call<RS, 2>(a.rp, roet, A0L, A0, A0R, apm, bmP, bpP);
+      rpt_call<RS, 2, WIDE>(a.rp, roet, AmL, Am, AmR, amm, bmA, bpA);
+      rpt_call<RS, 2, WIDE>(a.rp, roet, A0L, A0, A0R, apm, bmP, bpP);
     }
     const T hyA = CAPA ? T(0.5) * dyA : hy, hyP = CAPA ? T(0.5) * dyP : hy;
     if (t > j0) {
@@ -419,7 +425,26 @@ __device__ __forceinline__ double unsplit_body(const UnsplitArgs<T>& a, int wid)
       for (int m = 0; m < ME; m++) Wt[w][m] = Wn[w][m];
     }
     roet = roen;
+    if (!WIDE && !seen.all_tame()) {   // row t-1's limiter has used row t+1
+      smy = smy_before;
+      return max(j0, t - 1);
+    }
   }
+  return kMarched;
+}
+
+// `wid`: this wavefront's index among the a.nstrips * a.nrb of the launch.
+// Returns this lane's Courant number (0 past the last strip); the kernel adds it
+// to *a.cfl_bits (one atomic per workgroup where every wavefront of the
+// workgroup reaches that point, else one per wavefront).
+template <class RS, typename T, bool KAHAN, bool AUX = false, bool CAPA = false>
+__device__ __forceinline__ double unsplit_body(const UnsplitArgs<T>& a, int wid) {
+  if (wid >= a.nstrips * a.nrb) return 0.0;   // uniform per wavefront
+  T smx = T(0), smy = T(0);
+  march_both<RS, T>(a.rp.wide, 1 + wid / a.nstrips * a.H,
+                    [&](auto kind, int first) __attribute__((always_inline)) {
+    return unsplit_march<RS, T, KAHAN, AUX, CAPA, decltype(kind)::value>(a, wid, first, smx, smy);
+  });
   double cfl, cy;
   if constexpr (CAPA) {   // smx, smy hold Courant numbers
     cfl = (double)smx;

@@ -123,9 +123,13 @@ __global__ void __launch_bounds__(256) k_flux3(const Step3Args<double> a) {
     T Q[ME], QL[ME];
     load_cell3<ME>(a.qin, a.g, a.bc, a.ng, i, j, k, Q);
     from_left(Q, QL);
+    Watch<RS, T> seen;
+    seen.see(Q);
+    auto slice = [&](auto kind) __attribute__((always_inline)) {
+    constexpr bool WIDE = decltype(kind)::value;
     T W[MW][ME], s[MW], am[ME], ap[ME];
     typename RS::Roe roe;
-    RS::template rpn<DIR>(a.rp, QL, Q, W, s, am, ap, roe);
+    RS::template rpn<DIR, WIDE>(a.rp, QL, Q, W, s, am, ap, roe);
     // Courant number over interfaces 1..n+1 (flux3.f90:214-221)
     T smax = T(0);
     if (lane >= 1 && inside && c >= 1 && c <= n + 1) {
@@ -187,13 +191,13 @@ __global__ void __launch_bounds__(256) k_flux3(const Step3Args<double> a) {
       bmcq[m] = bpcq[m] = cmcq[m] = cpcq[m] = T(0);
     }
     if (m3 > 0) {
-      RS::template rpt3<DIR, 2>(roe, am, bmam, bpam);
-      RS::template rpt3<DIR, 2>(roe, ap, bmap, bpap);
-      RS::template rpt3<DIR, 3>(roe, am, cmam, cpam);
-      RS::template rpt3<DIR, 3>(roe, ap, cmap, cpap);
+      RS::template rpt3<DIR, 2, WIDE>(roe, am, bmam, bpam);
+      RS::template rpt3<DIR, 2, WIDE>(roe, ap, bmap, bpap);
+      RS::template rpt3<DIR, 3, WIDE>(roe, am, cmam, cpam);
+      RS::template rpt3<DIR, 3, WIDE>(roe, ap, cmap, cpap);
       if (m3 == 2) {
-        RS::template rpt3<DIR, 2>(roe, cq, bmcq, bpcq);
-        RS::template rpt3<DIR, 3>(roe, cq, cmcq, cpcq);
+        RS::template rpt3<DIR, 2, WIDE>(roe, cq, bmcq, bpcq);
+        RS::template rpt3<DIR, 3, WIDE>(roe, cq, cmcq, cpcq);
       }
     }
     // One family of transverse modifications (gadd: family 0, split direction
@@ -217,16 +221,16 @@ __global__ void __launch_bounds__(256) k_flux3(const Step3Args<double> a) {
         T x2[ME];
   #pragma unroll
         for (int m = 0; m < ME; m++) x2[m] = m4 == 2 ? zpap[m] - T(3) * zpcq[m] : zpap[m];
-        RS::template rpt3<DIR, ICO>(roe, x2, cmcpap, cpcpap);
+        RS::template rpt3<DIR, ICO, WIDE>(roe, x2, cmcpap, cpcpap);
   #pragma unroll
         for (int m = 0; m < ME; m++) x2[m] = m4 == 2 ? zpam[m] + T(3) * zpcq[m] : zpam[m];
-        RS::template rpt3<DIR, ICO>(roe, x2, cmcpam, cpcpam);
+        RS::template rpt3<DIR, ICO, WIDE>(roe, x2, cmcpam, cpcpam);
   #pragma unroll
         for (int m = 0; m < ME; m++) x2[m] = m4 == 2 ? zmap[m] - T(3) * zmcq[m] : zmap[m];
-        RS::template rpt3<DIR, ICO>(roe, x2, cmcmap, cpcmap);
+        RS::template rpt3<DIR, ICO, WIDE>(roe, x2, cmcmap, cpcmap);
   #pragma unroll
         for (int m = 0; m < ME; m++) x2[m] = m4 == 2 ? zmam[m] + T(3) * zmcq[m] : zmam[m];
-        RS::template rpt3<DIR, ICO>(roe, x2, cmcmam, cpcmam);
+        RS::template rpt3<DIR, ICO, WIDE>(roe, x2, cmcmam, cpcmam);
       }
   #pragma unroll
       for (int m = 0; m < ME; m++) {
@@ -286,6 +290,10 @@ __global__ void __launch_bounds__(256) k_flux3(const Step3Args<double> a) {
     // hadd's double-transverse input: the y-like splits with the correction
     family(std::integral_constant<int, 1>(), cmam, cpam, cmap, cpap, cmcq, cpcq, bmam, bpam,
            bmap, bpap, bmcq, bpcq, dt1);
+    };
+    // uniform over the wavefront (see Divided)
+    if (__builtin_expect(!a.rp.wide && seen.all_tame(), 1)) slice(std::false_type());
+    else slice(std::true_type());
   }
   block_atomic_max(cfl_wave, a.cfl_bits);
 }
