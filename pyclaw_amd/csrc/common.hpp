@@ -260,7 +260,7 @@ __device__ __forceinline__ void limit_waves(T (&W)[MW][ME], const T (&s)[MW], co
     wnorm2[w] = T(0);
 #pragma unroll
     for (int m = 0; m < ME; m++) wnorm2[w] = wnorm2[w] + W[w][m] * W[w][m];
-    r[w] = (s[w] > T(0) ? dotl[w] : dotr[w]) / wnorm2[w];
+    r[w] = quo(s[w] > T(0) ? dotl[w] : dotr[w], wnorm2[w]);
     usual = usual && (mthlim[w] == 1 || mthlim[w] == 4);
   }
   if (__builtin_expect(usual, 1)) {

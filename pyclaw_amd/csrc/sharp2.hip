@@ -182,8 +182,8 @@ __device__ __forceinline__ T weno_char_side(T hm2, T hm1, T h0, T hp1, T hp2, in
   T s1, s3;
   if constexpr (sizeof(T) == 4) {
     // the same weights as d_k / (eps + beta_k)^2: no fourth powers to underflow
-    const T r1 = T(1) / tt1, r2 = T(6) / tt2, r3 = T(3) / tt3;
-    const T t0 = T(1) / (r1 + r2 + r3);
+    const T r1 = quo(T(1), tt1), r2 = quo(T(6), tt2), r3 = quo(T(3), tt3);
+    const T t0 = quo(T(1), r1 + r2 + r3);
     s1 = r1 * t0;
     s3 = r3 * t0;
   } else {   // the reference's products of two squares, bit for bit
@@ -216,7 +216,7 @@ struct Evec<Shallow<T>, IXY, T, WIDE> {
     evr[0][0] = T(1); evr[mu][0] = u - c; evr[mv][0] = v;
     evr[0][1] = T(0); evr[mu][1] = T(0); evr[mv][1] = T(1);
     evr[0][2] = T(1); evr[mu][2] = u + c; evr[mv][2] = v;
-    T r2c = T(0.5) / c;
+    T r2c = quo(T(0.5), c);
     evl[0][0] = (u + c) * r2c; evl[0][mu] = -r2c; evl[0][mv] = T(0);
     evl[1][0] = -v; evl[1][mu] = T(0); evl[1][mv] = T(1);
     evl[2][0] = -(u - c) * r2c; evl[2][mu] = r2c; evl[2][mv] = T(0);
@@ -241,7 +241,7 @@ struct Evec<Euler<T>, IXY, T, WIDE> {
     evr[0][2] = T(1); evr[mu][2] = u; evr[mv][2] = v; evr[3][2] = q2;
     evr[0][3] = T(1); evr[mu][3] = u + c; evr[mv][3] = v; evr[3][3] = H + u * c;
     T b1 = gamma1 / (c * c), b2 = q2 * b1;
-    T r2c = T(0.5) / c;
+    T r2c = quo(T(0.5), c);
     evl[0][0] = T(0.5) * b2 + u * r2c; evl[0][mu] = -(T(0.5) * b1 * u + r2c);
     evl[0][mv] = -T(0.5) * b1 * v; evl[0][3] = T(0.5) * b1;
     evl[1][0] = -v; evl[1][mu] = T(0); evl[1][mv] = T(1); evl[1][3] = T(0);
