@@ -12,6 +12,9 @@
 #include "variant.hpp"  // first: selects the arithmetic variant
 #include <stdlib.h>
 
+#include <algorithm>
+#include <cmath>
+
 #include "launch.hpp"
 #include "unsplit.hpp"
 
@@ -24,9 +27,7 @@ __global__ void __launch_bounds__(256)
     k_unsplit(const UnsplitArgs<T> a) {
   // one Courant-number atomic per workgroup: one per wavefront serialises
   // (same address) over the thousands of wavefronts of a large grid
-  block_atomic_max(
-      unsplit_body<RS, T, KAHAN, AUX, CAPA>(a, blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)),
-      a.cfl_bits);
+  block_atomic_max(unsplit_block<RS, T, KAHAN, AUX, CAPA>(a, (int)xcd_block()), a.cfl_bits);
 }
 
 // Device-resident stepping: one launch = one attempted step of
@@ -47,8 +48,7 @@ __global__ void __launch_bounds__(256)
   a.dtdx = T(dt / bufs.dx);
   a.dtdy = T(dt / bufs.dy);
   a.cfl_bits = &ctl->cfl_bits;
-  const int wid = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  block_atomic_max(unsplit_body<RS, T, KAHAN>(a, wid), a.cfl_bits);
+  block_atomic_max(unsplit_block<RS, T, KAHAN>(a, (int)xcd_block()), a.cfl_bits);
 }
 
 // The step's control after it (step_ctl_apply).
@@ -64,37 +64,40 @@ namespace claw {
 namespace CLAW_VNS {
 
 namespace {
-// Rows per wavefront (march length H).  Each wavefront recomputes the x-slices of
-// 2 halo rows, so long marches waste less; but the grid must also fill the
-// device: with R wavefronts resident at once (from the kernel's occupancy), a
-// launch of W wavefronts runs in ceil(W / R) rounds of H + 2 row-steps each.
-// H minimises that product (ties: the longer march).  CLAWHIP_UNSPLIT_ROWS
-// overrides the choice (tuning sweeps).
+// Blocks per strip.  Four wavefronts of a block solve its rows and one more, each
+// after a warm-up worth about a row; a launch of k rounds of resident blocks costs
+// k times that, and the smallest such cost is taken.  Blocks of at most 128 rows:
+// longer ones leave nothing to fill in behind the early wavefronts (4096^2 FP64
+// acoustics, 64 / 128 / 186 / 256 rows: 402, 403, 411, 438 us).  At least 7, two
+// solves a wavefront: a grid that fills less than one round takes it (256^2 FP64
+// acoustics, 3 / 7 / 11 / 15 / 19 rows: 11.2, 10.7, 12.2, 14.4, 16.3 us).
+// CLAWHIP_UNSPLIT_ROWS overrides the solves per wavefront (tuning sweeps).
 template <class Kernel>
-int choose_rows(Kernel kernel, int nstrips, int my, int waves_hint) {
+int choose_blocks(Kernel kernel, int nstrips, int my, int waves_hint) {
+  if (const char* env = getenv("CLAWHIP_UNSPLIT_ROWS")) {
+    int h = atoi(env);
+    if (h >= 1 && h <= 4096) return (my + 4 * h - 2) / (4 * h - 1);
+  }
   // beyond two wavefronts per SIMD the measured gain of a third is smaller than
   // the halo rows the shorter marches add, so count at most two, unless the
   // kernel is compiled for more (unsplit_waves)
-  const long long resident = resident_waves((const void*)kernel, waves_hint > 2 ? waves_hint : 2);
-  if (resident == 0) return 16;
-  if (const char* env = getenv("CLAWHIP_UNSPLIT_ROWS")) {
-    int h = atoi(env);
-    if (h >= 1 && h <= 4096) return h;
-  }
-  // the shortest march considered: 3 rows.  A grid that fills less than one
-  // resident round takes it (256^2 FP64 acoustics step: H = 1, 2, 3, 4, 6 ran
-  // 26.8, 21.3, 21.0, 22.0, 25.0 us); shorter marches add more wavefronts than
-  // they save in each one's dependent row chain
-  int best = 16;
-  long long best_cost = -1;
-  for (int h = 3; h <= 64; h++) {
-    const long long waves = (long long)nstrips * ((my + h - 1) / h);
-    const long long cost = ((waves + resident - 1) / resident) * (long long)(h + 2);
-    if (best_cost < 0 || cost < best_cost || (cost == best_cost && h > best)) {
-      best = h;
+  const long long resident =
+      resident_waves((const void*)kernel, waves_hint > 2 ? waves_hint : 2) / 4;
+  if (resident == 0) return (my + 63) / 64;
+  const int most = (my + 6) / 7, least = (my + 127) / 128;
+  const double all = (double)my * nstrips / (4.0 * resident);   // rows of a wavefront, one round
+  int best = most;
+  double best_cost = 1e300;
+  for (long long k = 1; all + k < best_cost; k++) {
+    const int n = (int)std::min((long long)most, k * resident / nstrips);
+    if (n < least) continue;
+    const double rounds = std::ceil((double)nstrips * n / resident);
+    const double cost = rounds * (((double)my / n + 1) / 4 + 1);
+    if (cost < best_cost) {
+      best = n;
       best_cost = cost;
     }
-    if ((my + h - 1) / h == 1) break;
+    if (n == most) break;
   }
   return best;
 }
@@ -123,14 +126,12 @@ int run_unsplit(const clawhip_rp& rp, const void* q_in, const Geom& gin, void* q
   for (int w = 0; w < kMaxWaves; w++) a.mthlim[w] = w < RS::mwaves ? mthlim[w] : 0;
   a.dtdx = T(dt / dx); a.dtdy = T(dt / dy);
   a.nstrips = (gout.mx + 59) / 60;
-  a.H = choose_rows(k_unsplit<RS, T, KAHAN, AUX, CAPA>, a.nstrips, gout.my,
-                    unsplit_waves<RS, T, AUX, CAPA>());
-  a.nrb = (gout.my + a.H - 1) / a.H;
+  a.nrb = choose_blocks(k_unsplit<RS, T, KAHAN, AUX, CAPA>, a.nstrips, gout.my,
+                        unsplit_waves<RS, T, AUX, CAPA>());
   a.qin = (const T*)q_in; a.qout = (T*)q_out;
   a.comp_in = (const T*)comp_in; a.comp_out = (T*)comp_out;
   a.cfl_bits = cfl_bits;
-  long long waves = (long long)a.nstrips * a.nrb;
-  int blocks = (int)((waves + 3) / 4);
+  const unsigned blocks = (unsigned)((long long)a.nstrips * a.nrb);
   hipLaunchKernelGGL((k_unsplit<RS, T, KAHAN, AUX, CAPA>), dim3(blocks), dim3(256), 0, stream, a);
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : (int)e;
@@ -148,12 +149,10 @@ int run_unsplit_ctl(const clawhip_rp& rp, const Geom& g, const int* lo, const in
   for (int w = 0; w < kMaxWaves; w++) a.mthlim[w] = w < RS::mwaves ? mthlim[w] : 0;
   a.dtdx = T(0); a.dtdy = T(0);
   a.nstrips = (g.mx + 59) / 60;
-  a.H = choose_rows(k_unsplit_ctl<RS, T, KAHAN>, a.nstrips, g.my, unsplit_waves<RS, T>());
-  a.nrb = (g.my + a.H - 1) / a.H;
+  a.nrb = choose_blocks(k_unsplit_ctl<RS, T, KAHAN>, a.nstrips, g.my, unsplit_waves<RS, T>());
   a.qin = nullptr; a.qout = nullptr; a.comp_in = nullptr; a.comp_out = nullptr;
   a.cfl_bits = nullptr;
-  long long waves = (long long)a.nstrips * a.nrb;
-  int blocks = (int)((waves + 3) / 4);
+  const unsigned blocks = (unsigned)((long long)a.nstrips * a.nrb);
   for (int n = 0; n < nsteps; n++) {
     hipLaunchKernelGGL((k_unsplit_ctl<RS, T, KAHAN>), dim3(blocks), dim3(256), 0, stream, a,
                        ctl, bufs);

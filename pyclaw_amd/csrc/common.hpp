@@ -209,6 +209,13 @@ __device__ __forceinline__ void wave_atomic_max(double v, unsigned long long* ds
   if ((threadIdx.x & 63) == 0 && v > 0.0) atomicMax(dst, (unsigned long long)__double_as_longlong(v));
 }
 
+// Each XCD takes a contiguous range of the blocks (the dispatcher deals them out
+// in turn over 8 XCDs), so that neighbouring blocks meet in one L2.
+__device__ __forceinline__ long long xcd_block() {
+  const unsigned n = gridDim.x, b = blockIdx.x, per = n / 8, rest = n % 8, x = b % 8, i = b / 8;
+  return (long long)x * per + min(x, rest) + i;
+}
+
 // The same for a workgroup of up to 256 threads: one atomic per workgroup.
 // Every thread of the workgroup calls it (it holds a barrier).
 __device__ __forceinline__ void block_atomic_max(double v, unsigned long long* dst) {

@@ -2,9 +2,9 @@
 // Riemann solver and method) advanced together: every launch sweeps all
 // members, each with its own dt and device step controller.
 //
-// The members' wavefronts are concatenated into one grid (largest members
-// first, so the small ones fill the tail); a wavefront finds its member by
-// binary search over the members' first-wavefront offsets and then runs the
+// The members' workgroups are concatenated into one grid (largest members
+// first, so the small ones fill the tail); a workgroup finds its member by
+// binary search over the members' first-block offsets and then runs the
 // same step body as the single-grid kernel (unsplit.hpp).  The last wavefront of
 // a member applies that member's accept/reject and next dt (stepctl.hpp).  A
 // step of the whole ensemble is one launch with no host synchronisation, so
@@ -25,7 +25,7 @@ namespace CLAW_VNS {
 struct EnsMember {
   int mx, my;
   int nstrips, nrb;
-  long long base;             // first wavefront of this member
+  long long base;             // first block of this member
   const void* q[2];
   void* comp[2];
   double dx, dy;
@@ -33,12 +33,11 @@ struct EnsMember {
 };
 
 struct EnsHeader {
-  int n, H, ng, order, trans;
+  int n, ng, order, trans;
   int mthlim[4];
   BCSpec bc;
   RPParams<double> rp64;
   RPParams<float> rp32;
-  long long waves;
 };
 
 constexpr long long kEnsAlign = 256;
@@ -60,13 +59,12 @@ __device__ __forceinline__ const RPParams<float>& ens_rp<float>(const EnsHeader&
 template <class RS, typename T, bool KAHAN>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(unsplit_waves<RS, T>())))
 k_ens_step(const EnsHeader* __restrict__ hdr, const EnsMember* __restrict__ mem) {
-  const long long gw = (long long)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  if (gw >= hdr->waves) return;
-  // member k: the last one whose first wavefront is <= gw
+  const long long blk = blockIdx.x;
+  // member k: the last one whose first block is <= blk
   int lo = 0, hi = hdr->n - 1;
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
-    if (mem[mid].base <= gw) lo = mid;
+    if (mem[mid].base <= blk) lo = mid;
     else hi = mid - 1;
   }
   const EnsMember& m = mem[lo];
@@ -82,7 +80,7 @@ k_ens_step(const EnsHeader* __restrict__ hdr, const EnsMember* __restrict__ mem)
   a.bc = hdr->bc;
   a.ng = hdr->ng; a.order = hdr->order; a.trans = hdr->trans;
   for (int w = 0; w < 4; w++) a.mthlim[w] = hdr->mthlim[w];
-  a.H = hdr->H; a.nstrips = m.nstrips; a.nrb = m.nrb;
+  a.nstrips = m.nstrips; a.nrb = m.nrb;
   a.qin = (const T*)m.q[cur];
   a.qout = (T*)m.q[1 - cur];
   a.comp_in = (const T*)m.comp[cur];
@@ -90,10 +88,7 @@ k_ens_step(const EnsHeader* __restrict__ hdr, const EnsMember* __restrict__ mem)
   a.dtdx = T(dt / m.dx);
   a.dtdy = T(dt / m.dy);
   a.cfl_bits = &ctl->cfl_bits;
-  const int local = (int)(gw - m.base);
-  // the members' Courant numbers go to their own controllers (many
-  // addresses), and a workgroup may span members that return above
-  wave_atomic_max(unsplit_body<RS, T, KAHAN>(a, local), a.cfl_bits);
+  block_atomic_max(unsplit_block<RS, T, KAHAN>(a, (int)(blk - m.base)), a.cfl_bits);
 }
 
 // Every member's step control after the step launch (step_ctl_apply), one
@@ -117,20 +112,20 @@ long long ens_resident_waves() {
   return r > 0 ? r : 1024;
 }
 
-long long ens_waves(const std::vector<EnsMember>& v, int H) {
-  long long w = 0;
-  for (const auto& m : v) w += (long long)((m.mx + 59) / 60) * ((m.my + H - 1) / H);
-  return w;
-}
+// Blocks of a member at h rows per wavefront: four wavefronts solve the block's rows
+// and one more.
+int ens_blocks(const EnsMember& m, int h) { return (m.my + 4 * h - 2) / (4 * h - 1); }
 
 // Rows per wavefront for the whole ensemble: the single-grid rule
-// (rounds x (H + 2)) over the total wavefront count.
+// (rounds x (h + 1)) over the total block count.
 int ens_choose_rows(const std::vector<EnsMember>& v) {
-  const long long R = ens_resident_waves();
+  const long long R = (ens_resident_waves() + 3) / 4;
   int best = 16;
   long long best_cost = -1;
-  for (int h = 2; h <= 64; h++) {
-    const long long cost = ((ens_waves(v, h) + R - 1) / R) * (h + 2);
+  for (int h = 2; h <= 32; h++) {
+    long long blocks = 0;
+    for (const auto& m : v) blocks += (long long)((m.mx + 59) / 60) * ens_blocks(m, h);
+    const long long cost = ((blocks + R - 1) / R) * (h + 1);
     if (best_cost < 0 || cost < best_cost || (cost == best_cost && h > best)) {
       best = h;
       best_cost = cost;
@@ -142,9 +137,10 @@ int ens_choose_rows(const std::vector<EnsMember>& v) {
 template <class RS, typename T, bool KAHAN>
 void ens_launch(const EnsHeader* h, const EnsMember* m, const long long* waves, int nsteps,
                 hipStream_t s) {
-  // wavefronts per workgroup: 1, 2 or 4 (the autotuner's second parameter)
+  // wavefronts per workgroup: 1, 2 or 4 (the autotuner's second parameter); fewer
+  // march more of the block's rows each
   const long long wpb = (waves[2] == 1 || waves[2] == 2) ? waves[2] : 4;
-  const unsigned blocks = (unsigned)((waves[0] + wpb - 1) / wpb);
+  const unsigned blocks = (unsigned)(waves[0] / 4);
   const unsigned ctl_blocks = (unsigned)((waves[1] + 255) / 256);
   for (int n = 0; n < nsteps; n++) {
     hipLaunchKernelGGL((k_ens_step<RS, T, KAHAN>), dim3(blocks), dim3((unsigned)(64 * wpb)), 0,
@@ -189,23 +185,22 @@ int ensemble_prepare(const clawhip_rp& rp, const clawhip_ens_member* members, in
   long long base = 0;
   for (auto& m : v) {
     m.nstrips = (m.mx + 59) / 60;
-    m.nrb = (m.my + H - 1) / H;
+    m.nrb = ens_blocks(m, H);
     m.base = base;
     base += (long long)m.nstrips * m.nrb;
   }
   EnsHeader h;
-  h.n = n; h.H = H; h.ng = ng; h.order = method[1]; h.trans = method[2];
+  h.n = n; h.ng = ng; h.order = method[1]; h.trans = method[2];
   for (int w = 0; w < 4; w++) h.mthlim[w] = mthlim[w];
   h.bc = to_bc(lo, hi, refl, 2);
   h.rp64 = to_params<double>(rp);
   h.rp32 = to_params<float>(rp);
-  h.waves = base;
   std::vector<char> buf((size_t)ensemble_table_bytes(n), 0);
   ::memcpy(buf.data(), &h, sizeof(h));
   ::memcpy(buf.data() + ens_members_offset(), v.data(), (size_t)n * sizeof(EnsMember));
   hipError_t e = hipMemcpy(table_dev, buf.data(), buf.size(), hipMemcpyHostToDevice);
   if (e != hipSuccess) return (int)e;
-  waves[0] = base; waves[1] = n;   // wavefronts of a step launch; members
+  waves[0] = 4 * base; waves[1] = n;   // wavefronts of a step launch; members
   waves[2] = 4;                    // wavefronts per workgroup (the caller may change it)
   return 0;
 }

@@ -6,7 +6,7 @@
 // Work decomposition (wave64):
 //   * a wavefront owns a strip of 64 columns c0-2 .. c0+61 and writes the 60
 //     columns c0 .. c0+59; lanes 0,1,62,63 only supply neighbour data.
-//   * it marches down rows j0 .. j0+H-1.  x-interfaces of a row are computed
+//   * it marches down its share of the rows.  x-interfaces of a row are computed
 //     lane-parallel (neighbour states, waves and fluctuations arrive by
 //     cross-lane moves); y-interfaces are lane-local, kept in a register
 //     window so each one is solved once.
@@ -37,7 +37,7 @@ struct UnsplitArgs {
   int ng, order, trans;
   int mthlim[kMaxWaves];
   T dtdx, dtdy;
-  int H, nstrips, nrb;
+  int nstrips, nrb;
   const T* qin;
   T* qout;
   const T* comp_in;              // Kahan compensation (FP32 path), output geometry
@@ -74,7 +74,11 @@ template <typename T>
 __device__ __forceinline__ T capa_of(const UnsplitArgs<T>& a, const T (&A)[UNSPLIT_MAX_AUX]) {
   T r = A[0];
 #pragma unroll
-  for (int k = 1; k < UNSPLIT_MAX_AUX; k++) r = k == a.capa ? A[k] : r;
+  for (int k = 1; k < UNSPLIT_MAX_AUX; k++) {
+    T v = A[k];
+    asm("" : "+v"(v));   // a choice of values: one of addresses would put A into memory
+    r = k == a.capa ? v : r;
+  }
   return r;
 }
 
@@ -197,8 +201,8 @@ __device__ __forceinline__ void cfl_y(const UnsplitArgs<T>& a, T& acc, const T (
 // 512 / that number), where a solver gains from more than the compiler's own
 // choice.  FP64 acoustics (180 VGPRs, 2 per SIMD) and FP32 + Kahan Euler (172
 // VGPRs, 2 per SIMD) fit 168 VGPRs with a few spilled dwords:
-//   - 4096^2 FP64 acoustics step: 476 -> 431 us;
-//   - 1024^2 FP32 + Kahan Euler step: 76.7 -> 71.0 us.
+//   - 4096^2 FP64 acoustics step: 476 -> 431 us (404 since);
+//   - 1024^2 FP32 + Kahan Euler step: 76.7 -> 71.0 us (52 since).
 // Forcing FP64 Euler (314 VGPRs) to 3 per SIMD doubles its time (heavy
 // spills); FP64 acoustics at 4 per SIMD (37 spilled dwords) takes 907 us.
 // 1 = no constraint.  The aux and capacity forms keep the compiler's choice.
@@ -222,24 +226,100 @@ constexpr int unsplit_waves() {
   return (AUX || CAPA) ? 1 : UnsplitWaves<RS, T>::value;
 }
 
-// The march of wavefront `wid` from row `first` on, its Courant numbers' maxima
-// added to smx, smy; returns as march_both wants it.
+// What a row still lacks when its own wavefront's march ends: its sums so far and
+// its lower y-interface's parts.
+template <class RS, typename T>
+struct RowEnd {
+  T acc[RS::meqn], qold[RS::meqn], qaddy[RS::meqn], hbm[RS::meqn], hbp[RS::meqn], Fy[RS::meqn];
+  T am[RS::meqn];   // upper y-interface: amdq
+  T capa;           // the row's capacity (CAPA)
+};
+
+// A row's sums less the part across the slice of the x-slice above.
+template <bool CAPA, int ME, typename T>
+__device__ __forceinline__ void take_g1(const UnsplitArgs<T>& a, T capa, const T (&g1)[ME],
+                                        T (&acc)[ME]) {
+#pragma unroll
+  for (int m = 0; m < ME; m++) {
+    if constexpr (CAPA) acc[m] = acc[m] - (a.dtdy * g1[m]) / capa;
+    else acc[m] = acc[m] - a.dtdy * g1[m];
+  }
+}
+
+// Row `row` (its sums after take_g1) completed with its upper y-interface's
+// second-order flux Fy and two parts bm, bp of amdq across the slice, and stored.
+template <class RS, bool KAHAN, bool CAPA, typename T>
+__device__ __forceinline__ void finish_row(const UnsplitArgs<T>& a, int c, int row, bool out_col,
+                                           const RowEnd<RS, T>& e, const T (&Fy)[RS::meqn],
+                                           const T (&bm)[RS::meqn], const T (&bp)[RS::meqn]) {
+  constexpr int ME = RS::meqn;
+  const T dtdx = a.dtdx, dtdy = a.dtdy, dyA = CAPA ? a.dtdy / e.capa : a.dtdy;
+  const T hyA = CAPA ? T(0.5) * dyA : T(0.5) * a.dtdy;
+  T g1y[ME], g2y[ME], g2l[ME], g1r[ME];
+#pragma unroll
+  for (int m = 0; m < ME; m++) {
+    g1y[m] = (T(0) - hyA * bm[m]) - e.hbm[m];
+    g2y[m] = (T(0) - hyA * bp[m]) - e.hbp[m];
+  }
+  from_left(g2y, g2l);
+  from_right(g1y, g1r);
+  T upd[ME];
+  if constexpr (CAPA) {
+    const T km = e.capa;
+#pragma unroll
+    for (int m = 0; m < ME; m++) {
+      T qaddy = e.qaddy[m] - dyA * e.am[m];
+      T v = e.acc[m] + (dtdx * g2l[m]) / km;
+      v = (v + qaddy) - (dtdy * (Fy[m] - e.Fy[m]) + dtdx * (g2y[m] - g1y[m])) / km;
+      upd[m] = v - (dtdx * g1r[m]) / km;
+    }
+  } else {
+#pragma unroll
+    for (int m = 0; m < ME; m++) {
+      T qaddy = e.qaddy[m] - dtdy * e.am[m];
+      T v = e.acc[m] + dtdx * g2l[m];
+      v = v + ((qaddy - dtdy * (Fy[m] - e.Fy[m])) - dtdx * (g2y[m] - g1y[m]));
+      upd[m] = v - dtdx * g1r[m];
+    }
+  }
+  if (out_col) {
+    T* po = cell_ptr2(a.qout, a.gout, c, row);
+    if (KAHAN) {
+      const T* pci = cell_ptr2(a.comp_in, a.gout, c, row);
+      T* pco = cell_ptr2(a.comp_out, a.gout, c, row);
+#pragma unroll
+      for (int m = 0; m < ME; m++) {
+        T y = upd[m] - pci[(long long)m * a.gout.fs];
+        T tq = e.qold[m] + y;
+        pco[(long long)m * a.gout.fs] = (tq - e.qold[m]) - y;
+        po[(long long)m * a.gout.fs] = tq;
+      }
+    } else {
+#pragma unroll
+      for (int m = 0; m < ME; m++) po[(long long)m * a.gout.fs] = upd[m];
+    }
+  }
+}
+
+// The solves of rows `first` .. jend of a strip: rows first .. jend - 1 are stored,
+// row jend is left in `end`, and `give` (if not null) gets what row `own` adds to
+// the row below it, per lane.  The Courant numbers' maxima are added to smx, smy;
+// returns as march_both wants it.
 template <class RS, typename T, bool KAHAN, bool AUX, bool CAPA, bool WIDE>
-__device__ __forceinline__ int unsplit_march(const UnsplitArgs<T>& a, int wid, int first, T& smx,
-                                             T& smy) {
+__device__ __forceinline__ int unsplit_march(const UnsplitArgs<T>& a, int strip, int first,
+                                             int jend, int own, T* give, RowEnd<RS, T>& end,
+                                             T& smx, T& smy) {
   constexpr int ME = RS::meqn, MW = RS::mwaves, NA = UNSPLIT_MAX_AUX;
   static_assert(AUX || (RS::maux == 0 && !CAPA), "aux solvers and capacity need the aux window");
   using Roe = typename RS::Roe;
   const int lane = threadIdx.x & 63;
-  const int strip = wid % a.nstrips, rb = wid / a.nstrips;
   const int mx = a.gout.mx, my = a.gout.my;
   const int c = 1 + strip * 60 - 2 + lane;
   const int j0 = first;
-  const int jend = min(1 + (rb + 1) * a.H, my + 1);
   const bool out_col = lane >= 2 && lane < 62 && c >= 1 && c <= mx;
   const bool cflx_col = lane >= 1 && c >= 1 && c <= mx + 1;   // lane 0 has no left state
   const bool cfly_col = c >= 0 && c <= mx + 1;
-  const T dtdx = a.dtdx, dtdy = a.dtdy, hy = T(0.5) * a.dtdy;
+  const T dtdx = a.dtdx, dtdy = a.dtdy;
 
   T Qm[ME], Q0[ME], Q1[ME];
   T Am[NA], A0[NA], A1[NA];   // aux rows t-1, t, t+1 (AUX)
@@ -293,12 +373,16 @@ __device__ __forceinline__ int unsplit_march(const UnsplitArgs<T>& a, int wid, i
     load_aux<AUX>(a, c, t + 1, A1);
     // ---- x-slice t
     xpass<RS, AUX, CAPA, WIDE>(a, Q0, Am, A0, A1, cflx_col && t <= my + 1, smx, xr);
+    take_g1<CAPA>(a, CAPA ? capa_of(a, Am) : T(1), xr.g1, acc_prev);
+    if (give && t == own) {
+#pragma unroll
+      for (int m = 0; m < ME; m++) give[(0 * ME + m) * 64] = xr.g1[m];
+    }
     T acc_next[ME];
     if constexpr (CAPA) {
-      const T km = capa_of(a, Am), k0 = capa_of(a, A0), k1 = capa_of(a, A1);
+      const T k0 = capa_of(a, A0), k1 = capa_of(a, A1);
 #pragma unroll
       for (int m = 0; m < ME; m++) {
-        acc_prev[m] = acc_prev[m] - (dtdy * xr.g1[m]) / km;
         acc_cur[m] = (acc_cur[m] + xr.qadd[m]) -
                      (dtdx * (xr.Fr[m] - xr.Fl[m]) + dtdy * (xr.g2[m] - xr.g1[m])) / k0;
         acc_next[m] = (KAHAN ? T(0) : Q1[m]) + (dtdy * xr.g2[m]) / k1;
@@ -306,7 +390,6 @@ __device__ __forceinline__ int unsplit_march(const UnsplitArgs<T>& a, int wid, i
     } else {
 #pragma unroll
       for (int m = 0; m < ME; m++) {
-        acc_prev[m] = acc_prev[m] - dtdy * xr.g1[m];
         acc_cur[m] = ((acc_cur[m] + xr.qadd[m]) - dtdx * (xr.Fr[m] - xr.Fl[m])) - dtdy * (xr.g2[m] - xr.g1[m]);
         acc_next[m] = (KAHAN ? T(0) : Q1[m]) + dtdy * xr.g2[m];
       }
@@ -352,55 +435,31 @@ __device__ __forceinline__ int unsplit_march(const UnsplitArgs<T>& a, int wid, i
       rpt_call<RS, 2, WIDE>(a.rp, roet, AmL, Am, AmR, amm, bmA, bpA);
       rpt_call<RS, 2, WIDE>(a.rp, roet, A0L, A0, A0R, apm, bmP, bpP);
     }
-    const T hyA = CAPA ? T(0.5) * dyA : hy, hyP = CAPA ? T(0.5) * dyP : hy;
-    if (t > j0) {
-      // row t-1 is complete: interface t-1 (apdq side, carried) and t (amdq side)
-      T g1y[ME], g2y[ME], g2l[ME], g1r[ME];
+    if (t > j0) {   // row t-1 is complete: interfaces t-1 (apdq side, carried), t (amdq side)
+      RowEnd<RS, T> e;
 #pragma unroll
       for (int m = 0; m < ME; m++) {
-        g1y[m] = (T(0) - hyA * bmA[m]) - hbm_p[m];
-        g2y[m] = (T(0) - hyA * bpA[m]) - hbp_p[m];
+        e.acc[m] = acc_prev[m];
+        e.qold[m] = qold_prev[m];
+        e.qaddy[m] = qaddy_p[m];
+        e.hbm[m] = hbm_p[m];
+        e.hbp[m] = hbp_p[m];
+        e.Fy[m] = Fy_p[m];
+        e.am[m] = amt[m];
       }
-      from_left(g2y, g2l);
-      from_right(g1y, g1r);
-      T upd[ME];
-      if constexpr (CAPA) {
-        const T km = capa_of(a, Am);
+      e.capa = CAPA ? capa_of(a, Am) : T(1);
+      finish_row<RS, KAHAN, CAPA>(a, c, t - 1, out_col, e, Fy, bmA, bpA);
+    }
+    if (give && t == own) {
 #pragma unroll
-        for (int m = 0; m < ME; m++) {
-          T qaddy = qaddy_p[m] - dyA * amt[m];
-          T v = acc_prev[m] + (dtdx * g2l[m]) / km;
-          v = (v + qaddy) - (dtdy * (Fy[m] - Fy_p[m]) + dtdx * (g2y[m] - g1y[m])) / km;
-          upd[m] = v - (dtdx * g1r[m]) / km;
-        }
-      } else {
-#pragma unroll
-        for (int m = 0; m < ME; m++) {
-          T qaddy = qaddy_p[m] - dtdy * amt[m];
-          T v = acc_prev[m] + dtdx * g2l[m];
-          v = v + ((qaddy - dtdy * (Fy[m] - Fy_p[m])) - dtdx * (g2y[m] - g1y[m]));
-          upd[m] = v - dtdx * g1r[m];
-        }
-      }
-      if (out_col) {
-        T* po = cell_ptr2(a.qout, a.gout, c, t - 1);
-        if (KAHAN) {
-          const T* pci = cell_ptr2(a.comp_in, a.gout, c, t - 1);
-          T* pco = cell_ptr2(a.comp_out, a.gout, c, t - 1);
-#pragma unroll
-          for (int m = 0; m < ME; m++) {
-            T y = upd[m] - pci[(long long)m * a.gout.fs];
-            T tq = qold_prev[m] + y;
-            pco[(long long)m * a.gout.fs] = (tq - qold_prev[m]) - y;
-            po[(long long)m * a.gout.fs] = tq;
-          }
-        } else {
-#pragma unroll
-          for (int m = 0; m < ME; m++) po[(long long)m * a.gout.fs] = upd[m];
-        }
+      for (int m = 0; m < ME; m++) {
+        give[(1 * ME + m) * 64] = Fy[m];
+        give[(2 * ME + m) * 64] = bmA[m];
+        give[(3 * ME + m) * 64] = bpA[m];
       }
     }
     // ---- carry: row t partials from interface t (apdq side); shift windows
+    const T hyP = T(0.5) * dyP;
 #pragma unroll
     for (int m = 0; m < ME; m++) {
       qaddy_p[m] = T(0) - dyP * apt[m];
@@ -430,31 +489,75 @@ __device__ __forceinline__ int unsplit_march(const UnsplitArgs<T>& a, int wid, i
       return max(j0, t - 1);
     }
   }
+#pragma unroll
+  for (int m = 0; m < ME; m++) {
+    end.acc[m] = acc_prev[m];
+    end.qold[m] = qold_prev[m];
+    end.qaddy[m] = qaddy_p[m];
+    end.hbm[m] = hbm_p[m];
+    end.hbp[m] = hbp_p[m];
+    end.Fy[m] = Fy_p[m];
+    end.am[m] = amt[m];
+  }
+  end.capa = CAPA ? capa_of(a, Am) : T(1);
   return kMarched;
 }
 
-// `wid`: this wavefront's index among the a.nstrips * a.nrb of the launch.
-// Returns this lane's Courant number (0 past the last strip); the kernel adds it
-// to *a.cfl_bits (one atomic per workgroup where every wavefront of the
-// workgroup reaches that point, else one per wavefront).
+// This lane's Courant number from its maxima of a march.
+template <bool CAPA, typename T>
+__device__ __forceinline__ double courant(const UnsplitArgs<T>& a, T smx, T smy) {
+  // with CAPA smx, smy hold Courant numbers
+  const double cx = CAPA ? (double)smx : (double)a.dtdx * (double)smx;
+  const double cy = CAPA ? (double)smy : (double)a.dtdy * (double)smy;
+  return cy > cx ? cy : cx;
+}
+
+// A workgroup of up to four wavefronts that march one above the other: block `blk`
+// of the a.nstrips * a.nrb takes an even share of a strip's rows.  The last row
+// of a wavefront lacks what the next row's solves add to it, which is the next
+// wavefront's first row: it comes from there through local memory instead of being
+// solved twice.  Only the last wavefront solves the row past the block, and owns a
+// row less for it.  Bound by instruction issue, so a row less to solve per wavefront
+// counts, as does the even share: against wavefronts that each solved their next
+// row, with the last round of blocks part empty, 1024^2 Euler FP32 + Kahan (6 rows a
+// wavefront) takes 52 us after 57, FP64 (18 rows) 109 after 115, 256^2 FP64 acoustics
+// 10.2 after 13, an ensemble step of 128 members 306 after 342.  Returns this lane's
+// Courant number.
 template <class RS, typename T, bool KAHAN, bool AUX = false, bool CAPA = false>
-__device__ __forceinline__ double unsplit_body(const UnsplitArgs<T>& a, int wid) {
-  if (wid >= a.nstrips * a.nrb) return 0.0;   // uniform per wavefront
+__device__ __forceinline__ double unsplit_block(const UnsplitArgs<T>& a, int blk) {
+  constexpr int ME = RS::meqn;
+  __shared__ T handed[3][4 * ME * 64];
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+  const int strip = blk % a.nstrips, rb = blk / a.nstrips;
+  const int r0 = (int)((long long)rb * a.gout.my / a.nrb);
+  const int solves = (int)((long long)(rb + 1) * a.gout.my / a.nrb) - r0 + 1;
+  const int active = min((int)(blockDim.x >> 6), solves);
+  const int own = 1 + r0 + w * solves / active, jend = r0 + (w + 1) * solves / active;
   T smx = T(0), smy = T(0);
-  march_both<RS, T>(a.rp.wide, 1 + wid / a.nstrips * a.H,
-                    [&](auto kind, int first) __attribute__((always_inline)) {
-    return unsplit_march<RS, T, KAHAN, AUX, CAPA, decltype(kind)::value>(a, wid, first, smx, smy);
-  });
-  double cfl, cy;
-  if constexpr (CAPA) {   // smx, smy hold Courant numbers
-    cfl = (double)smx;
-    cy = (double)smy;
-  } else {
-    cfl = (double)a.dtdx * (double)smx;
-    cy = (double)a.dtdy * (double)smy;
+  RowEnd<RS, T> end;
+  if (w < active) {
+    T* give = w > 0 ? handed[w - 1] + lane : nullptr;
+    march_both<RS, T>(a.rp.wide, own, [&](auto kind, int first) __attribute__((always_inline)) {
+      return unsplit_march<RS, T, KAHAN, AUX, CAPA, decltype(kind)::value>(
+          a, strip, first, jend, own, give, end, smx, smy);
+    });
   }
-  if (cy > cfl) cfl = cy;
-  return cfl;
+  __syncthreads();
+  if (w < active - 1) {
+    T g1[ME], Fy[ME], bm[ME], bp[ME];
+    const T* got = handed[w] + lane;
+#pragma unroll
+    for (int m = 0; m < ME; m++) {
+      g1[m] = got[(0 * ME + m) * 64];
+      Fy[m] = got[(1 * ME + m) * 64];
+      bm[m] = got[(2 * ME + m) * 64];
+      bp[m] = got[(3 * ME + m) * 64];
+    }
+    const int c = 1 + strip * 60 - 2 + lane;
+    take_g1<CAPA>(a, end.capa, g1, end.acc);
+    finish_row<RS, KAHAN, CAPA>(a, c, jend, lane >= 2 && lane < 62 && c <= a.gout.mx, end, Fy, bm, bp);
+  }
+  return courant<CAPA>(a, smx, smy);
 }
 
 }  // namespace claw

@@ -69,13 +69,6 @@ __device__ __forceinline__ long long slice_no(int a, int b, int na, int nb) {
   return DIR == 2 ? (long long)a * (nb + 2) + b : (long long)b * (na + 2) + a;
 }
 
-// Each XCD takes a contiguous range of the blocks (the dispatcher deals them out
-// in turn over 8 XCDs), so that neighbouring slices meet in one L2.
-__device__ __forceinline__ long long xcd_block() {
-  const unsigned n = gridDim.x, b = blockIdx.x, per = n / 8, rest = n % 8, x = b % 8, i = b / 8;
-  return (long long)x * per + min(x, rest) + i;
-}
-
 // component slots: 0..ME-1 qadd, ME..2ME-1 fadd, then gadd / hadd as
 // 2ME + m + ME * (side - 1 + 2 * (off + 1)), H after the 6 ME of G.
 template <int ME>
