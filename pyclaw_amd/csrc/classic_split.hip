@@ -60,6 +60,7 @@ struct SweepArgs {
   int ng, order;
   int mthlim[kMaxWaves];
   T dtdx;               // dt / delta of the sweep direction
+  T dtdy;               // k_xysweep: of its y-sweep
   // k_xsweep
   int nstrips;
   int xrows;            // rows per wavefront
@@ -416,6 +417,191 @@ __global__ void __launch_bounds__(256)
   block_atomic_max(run && live ? (double)a.dtdx * (double)smax : 0.0, a.cfl_bits);
 }
 
+// ---------------------------------------------------------------- x- and y-sweep in one
+// The 3D FP32 + Kahan x- and y-sweeps, out of place: a wavefront marches a run of H
+// rows of one plane along y over a 60-column strip; each row is x-swept across the
+// lanes as it enters the window (k_xsweep's row) and its y-interfaces are solved lane
+// by lane (k_march's), so the state and its compensation pass through memory once for
+// both sweeps.  Written for the z-sweep: columns 0..mx+1 and rows 0..my+1 of all
+// planes, swept where the two kernels' order sweeps them, the rest copied.  FP32 only:
+// the two are bound by memory there (384^3: 1.48 + 1.38 ms, together 1.93, and the
+// step 4.06 -> 3.04 ms), while in FP64 both are bound by instruction issue and the
+// registers of the two together leave one wavefront a SIMD.  168 registers, 3
+// wavefronts a SIMD, 7 dwords spilled.
+template <class RS, typename T>
+__global__ void __launch_bounds__(256)
+    __attribute__((amdgpu_waves_per_eu(3))) k_xysweep(const SweepArgs<T> a) {
+  static_assert(sizeof(T) == 4 && RS::maux == 0, "FP32, no aux");
+  constexpr int ME = RS::meqn, MW = RS::mwaves;
+  using Roe = typename RS::Roe;
+  const int lane = threadIdx.x & 63;
+  const int wid = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  const int mx = a.gin.mx, my = a.gin.my, mz = a.gin.mz, ng = a.ng;
+  const int strip = wid % a.nstrips, rest = wid / a.nstrips;
+  const int k = rest % a.npencil - 1, rb = rest / a.npencil;   // planes -1 .. mz+2
+  const bool run = rb < a.nrb;                                 // uniform per wavefront
+  const bool plane = k >= 0 && k <= mz + 1;                    // swept at all
+  const int j0 = 1 + rb * a.H, jend = min(j0 + a.H, my + 1);
+  const int c = 1 + strip * 60 - 2 + lane;
+  const bool own = lane >= 2 && lane < 62 && c >= 1 && c <= mx;
+  const bool mine = own || c == 0 || (c == mx + 1 && strip == a.nstrips - 1);
+  const bool xcfl = lane >= 1 && c >= 1 && c <= mx + 1;
+  const Column col = make_column(a.gin, a.bc, ng, c);
+  T smx = T(0), smy = T(0);
+
+  // row r as it is, and its compensation (0 where the x-sweep has none)
+  auto load = [&](int r, T (&Q)[ME], T (&C)[ME]) __attribute__((always_inline)) {
+    load_row3<ME>(a.qin, a.gin, a.bc, ng, col, r, k, Q);
+    const bool has = own && r >= 1 && r <= my && k >= 1 && k <= mz;
+    const T* pc = cell_ptr3(a.comp_in, a.gin, c, r, k);
+#pragma unroll
+    for (int m = 0; m < ME; m++) C[m] = has ? pc[(long long)m * a.gin.fs] : T(0);
+  };
+  auto store = [&](int r, const T (&Q)[ME]) __attribute__((always_inline)) {
+    if (!mine) return;
+    T* po = cell_ptr3(a.qout, a.gout, c, r, k);
+#pragma unroll
+    for (int m = 0; m < ME; m++) po[(long long)m * a.gout.fs] = Q[m];
+  };
+  // row r after its x-sweep
+  auto sweep = [&](int r, T (&Q)[ME], T (&C)[ME]) __attribute__((always_inline)) {
+    if (r < 0 || r > my + 1) return;   // uniform
+    T QL[ME], W[MW][ME], s[MW], am[ME], ap[ME];
+    Roe roe;
+    from_left(Q, QL);
+    rpn_call<RS, 1, false>(a.rp, QL, Q, QL, Q, W, s, am, ap, roe);
+    if (xcfl) {
+#pragma unroll
+      for (int w = 0; w < MW; w++) smx = cfl_term(smx, T(fabs(s[w])));
+    }
+    T F[ME];
+#pragma unroll
+    for (int m = 0; m < ME; m++) F[m] = T(0);
+    if (a.order != 1) {
+      T Wn[MW][ME];
+#pragma unroll
+      for (int w = 0; w < MW; w++) from_right(W[w], Wn[w]);
+      T dotr[MW], dotl[MW];
+      wave_dots<ME, MW>(W, Wn, dotr);
+      from_left(dotr, dotl);
+      limit_waves<ME, MW>(W, s, dotl, dotr, a.mthlim);
+      corr_flux<ME, MW, true>(W, s, a.dtdx, F, a.rp.fwave);
+    }
+    T amn[ME], Fr[ME];
+    from_right(am, amn);
+    from_right(F, Fr);
+    const bool kahan = r >= 1 && r <= my && k >= 1 && k <= mz;   // uniform
+#pragma unroll
+    for (int m = 0; m < ME; m++) {
+      T qadd = (T(0) - a.dtdx * ap[m]) - a.dtdx * amn[m];
+      T upd = qadd - a.dtdx * (Fr[m] - F[m]);
+      T y = upd - C[m];   // C = 0 outside the grid
+      T tq = Q[m] + y;
+      C[m] = own && kahan ? (tq - Q[m]) - y : T(0);
+      Q[m] = own ? tq : Q[m];
+    }
+  };
+
+  if (run && !plane) {   // planes the x-sweep copies and the y-sweep leaves
+    T Q[ME];
+    for (int r = j0 == 1 ? 0 : j0; r < (jend == my + 1 ? my + 2 : jend); r++) {
+      load_row3<ME>(a.qin, a.gin, a.bc, ng, col, r, k, Q);
+      store(r, Q);
+    }
+  } else if (run) {
+    const T dtdy = a.dtdy;
+    T Qm[ME], Q0[ME], Q1[ME], Qn[ME], C0[ME], C1[ME], Cn[ME], Cp[ME];
+    load(j0 - 2, Qm, Cp);
+    load(j0 - 1, Q0, Cp);
+    load(j0, Q1, C1);
+    load(j0 + 1, Qn, Cn);
+    sweep(j0 - 2, Qm, Cp);
+    sweep(j0 - 1, Q0, Cp);
+    sweep(j0, Q1, C1);
+    if (j0 == 1) store(0, Q0);
+    T Wt[MW][ME], st[MW], amt[ME], apt[ME], dotl[MW];
+    Roe roet;
+    {
+      T Wp[MW][ME], sp[MW], amp[ME], app[ME];
+      Roe roep;
+      rpn_call<RS, 2, false>(a.rp, Qm, Q0, Qm, Q0, Wp, sp, amp, app, roep);
+      if (j0 - 1 >= 1) {
+#pragma unroll
+        for (int w = 0; w < MW; w++) smy = cfl_term(smy, fabs(sp[w]));
+      }
+      rpn_call<RS, 2, false>(a.rp, Q0, Q1, Q0, Q1, Wt, st, amt, apt, roet);
+#pragma unroll
+      for (int w = 0; w < MW; w++) smy = cfl_term(smy, fabs(st[w]));
+      wave_dots<ME, MW>(Wp, Wt, dotl);
+    }
+    T qold_prev[ME], qadd_p[ME], F_p[ME];
+#pragma unroll
+    for (int m = 0; m < ME; m++) {
+      Q0[m] = Q1[m];
+      C0[m] = C1[m];
+      qold_prev[m] = qadd_p[m] = F_p[m] = Cp[m] = T(0);
+    }
+    for (int t = j0; t <= jend; t++) {
+#pragma unroll
+      for (int m = 0; m < ME; m++) { Q1[m] = Qn[m]; C1[m] = Cn[m]; }
+      if (t < jend) load(t + 2, Qn, Cn);   // at most row my + 2
+      sweep(t + 1, Q1, C1);
+      if (t == my && jend == my + 1) store(my + 1, Q1);
+      T Wn[MW][ME], sn[MW], amn[ME], apn[ME], dotn[MW];
+      Roe roen;
+      rpn_call<RS, 2, false>(a.rp, Q0, Q1, Q0, Q1, Wn, sn, amn, apn, roen);
+      if (t + 1 <= my + 1) {
+#pragma unroll
+        for (int w = 0; w < MW; w++) smy = cfl_term(smy, fabs(sn[w]));
+      }
+      T F[ME];
+#pragma unroll
+      for (int m = 0; m < ME; m++) F[m] = T(0);
+#pragma unroll
+      for (int w = 0; w < MW; w++) dotn[w] = T(0);
+      if (a.order != 1) {
+        wave_dots<ME, MW>(Wt, Wn, dotn);
+        limit_waves<ME, MW>(Wt, st, dotl, dotn, a.mthlim);
+        corr_flux<ME, MW, true>(Wt, st, dtdy, F, a.rp.fwave);
+      }
+      if (t > j0 && mine) {
+        T* po = cell_ptr3(a.qout, a.gout, c, t - 1, k);
+        T* pco = cell_ptr3(a.comp_out, a.gout, c, t - 1, k);
+#pragma unroll
+        for (int m = 0; m < ME; m++) {
+          T qadd = qadd_p[m] - dtdy * amt[m];
+          T d = qadd - dtdy * (F[m] - F_p[m]);
+          T y = d - Cp[m];
+          T tq = qold_prev[m] + y;
+          pco[(long long)m * a.gout.fs] = (tq - qold_prev[m]) - y;
+          po[(long long)m * a.gout.fs] = tq;
+        }
+      }
+#pragma unroll
+      for (int m = 0; m < ME; m++) {
+        qadd_p[m] = T(0) - dtdy * apt[m];
+        F_p[m] = F[m];
+        amt[m] = amn[m];
+        apt[m] = apn[m];
+        qold_prev[m] = Q0[m];
+        Q0[m] = Q1[m];
+        Cp[m] = C0[m];
+        C0[m] = C1[m];
+      }
+#pragma unroll
+      for (int w = 0; w < MW; w++) {
+        st[w] = sn[w];
+        dotl[w] = dotn[w];
+#pragma unroll
+        for (int m = 0; m < ME; m++) Wt[w][m] = Wn[w][m];
+      }
+      roet = roen;
+    }
+  }
+  const double cx = (double)a.dtdx * (double)smx, cy = mine ? (double)a.dtdy * (double)smy : 0.0;
+  block_atomic_max(cx > cy ? cx : cy, a.cfl_bits);
+}
+
 // ---------------------------------------------------------------- launchers
 namespace {
 // Rows per wavefront of an out-of-place y/z sweep, or CLAWHIP_SPLIT_ROWS (tuning
@@ -458,6 +644,7 @@ SweepArgs<T> base_args(const clawhip_rp& rp, const Geom& gin, const Geom& gout, 
   a.ng = ng; a.order = method[1];
   for (int w = 0; w < kMaxWaves; w++) a.mthlim[w] = w < mwaves ? mthlim[w] : 0;
   a.dtdx = T(dtdx);
+  a.dtdy = T(0);
   a.qin = (const T*)qin; a.qout = (T*)qout;
   a.comp_in = (const T*)cin; a.comp_out = (T*)cout;
   a.cfl_bits = cfl;
@@ -528,6 +715,19 @@ int launch_march(SweepArgs<T> a, hipStream_t stream) {
   return e == hipSuccess ? 0 : (int)e;
 }
 
+template <class RS, typename T>
+int launch_xy(SweepArgs<T> a, hipStream_t stream) {
+  a.nstrips = (a.gin.mx + 59) / 60;
+  a.npencil = a.gin.mz + 4;
+  const long long columns = (long long)a.nstrips * a.npencil;
+  a.H = march_rows_split(k_xysweep<RS, T>, 0, columns, a.gin.my);
+  a.nrb = (a.gin.my + a.H - 1) / a.H;
+  hipLaunchKernelGGL((k_xysweep<RS, T>), dim3((unsigned)((columns * a.nrb + 3) / 4)), dim3(256), 0,
+                     stream, a);
+  hipError_t e = hipGetLastError();
+  return e == hipSuccess ? 0 : (int)e;
+}
+
 // 2D: x-sweep into the padded intermediate, y-sweep into the compact output.
 template <class RS, typename T, bool KAHAN>
 int run_split2(const clawhip_rp& rp, const void* q_in, const Geom& gin, void* q_out,
@@ -577,14 +777,21 @@ int run_split3(const clawhip_rp& rp, const void* q_in, const Geom& gin, void* q_
   gw.fs = gw.ss * (long long)(gout.mz + 2 * ng);
   auto ax = base_args<T>(rp, gin, gw, lo, hi, refl, 3, ng, method, mthlim, RS::mwaves, dt / dx,
                          q_in, work, cin, cwork, cfl);
-  int rc = launch_x<RS, T, KAHAN, 3, true>(ax, stream);
-  if (rc) return rc;
-  auto ay = base_args<T>(rp, gw, gw, lo, hi, refl, 3, ng, method, mthlim, RS::mwaves, dt / dy,
-                         work, work, cwork, cwork, cfl);
-  ay.i_lo = 0; ay.i_hi = gout.mx + 1; ay.p_lo = 0; ay.p_hi = gout.mz + 1;
-  ay.w_ilo = 0; ay.w_ihi = gout.mx + 1; ay.w_plo = 0; ay.w_phi = gout.mz + 1;
-  rc = launch_march<RS, T, KAHAN, 2, true>(ay, stream);
-  if (rc) return rc;
+  int rc;
+  if constexpr (KAHAN) {
+    ax.dtdy = T(dt / dy);
+    rc = launch_xy<RS, T>(ax, stream);
+    if (rc) return rc;
+  } else {
+    rc = launch_x<RS, T, KAHAN, 3, true>(ax, stream);
+    if (rc) return rc;
+    auto ay = base_args<T>(rp, gw, gw, lo, hi, refl, 3, ng, method, mthlim, RS::mwaves, dt / dy,
+                           work, work, cwork, cwork, cfl);
+    ay.i_lo = 0; ay.i_hi = gout.mx + 1; ay.p_lo = 0; ay.p_hi = gout.mz + 1;
+    ay.w_ilo = 0; ay.w_ihi = gout.mx + 1; ay.w_plo = 0; ay.w_phi = gout.mz + 1;
+    rc = launch_march<RS, T, KAHAN, 2, true>(ay, stream);
+    if (rc) return rc;
+  }
   auto az = base_args<T>(rp, gw, gout, lo, hi, refl, 3, ng, method, mthlim, RS::mwaves, dt / dz,
                          work, q_out, cwork, cout, cfl);
   az.i_lo = 0; az.i_hi = gout.mx + 1; az.p_lo = 0; az.p_hi = gout.my + 1;

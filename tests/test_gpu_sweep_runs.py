@@ -69,3 +69,41 @@ def test_split2_runs_bit_exact(mx, my):
         out = q_from_device(qo)
         assert np.array_equal(O.interior(out, ng) if whole else out, O.interior(ref, ng))
         assert float(cfl.item()) == c
+
+
+@pytest.mark.parametrize("mx,my,mz", [(60, 2, 3), (61, 3, 2), (59, 4, 5), (121, 9, 2), (2, 37, 4),
+                                      (7, 130, 3), (64, 64, 5)])
+def test_split3_fp32_one_pass_xy(mx, my, mz):
+    """The FP32 + Kahan step's x- and y-sweep in one pass, against the FP64 oracle's three
+    sweeps from the same FP32 state, with a compensation of a few units in the last place.
+    A cell's change is three sums of some 50 products of terms no larger than 4 max|q|
+    times the Courant number c, each rounded to 2^-24: 3 * 50 * 4 * c * 2^-24 max|q|."""
+    from pyclaw_amd import kernels as K
+    from pyclaw_amd.device import q_from_device, q_to_device
+    ng, bcl, bcu = 2, [1, 2, 3], [1, 2, 3]
+    print("split3 xy", (mx, my, mz), flush=True)
+    rng = np.random.default_rng(mx + my)
+    q = seeded_state(rng, O.EULER3, (mx, my, mz)).astype(np.float32)
+    comp = (1e-7 * rng.standard_normal(q.shape)).astype(np.float32)
+    meth = O.method_array(dimensional_split=True)
+    dx, dy, dz = 1.0 / mx, 0.9 / my, 1.1 / mz
+    dt = 0.05 * min(dx, dy, dz)
+    start = np.asfortranarray(q.astype(np.float64) - comp.astype(np.float64))
+    qbc = O.with_ghosts(start, ng)
+    O.bc3(qbc, ng, bcl, bcu)
+    rp = O.make_rp(O.EULER3)
+    cs = []
+    for k in (1, 2, 3):
+        src = qbc.copy(order="F") if k == 1 else qbc
+        cs.append(O.step3ds(rp, src, qbc, ng, dx, dy, dz, dt, meth, [4] * 3, k))
+    qi = q_to_device(np.asfortranarray(q.astype(np.float64))).float()
+    ci = q_to_device(np.asfortranarray(comp.astype(np.float64))).float()
+    qo, co = torch.empty_like(qi), torch.empty_like(ci)
+    cfl = torch.zeros(1, dtype=torch.float64, device="cuda")
+    K.step3_split(K.make_rp(5, {"gamma": 1.4}), qi, qo, cfl, bcl, bcu, [1, 2, 3], meth, [4] * 3,
+                  dx, dy, dz, dt, comp_in=ci, comp_out=co)
+    torch.cuda.synchronize()
+    out = q_from_device(qo.double()) - q_from_device(co.double())
+    bound = 3 * 50 * 4 * max(cs) * 2.0 ** -24 * np.abs(start).max()
+    assert np.abs(out - O.interior(qbc, ng)).max() <= bound
+    assert abs(float(cfl.item()) - max(cs)) <= 50 * 2.0 ** -24 * max(cs)
