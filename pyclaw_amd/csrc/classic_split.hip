@@ -11,6 +11,7 @@
 //   for the limiter.  Used for the 2D y-sweep (columns 1-ng..mx+ng,
 //   step2ds.f90:180), and the 3D y- and z-sweeps (pencils 0..m+1,
 //   step3ds.f90:215-216, 298-299).
+// k_xysweep: the 3D FP32 + Kahan x- and y-sweeps in one pass.
 // The 2D split uses flux2's 0.5*cqxx; the 3D split flux3's cqxx with the 0.5
 // inside the sum (flux3.f90:244) -- the HALF_IN_SUM template flag.
 #include "variant.hpp"  // first: selects the arithmetic variant
@@ -228,8 +229,9 @@ __device__ __forceinline__ long long cell_off(const Geom& g, int i, int s, int p
 // ahead of the workgroup's barrier, so nobody reads a row already swept.  One
 // wavefront a pencil left 768 of them on 1024 SIMDs at 210x170x190.  With the
 // runs, the row loaded ahead and one Courant-number atomic per workgroup the
-// split step takes 1.04 instead of 1.33 ms there (FP64) and 4.13 instead of
-// 5.24 ms at 384^3 (FP32 + Kahan).
+// split step takes 1.04 instead of 1.33 ms there (FP64; 0.82 with the shared
+// reciprocals) and 4.13 instead of 5.24 ms at 384^3 (FP32 + Kahan; 3.04 with
+// k_xysweep).
 // Wavefronts per SIMD a march is compiled for, where that differs from the
 // compiler's choice: FP64 euler_3D sits 4 registers above the 256 of 2 per SIMD
 // and fits them without spills (210x170x190 step 1.07 -> 0.95 ms).  FP32 + Kahan
@@ -803,7 +805,7 @@ int run_split3(const clawhip_rp& rp, const void* q_in, const Geom& gin, void* q_
 // (the reference's qbc, filled by the caller: BC_GIVEN on every side).  Sweep 1
 // reads q_in and writes every cell of q_out (interior columns updated on all
 // rows, ghost columns copied), as step2ds/step3ds with ids/idir = 1 do; sweeps
-// 2 and 3 update q_out in place (q_in == q_out), marching whole pencils.
+// 2 and 3 update q_out in place (q_in == q_out).
 template <class RS>
 int run_sweep(const clawhip_rp& rp, int ndim, int dir, const void* q_in, const Geom& gin,
               void* q_out, const Geom& gout, int ng, const int* method, const int* mthlim,
