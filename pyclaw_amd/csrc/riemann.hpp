@@ -75,25 +75,33 @@ struct RPParams {
 
 // a / b: FP32 by the hardware reciprocal, as the build's FP32 division (about 1 ulp),
 // without its scaling of denominators above 2^96 (compare, select and two
-// multiplications more): the same bits up to 2^126, where 1 / b leaves the normal
-// numbers.  2048^2 flagged SharpClaw march 85 -> 80 us, 1024^2 Euler step 64 -> 62,
-// ensemble step 2 %.
+// multiplications more): the same bits up to |b| = 2^126; beyond, 1 / b is flushed.
+// So only for |a| <= 1 (such a quotient is flushed either way) and for denominators
+// that stay below by what they are: roots and their sums (at most 2^66), and depths (one
+// above 2^126 has overflowed g h^2 in the fluxes, and its velocity, at most 4, is lost
+// against sqrt(g h)).  Written a / b everywhere else; limit_waves tests its
+// denominators (wave norms above 2^63).  2048^2 flagged SharpClaw march
+// 85 -> 80 us, 1024^2 Euler step 64 -> 62, ensemble step 2 %.
 template <typename T>
 __device__ __forceinline__ T quo(T a, T b) {
   if constexpr (sizeof(T) == 4) return a * __builtin_amdgcn_rcpf(b);
   else return a / b;
 }
 
-template <typename T, bool WIDE>
+// ANY: an FP32 denominator of any magnitude (see quo)
+template <typename T, bool WIDE, bool ANY = false>
 struct Divided {
   T d;
   __device__ __forceinline__ explicit Divided(T den) : d(den) {}
   __device__ __forceinline__ Divided(T den, T) : d(den) {}
   __device__ __forceinline__ T reciprocal() const { return T(0); }   // not used
-  __device__ __forceinline__ friend T operator/(T a, const Divided& o) { return quo(a, o.d); }
+  __device__ __forceinline__ friend T operator/(T a, const Divided& o) {
+    if constexpr (ANY) return a / o.d;
+    else return quo(a, o.d);
+  }
 };
-template <>
-struct Divided<double, false> {
+template <bool ANY>
+struct Divided<double, false, ANY> {
   double d, r;
   __device__ __forceinline__ explicit Divided(double den) : d(den) {
     r = __builtin_amdgcn_rcp(den);
@@ -179,8 +187,8 @@ struct Acoustics {
     const T zz = p.zz, cc = p.cc;
     T delta1 = qR[0] - qL[0];
     T delta2 = qR[mu] - qL[mu];
-    T a1 = quo(-delta1 + zz * delta2, T(2) * zz);
-    T a2 = quo(delta1 + zz * delta2, T(2) * zz);
+    T a1 = (-delta1 + zz * delta2) / (T(2) * zz);
+    T a2 = (delta1 + zz * delta2) / (T(2) * zz);
     wave[0][0] = -a1 * zz; wave[0][mu] = a1; wave[0][mv] = T(0); s[0] = -cc;
     wave[1][0] = a2 * zz; wave[1][mu] = a2; wave[1][mv] = T(0); s[1] = cc;
 #pragma unroll
@@ -194,8 +202,8 @@ struct Acoustics {
                                              T (&bm)[meqn], T (&bp)[meqn]) {
     constexpr int mu = IXY == 1 ? 1 : 2, mv = IXY == 1 ? 2 : 1;
     const T zz = p.zz, cc = p.cc;
-    T a1 = quo(-asdq[0] + zz * asdq[mv], T(2) * zz);
-    T a2 = quo(asdq[0] + zz * asdq[mv], T(2) * zz);
+    T a1 = (-asdq[0] + zz * asdq[mv]) / (T(2) * zz);
+    T a2 = (asdq[0] + zz * asdq[mv]) / (T(2) * zz);
     bm[0] = cc * a1 * zz; bm[mu] = T(0); bm[mv] = -cc * a1;
     bp[0] = cc * a2 * zz; bp[mu] = T(0); bp[mv] = cc * a2;
   }
@@ -269,7 +277,8 @@ struct EulerT {
 
   template <int IXY, bool WIDE>
   __device__ static __forceinline__ Roe roe_avg(T gamma1, const T* qL, const T* qR,
-                                                const Divided<T, WIDE>& rhol, const Divided<T, WIDE>& rhor) {
+                                                const Divided<T, WIDE, true>& rhol,
+                                                const Divided<T, WIDE, true>& rhor) {
     constexpr int mu = IXY == 1 ? 1 : 2, mv = IXY == 1 ? 2 : 1;
     Roe r;
     const T rootl = root<WIDE>(qL[0]), rootr = root<WIDE>(qR[0]);
@@ -295,7 +304,7 @@ struct EulerT {
     constexpr int mu = IXY == 1 ? 1 : 2, mv = IXY == 1 ? 2 : 1;
     const T gamma = p.gamma, gamma1 = p.gamma1;
     T irl = T(0), irr = T(0), ia2 = T(0);   // shared reciprocals (fast variant)
-    const Divided<T, WIDE> rhol(qL[0]), rhor(qR[0]);
+    const Divided<T, WIDE, true> rhol(qL[0]), rhor(qR[0]);
     if constexpr (kSharedReciprocals) r = roe_avg_shared<IXY, WIDE>(gamma1, qL, qR, irl, irr, ia2);
     else r = roe_avg<IXY, WIDE>(gamma1, qL, qR, rhol, rhor);
     T d0 = qR[0] - qL[0], d1 = qR[mu] - qL[mu], d2 = qR[mv] - qL[mv], d3 = qR[3] - qL[3];
@@ -359,13 +368,13 @@ struct EulerT {
         c1 = root<WIDE>(gamma * p1 * ir1);
         s1 = rhou1 * ir1 - c1;
       } else {
-        const Divided<T, WIDE> drho1(rho1);
+        const Divided<T, WIDE, true> drho1(rho1);
         p1 = gamma1 * (en1 - T(0.5) * (rhou1 * rhou1 + rhov1 * rhov1) / drho1);
         c1 = root<WIDE>(gamma * p1 / drho1);
         s1 = rhou1 / drho1 - c1;
       }
       T sfract;
-      if (s0 < T(0) && s1 > T(0)) sfract = quo(s0 * (s1 - s[0]), s1 - s0);
+      if (s0 < T(0) && s1 > T(0)) sfract = s0 * (s1 - s[0]) / (s1 - s0);
       else if (s[0] < T(0)) sfract = s[0];
       else sfract = T(0);
 #pragma unroll
@@ -398,12 +407,12 @@ struct EulerT {
         c2 = root<WIDE>(gamma * p2 * ir2);
         s2 = rhou2 * ir2 + c2;
       } else {
-        const Divided<T, WIDE> drho2(rho2);
+        const Divided<T, WIDE, true> drho2(rho2);
         p2 = gamma1 * (en2 - T(0.5) * (rhou2 * rhou2 + rhov2 * rhov2) / drho2);
         c2 = root<WIDE>(gamma * p2 / drho2);
         s2 = rhou2 / drho2 + c2;
       }
-      if (s2 < T(0) && s3 > T(0)) sfract = quo(s2 * (s3 - s[3]), s3 - s2);
+      if (s2 < T(0) && s3 > T(0)) sfract = s2 * (s3 - s[3]) / (s3 - s2);
       else if (s[3] < T(0)) sfract = s[3];
       else break;
 #pragma unroll
@@ -515,7 +524,7 @@ struct Shallow {
       T hu1 = qL[mu] + wave[0][mu];
       T s1 = quo(hu1, h1) - root<WIDE>(grav * h1);
       T sfract;
-      if (s0 < T(0) && s1 > T(0)) sfract = quo(s0 * (s1 - s[0]), s1 - s0);
+      if (s0 < T(0) && s1 > T(0)) sfract = s0 * (s1 - s[0]) / (s1 - s0);
       else if (s[0] < T(0)) sfract = s[0];
       else sfract = T(0);
 #pragma unroll
@@ -528,7 +537,7 @@ struct Shallow {
       T h3 = qR[0] - wave[2][0];
       T hu3 = qR[mu] - wave[2][mu];
       T s3 = quo(hu3, h3) + root<WIDE>(grav * h3);
-      if (s3 < T(0) && s03 > T(0)) sfract = quo(s3 * (s03 - s[2]), s03 - s3);
+      if (s3 < T(0) && s03 > T(0)) sfract = s3 * (s03 - s[2]) / (s03 - s3);
       else if (s[2] < T(0)) sfract = s[2];
       else break;
 #pragma unroll
@@ -615,7 +624,7 @@ struct Euler3 {
     constexpr int mw = IXY == 1 ? 3 : (IXY == 2 ? 1 : 2);
     const T gamma = p.gamma, gamma1 = p.gamma1;
     const T rootl = root<WIDE>(qL[0]), rootr = root<WIDE>(qR[0]);
-    const Divided<T, WIDE> rhol(qL[0]), rhor(qR[0]);
+    const Divided<T, WIDE, true> rhol(qL[0]), rhor(qR[0]);
     // the fast variant's shared reciprocals (kSharedReciprocals): 1/rho per side
     // (and 1/sqrt(rho) = sqrt(rho)/rho), the Roe denominator, 1/a^2
     T irl = T(0), irr = T(0), ia2 = T(0);
@@ -711,13 +720,13 @@ struct Euler3 {
         c1 = root<WIDE>(gamma * p1 * ir1);
         s1 = rhou1 * ir1 - c1;
       } else {
-        const Divided<T, WIDE> drho1(rho1);
+        const Divided<T, WIDE, true> drho1(rho1);
         p1 = gamma1 * (en1 - T(0.5) * (rhou1 * rhou1 + rhov1 * rhov1 + rhow1 * rhow1) / drho1);
         c1 = root<WIDE>(gamma * p1 / drho1);
         s1 = rhou1 / drho1 - c1;
       }
       T sfract;
-      if (s0 < T(0) && s1 > T(0)) sfract = quo(s0 * (s1 - s[0]), s1 - s0);
+      if (s0 < T(0) && s1 > T(0)) sfract = s0 * (s1 - s[0]) / (s1 - s0);
       else if (s[0] < T(0)) sfract = s[0];
       else sfract = T(0);
 #pragma unroll
@@ -747,12 +756,12 @@ struct Euler3 {
         c2 = root<WIDE>(gamma * p2 * ir2);
         s2 = rhou2 * ir2 + c2;
       } else {
-        const Divided<T, WIDE> drho2(rho2);
+        const Divided<T, WIDE, true> drho2(rho2);
         p2 = gamma1 * (en2 - T(0.5) * (rhou2 * rhou2 + rhov2 * rhov2 + rhow2 * rhow2) / drho2);
         c2 = root<WIDE>(gamma * p2 / drho2);
         s2 = rhou2 / drho2 + c2;
       }
-      if (s2 < T(0) && s3 > T(0)) sfract = quo(s2 * (s3 - s[2]), s3 - s2);
+      if (s2 < T(0) && s3 > T(0)) sfract = s2 * (s3 - s[2]) / (s3 - s2);
       else if (s[2] < T(0)) sfract = s[2];
       else break;
 #pragma unroll
@@ -844,7 +853,7 @@ struct ShallowHLLE {
     const T cbar = root<WIDE>(T(0.5) * grav * (h_l + h_r));
     const T s1 = dmin(u_l - root<WIDE>(grav * h_l), ubar - cbar);
     const T s2 = dmax(u_r + root<WIDE>(grav * h_r), ubar + cbar);
-    const Divided<T, WIDE> ds(s1 - s2);
+    const Divided<T, WIDE, true> ds(s1 - s2);
     const T hm = (qR[mu] - qL[mu] - s2 * qR[0] + s1 * qL[0]) / ds;
     const T hum = (qR[mu] * u_r - qL[mu] * u_l + T(0.5) * grav * (h_r * h_r - h_l * h_l) -
                    s2 * qR[mu] + s1 * qL[mu]) / ds;

@@ -182,8 +182,8 @@ __device__ __forceinline__ T weno_char_side(T hm2, T hm1, T h0, T hp1, T hp2, in
   T s1, s3;
   if constexpr (sizeof(T) == 4) {
     // the same weights as d_k / (eps + beta_k)^2: no fourth powers to underflow
-    const T r1 = quo(T(1), tt1), r2 = quo(T(6), tt2), r3 = quo(T(3), tt3);
-    const T t0 = quo(T(1), r1 + r2 + r3);
+    const T r1 = quo(T(1), tt1), r2 = T(6) / tt2, r3 = T(3) / tt3;
+    const T t0 = quo(T(1), r1 + r2 + r3);   // the sum is at most 10 / eps^2 = 1e37
     s1 = r1 * t0;
     s3 = r3 * t0;
   } else {   // the reference's products of two squares, bit for bit
@@ -233,7 +233,8 @@ struct Evec<Euler<T>, IXY, T, WIDE> {
                                              T (&evl)[4][4], T (&evr)[4][4]) {
     constexpr int mu = IXY == 1 ? 1 : 2, mv = IXY == 1 ? 2 : 1;
     const T gamma1 = p.gamma1;
-    auto r = Euler<T>::template roe_avg<IXY, WIDE>(gamma1, qL, qR, Divided<T, WIDE>(qL[0]), Divided<T, WIDE>(qR[0]));
+    auto r = Euler<T>::template roe_avg<IXY, WIDE>(
+        gamma1, qL, qR, Divided<T, WIDE, true>(qL[0]), Divided<T, WIDE, true>(qR[0]));
     T u = r.u, v = r.v, c = r.a, H = r.enth;
     T q2 = T(0.5) * r.u2v2;
     evr[0][0] = T(1); evr[mu][0] = u - c; evr[mv][0] = v; evr[3][0] = H - u * c;
