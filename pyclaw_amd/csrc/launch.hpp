@@ -50,7 +50,7 @@ inline RPParams<T> to_params(const clawhip_rp& r) {
   p.wide = 0;
   for (double v : {r.gamma, r.gamma - 1.0, r.grav}) {
     const double m = v < 0 ? -v : v;
-    if (!(m == 0.0 || (m > 0x1p-200 && m < 0x1p200))) p.wide = 1;
+    if (!(m == 0.0 || (m > 0x1p-60 && m < 0x1p60))) p.wide = 1;
   }
   return p;
 }

@@ -53,7 +53,7 @@ struct RPParams {
   T dry_tolerance;       // shallow water with bathymetry
   int efix;
   int fwave;             // the solver returns f-waves (step2's use_fwave)
-  int wide;              // a parameter is beyond 2^+-200: see Divided
+  int wide;              // a parameter is beyond 2^+-60: see Divided
 };
 
 // ---- several quotients over one denominator, square roots
@@ -68,10 +68,18 @@ struct RPParams {
 // spent half their cycles on them (1024^2 Euler step 128 -> 119 us, 2048^2 shallow-
 // water WENO5 stage 465 -> 398, 210x170x190 euler_3D step 0.99 -> 0.82 ms).
 // WIDE = true, and every type but double: the plain division and sqrt.  The
-// reference-equal FP64 kernels take it where a state has a value beyond 2^200 or
-// a nonzero one below 2^-700 (Watch; decaying tails reach denormals): a
+// reference-equal FP64 kernels take it where a state has a value beyond 2^40 or
+// a nonzero one below 2^-320 (Watch; decaying tails reach denormals): a
 // march with several solves a row starts again at that row with the plain division
 // (march_both), the split sweeps go on with it.
+// Why there: numerators hold products of two small values (a velocity times a jump,
+// v d2 in a Roe solve's a3, where the other terms are zero).  A jump of values in
+// [2^-L, 2^U) is 0 or at least 2^-(L+52), an averaged velocity over the sound speed
+// at least 2^-(L+U+53), their product in a sum of such terms at least
+// 2^-(2L+U+157); a parameter (within 2^+-60) takes 30 more.  The classic steps have
+// L = 320: 2^-867.  WENO5 makes edge values as small as eps^2 / M^3 of a zero region
+// beside a jump M < 2^41: L = 362, 2^-951.  Only a product of three small values, where
+// those of two cancel, may lie below: its quotient's last bit can differ.
 
 // a / b: FP32 by the hardware reciprocal, as the build's FP32 division (about 1 ulp),
 // without its scaling of denominators above 2^96 (compare, select and two
@@ -138,7 +146,7 @@ template <class RS, typename T>
 constexpr bool watched() { return RS::shares && sizeof(T) == 8 && CLAW_FAST == 0; }
 
 // The magnitudes of the values a lane has met: tame() while all are zero or in
-// [2^-700, 2^200) (not NaN).  Kept as the smallest and largest of the words that
+// (2^-320, 2^40) (not NaN).  Kept as the smallest and largest of the words that
 // hold a value's exponent and leading digits (doubled, which drops the sign; a
 // zero, less one, is the largest), so that watching costs no branch.
 template <class RS, typename T>
@@ -162,7 +170,7 @@ struct Watch {
     return !watched<RS, T>() || __ballot(!tame()) == 0ull;
   }
   __device__ __forceinline__ bool tame() const {
-    return least >= 2u * 0x14300000u && most < 2u * 0x4c700000u;
+    return least >= 2u * 0x2bf00000u && most < 2u * 0x42700000u;
   }
 };
 

@@ -1,8 +1,9 @@
 """The reference-equal FP64 solves share reciprocals between quotients while a
-wavefront's values lie in [2^-700, 2^200) or are zero, and divide plainly
-otherwise (riemann.hpp Divided).  States on both sides of those bounds -- tails
-that decay through 2^-700 to denormals and zeros, values around 2^200 -- are
-stepped bit for bit as the oracle does, by every march that chooses."""
+wavefront's values lie in (2^-320, 2^40) or are zero, and divide plainly
+otherwise (riemann.hpp Divided).  States whose tails decay through the lower bound
+to denormals and zeros, in half of the columns of every row, are stepped bit for bit
+as the oracle does, by every march that chooses (the choice in mid-march and the upper
+bound: test_gpu_division_guard.py).  Acoustics divides plainly whatever the values."""
 import numpy as np
 import pytest
 import torch
@@ -13,9 +14,10 @@ from tests.test_gpu_sharp import PD, _orp
 
 pytestmark = pytest.mark.gpu
 
-# decimal exponents of the values' magnitudes: around 2^-700 (5e-211), down to the
-# smallest denormal, around 2^200 (1.6e60; the linear solver only)
-RANGES = {"edge": (-213.0, -209.0), "denormal": (-323.5, -190.0), "large": (59.0, 61.5)}
+# decimal exponents of the values' magnitudes: around 2^-320 (4.7e-97), around 2^-700,
+# down to the smallest denormal, around 2^200 (the linear solver only)
+RANGES = {"bound": (-99.0, -94.0), "edge": (-213.0, -209.0), "denormal": (-323.5, -190.0),
+          "large": (59.0, 61.5)}
 
 
 def _tails(kind, shape, span, rng):
@@ -37,7 +39,8 @@ def _tails(kind, shape, span, rng):
 
 
 CASES = [(O.ACOUSTICS, "edge"), (O.ACOUSTICS, "denormal"), (O.ACOUSTICS, "large"),
-         (O.SHALLOW, "edge"), (O.SHALLOW, "denormal"), (O.EULER, "edge"), (O.EULER, "denormal")]
+         (O.SHALLOW, "edge"), (O.SHALLOW, "denormal"), (O.EULER, "edge"), (O.EULER, "denormal"),
+         (O.SHALLOW, "bound"), (O.EULER, "bound")]
 
 
 def _device(q):
@@ -97,7 +100,7 @@ def test_sharp_operator_bit_exact(kind, span):
         assert float(cfl.item()) == c
 
 
-@pytest.mark.parametrize("span", ["edge", "denormal"])
+@pytest.mark.parametrize("span", ["edge", "denormal", "bound"])
 def test_3d_steps_bit_exact(span):
     from pyclaw_amd import kernels as K
     from pyclaw_amd.device import q_from_device
