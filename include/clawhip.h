@@ -71,7 +71,7 @@ enum {
                                    * development/rp_approaches/rpn2_euler_5wave.f,
                                    * rpt2_euler_5wave.f): euler_4wave_2D plus a passive
                                    * tracer q[4]; classic 2D steps, SharpClaw with
-                                   * char_decomp 0 */
+                                   * char_decomp 0 (CLAWHIP_F64: CLAWHIP_E_KIND) */
   CLAWHIP_RP_SHALLOW_FWAVE = 11    /* shallow_bathymetry_fwave_2D (clawpack/riemann): shallow
                                    * water over bathymetry b = aux[0], f-waves (set
                                    * rp.fwave = 1); no transverse solver (split, or unsplit

@@ -1301,7 +1301,10 @@ int launch_sharp_stage(const clawhip_rp& rp, int dtype, int char_decomp, const G
     case CLAWHIP_RP_SHALLOW: return dispatch_stage<Shallow, false>(ARGS);
     case CLAWHIP_RP_SHALLOW_HLLE: return dispatch_stage<ShallowHLLE, false>(ARGS);
     case CLAWHIP_RP_EULER: return dispatch_stage<Euler, false>(ARGS);
+#if CLAW_FAST   // the reference-equal build refuses it: an earlier form of that march did
+                // not finish on the device once, cause not shown, and no later form has run
     case CLAWHIP_RP_EULER5: return dispatch_stage<Euler5, false>(ARGS);
+#endif
     case CLAWHIP_RP_ACOUSTICS: return dispatch_stage<Acoustics, false>(ARGS);
     case CLAWHIP_RP_ADVECTION: return dispatch_stage<Advection, false>(ARGS);
   }
@@ -1333,7 +1336,9 @@ int launch_sharp_ssp33_run(const clawhip_rp& rp, int dtype, int char_decomp, con
     case CLAWHIP_RP_SHALLOW: return RUN(Shallow, false);
     case CLAWHIP_RP_SHALLOW_HLLE: return RUN(ShallowHLLE, false);
     case CLAWHIP_RP_EULER: return RUN(Euler, false);
+#if CLAW_FAST   // as in launch_sharp_stage
     case CLAWHIP_RP_EULER5: return RUN(Euler5, false);
+#endif
     case CLAWHIP_RP_ACOUSTICS: return RUN(Acoustics, false);
     case CLAWHIP_RP_ADVECTION: return RUN(Advection, false);
   }

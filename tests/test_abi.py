@@ -62,6 +62,28 @@ def _small_solution(pyclaw, meqn, num_aux=0):
     return pyclaw.Solution(state, domain)
 
 
+def test_euler5_fp64_sharpclaw_is_switched_off():
+    """The FP64 SharpClaw stage of euler_5wave_2D did not finish on the device once,
+    cause not shown: the solver's setup and the entry points refuse it before any
+    device work; the classic solver takes it."""
+    import pyclaw_amd as pyclaw
+    from pyclaw_amd import kernels as K
+    from pyclaw_amd import riemann
+    s = pyclaw.SharpClawSolver2D(riemann.euler_5wave_2D)
+    with pytest.raises(NotImplementedError, match="euler_5wave_2D"):
+        s.setup(_small_solution(pyclaw, 5))
+    pyclaw.ClawSolver2D(riemann.euler_5wave_2D).setup(_small_solution(pyclaw, 5))
+    lib, rp, g = L.lib(), K.make_rp(10, {}), L.geom2(8, 8)
+    d, e = ctypes.c_void_p(16), ctypes.c_void_p(32)
+    n, bc = None, L.ints([1, 1])
+    assert lib.clawhip_sharp2_stage(
+        ctypes.byref(rp), L.F64, 0, ctypes.byref(g), bc, bc, L.ints([1, 2]), 0, K.OUT_D, 0.1, 0.0,
+        1.0, 1.0, d, n, n, n, n, n, n, e, n, n, n, n, n, n, n, n, n, n, n, 0, d, n) == -2
+    assert lib.clawhip_sharp2_ssp33_run(
+        ctypes.byref(rp), L.F64, 0, ctypes.byref(g), bc, bc, L.ints([1, 2]), 1.0, 1.0, d, e, n, n,
+        d, d, n, n, n, n, n, n, n, 0.0, 0.0, 0, d, 1, n, n) == -2
+
+
 def test_unsupported_options_raise_at_setup():
     """Options the device solvers do not implement fail loudly at setup instead of
     being ignored (no GPU needed: setup raises before any device work)."""
