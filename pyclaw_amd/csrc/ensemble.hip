@@ -5,10 +5,10 @@
 // The members' workgroups are concatenated into one grid (largest members
 // first, so the small ones fill the tail); a workgroup finds its member by
 // binary search over the members' first-block offsets and then runs the
-// same step body as the single-grid kernel (unsplit.hpp).  The last wavefront of
-// a member applies that member's accept/reject and next dt (stepctl.hpp).  A
-// step of the whole ensemble is one launch with no host synchronisation, so
-// runs of steps are captured in a HIP graph.
+// same step body as the single-grid kernel (unsplit.hpp).  A second launch applies
+// every member's accept/reject and next dt (k_ens_ctl, stepctl.hpp).  A step of the
+// whole ensemble is those two launches with no host synchronisation, so runs of
+// steps are captured in a HIP graph.
 #include "variant.hpp"  // first: selects the arithmetic variant
 #include <stdlib.h>
 #include <string.h>
@@ -59,7 +59,12 @@ __device__ __forceinline__ const RPParams<float>& ens_rp<float>(const EnsHeader&
 template <class RS, typename T, bool KAHAN>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(unsplit_waves<RS, T>())))
 k_ens_step(const EnsHeader* __restrict__ hdr, const EnsMember* __restrict__ mem) {
-  const long long blk = blockIdx.x;
+  // The table's blocks are of four wavefronts; workgroups of fewer share a block's
+  // rows, so that a wavefront's rows do not depend on the grouping (64 members of 16 to
+  // 48 cells a side, 1 / 2 / 4 wavefronts: 27.6, 25.5, 24.5 us a step; 40.7, 31.1, 23.8
+  // with a block to each workgroup; 512 of 64 to 512: 1143, 1157, 1154).
+  const int parts = 256 / (int)blockDim.x;
+  const long long blk = blockIdx.x / parts;
   // member k: the last one whose first block is <= blk
   int lo = 0, hi = hdr->n - 1;
   while (lo < hi) {
@@ -80,7 +85,7 @@ k_ens_step(const EnsHeader* __restrict__ hdr, const EnsMember* __restrict__ mem)
   a.bc = hdr->bc;
   a.ng = hdr->ng; a.order = hdr->order; a.trans = hdr->trans;
   for (int w = 0; w < 4; w++) a.mthlim[w] = hdr->mthlim[w];
-  a.nstrips = m.nstrips; a.nrb = m.nrb;
+  a.nstrips = m.nstrips; a.nrb = m.nrb * parts;
   a.qin = (const T*)m.q[cur];
   a.qout = (T*)m.q[1 - cur];
   a.comp_in = (const T*)m.comp[cur];
@@ -88,7 +93,8 @@ k_ens_step(const EnsHeader* __restrict__ hdr, const EnsMember* __restrict__ mem)
   a.dtdx = T(dt / m.dx);
   a.dtdy = T(dt / m.dy);
   a.cfl_bits = &ctl->cfl_bits;
-  block_atomic_max(unsplit_block<RS, T, KAHAN>(a, (int)(blk - m.base)), a.cfl_bits);
+  block_atomic_max(unsplit_block<RS, T, KAHAN>(a, (int)(blockIdx.x - m.base * parts)),
+                   a.cfl_bits);
 }
 
 // Every member's step control after the step launch (step_ctl_apply), one
@@ -137,10 +143,9 @@ int ens_choose_rows(const std::vector<EnsMember>& v) {
 template <class RS, typename T, bool KAHAN>
 void ens_launch(const EnsHeader* h, const EnsMember* m, const long long* waves, int nsteps,
                 hipStream_t s) {
-  // wavefronts per workgroup: 1, 2 or 4 (the autotuner's second parameter); fewer
-  // march more of the block's rows each
+  // wavefronts per workgroup: 1, 2 or 4 (the autotuner's second parameter)
   const long long wpb = (waves[2] == 1 || waves[2] == 2) ? waves[2] : 4;
-  const unsigned blocks = (unsigned)(waves[0] / 4);
+  const unsigned blocks = (unsigned)(waves[0] / wpb);
   const unsigned ctl_blocks = (unsigned)((waves[1] + 255) / 256);
   for (int n = 0; n < nsteps; n++) {
     hipLaunchKernelGGL((k_ens_step<RS, T, KAHAN>), dim3(blocks), dim3((unsigned)(64 * wpb)), 0,

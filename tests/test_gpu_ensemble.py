@@ -54,3 +54,25 @@ def test_ensemble_members_equal_single_runs(precision):
         assert ctls[k].attempts == 21 == host.attempts
         assert ctls[k].accepted == host.accepted and ctls[k].t == host.t, k
         assert np.array_equal(ens.member_q(k), sol.state.q), (k, (mx, my))
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32k"])
+@pytest.mark.parametrize("group,rows", [(1, 0), (2, 0), (1, 2), (2, 3), (4, 2), (1, 16), (2, 16)])
+def test_groups_of_wavefronts(group, rows, precision):
+    """1, 2 and 4 wavefronts per workgroup over members of few rows (shares of no rows
+    among them) and of many: the same members, bit for bit."""
+    from pyclaw_amd.ensemble import Ensemble
+    sizes = [(61, 2), (7, 3), (64, 5), (60, 8), (121, 31), (20, 130)]
+    print("ensemble groups", group, rows, precision, flush=True)
+    ens = Ensemble(_solver(precision), [_solution(mx, my, 7 + k)
+                                        for k, (mx, my) in enumerate(sizes)])
+    ens._prepare(rows)
+    ens._waves[2] = group
+    ens.run_steps(5, use_graph=False)
+    ctls = ens.controllers()
+    for k, (mx, my) in enumerate(sizes):
+        solver, sol = _solver(precision), _solution(mx, my, 7 + k)
+        solver.dt = solver.dt_initial
+        solver.run_steps(sol, 5)
+        assert ctls[k].attempts == 5 and ctls[k].t == sol.t, k
+        assert np.array_equal(ens.member_q(k), sol.state.q), (k, (mx, my))
