@@ -25,6 +25,7 @@
 // array, so that a direction's results are read while they are cached.  Bound:
 // HBM, by the work array's write and its 27-fold gather; the path exists for
 // parity with ClawSolver3D's unsplit default, the split step is the fast 3D path.
+#include <algorithm>
 #include <type_traits>
 
 #include "launch.hpp"
@@ -294,7 +295,7 @@ __global__ void __launch_bounds__(256) k_flux3(const Step3Args<double> a) {
 // One slice's update of a cell at transverse offsets (DA, DB) from the slice
 // (step3.f90:189-225 and the y / z equivalents): v is the cell's running value,
 // wk field m's qadd of the slice (uniform), at the cell's byte offset in it (32
-// bits: a component of a work array that fits in memory is under 4 GB).
+// bits: launch_step3 refuses a component of 4 GB).
 template <int ME, int DA, int DB>
 __device__ __forceinline__ double term3(double v, const double* wk, long long st, unsigned at,
                                         double dtn, double dt1, double dt2) {
@@ -391,10 +392,20 @@ void launch_apply3(const Step3Args<double>& a, hipStream_t stream) {
 }
 }  // namespace
 
+namespace {
+// Elements of a component of each direction's slice results.
+void step3_strides(int mx, int my, int mz, long long (&s)[3]) {
+  s[0] = (long long)(mx + 1) * (my + 2) * (mz + 2);
+  s[1] = (long long)(my + 1) * (mz + 2) * (mx + 2);
+  s[2] = (long long)(mz + 1) * (mx + 2) * (my + 2);
+}
+}  // namespace
+
+// The directions take the work array in turn: the largest one's results.
 long long step3_work_elems(int meqn, int mx, int my, int mz) {
-  const long long per = 14LL * meqn;
-  return per * ((long long)(mx + 1) * (my + 2) * (mz + 2) + (long long)(my + 1) * (mz + 2) *
-                (mx + 2) + (long long)(mz + 1) * (mx + 2) * (my + 2));
+  long long s[3];
+  step3_strides(mx, my, mz, s);
+  return 14LL * meqn * std::max({s[0], s[1], s[2]});
 }
 
 int launch_step3(const clawhip_rp& rp, const void* q_in, const Geom& gin, void* q_out,
@@ -417,12 +428,14 @@ int launch_step3(const clawhip_rp& rp, const void* q_in, const Geom& gin, void* 
   a.qout = (double*)q_out;
   a.cfl_bits = cfl;
   const int mx = gin.mx, my = gin.my, mz = gin.mz;
-  const long long s1 = (long long)(mx + 1) * (my + 2) * (mz + 2);
-  const long long s2 = (long long)(my + 1) * (mz + 2) * (mx + 2);
-  const long long s3 = (long long)(mz + 1) * (mx + 2) * (my + 2);
+  long long stride[3];
+  step3_strides(mx, my, mz, stride);
+  // k_apply3 addresses a component with 32 bits (state and work array together are then
+  // beyond any device's memory)
+  if (std::max({stride[0], stride[1], stride[2]}) * (long long)sizeof(double) >= 1LL << 32)
+    return CLAWHIP_E_ARG;
   // the directions share the work array (the entry point refuses q_out == q_in,
   // so all of them read the old state); each adds its slices to the sum so far
-  const long long stride[3] = {s1, s2, s3};
   Geom go = gin;
   go.g = 0; go.rs = mx; go.ss = (long long)mx * my; go.fs = go.ss * mz;
   Step3Args<double> d[3] = {a, a, a};

@@ -46,6 +46,16 @@ def test_mlp_param_count():
     assert L.lib().clawhip_mlp_param_count() == 16 * 32 + 32 * 32 + 32 + 32 + 1
 
 
+@pytest.mark.parametrize("mx,my,mz", [(96, 64, 80), (2, 3, 300), (300, 3, 2), (7, 300, 2),
+                                      (300, 300, 300)])
+def test_step3_work_is_one_direction_at_a_time(mx, my, mz):
+    """The unsplit 3D step's directions use one work region in turn: 14 values per field,
+    slice (ghost slices included) and position 1..n+1 of the largest direction."""
+    n = (mx, my, mz)
+    slices = [14 * 5 * (n[d] + 1) * (n[d - 1] + 2) * (n[d - 2] + 2) for d in range(3)]
+    assert L.lib().clawhip_step3_unsplit_work_elems(5, mx, my, mz) == max(slices)
+
+
 def test_missing_library_raises(monkeypatch, tmp_path):
     monkeypatch.setattr(L, "_lib", None)
     monkeypatch.setattr(L, "LIB_PATH", str(tmp_path / "libclawhip.so"))

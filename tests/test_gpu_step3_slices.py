@@ -1,7 +1,8 @@
 """The unsplit 3D step lays its slices end to end over the wavefronts
 (unsplit3.hip k_flux3): slice lengths around a wavefront's 60 owned cells and far
 below them, one slice ending anywhere in a wavefront, in each direction, bit for
-bit against the oracle; and the step with its output in its input's place."""
+bit against the oracle and within the work array; a step onto its own input, which the
+directions would read back half done, is refused."""
 import numpy as np
 import pytest
 import torch
@@ -31,7 +32,21 @@ def test_step3_slices_bit_exact(shape):
     qi = q_to_device(q)
     out = torch.empty_like(qi)
     cfl = torch.zeros(1, dtype=torch.float64, device="cuda")
-    K.step3_unsplit(rp, qi, out, cfl, bcl, bcu, [1, 2, 3], meth, [4] * 3, dx, dy, dz, dt)
+    n = int(K.L.lib().clawhip_step3_unsplit_work_elems(5, *shape))
+    work = torch.full((n + 512,), -1.5, dtype=torch.float64, device="cuda")
+    K.step3_unsplit(rp, qi, out, cfl, bcl, bcu, [1, 2, 3], meth, [4] * 3, dx, dy, dz, dt,
+                    work=work[:n])
     torch.cuda.synchronize()
+    assert bool((work[n:] == -1.5).all())
     assert np.array_equal(q_from_device(out), O.interior(ref, ng))
     assert float(cfl.item()) == c_ref
+
+
+def test_step3_onto_its_input_is_refused():
+    from pyclaw_amd import kernels as K
+    from pyclaw_amd.device import q_to_device
+    qi = q_to_device(seeded_state(np.random.default_rng(1), O.EULER3, (4, 5, 6)))
+    cfl = torch.zeros(1, dtype=torch.float64, device="cuda")
+    with pytest.raises(K.L.ClawhipError):
+        K.step3_unsplit(K.make_rp(5, {"gamma": 1.4}), qi, qi, cfl, [1] * 3, [1] * 3, [1, 2, 3],
+                        [1, 2, 22, 0, 0, 0, 0], [4] * 3, 0.25, 0.2, 0.2, 0.01)
