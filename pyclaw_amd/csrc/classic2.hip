@@ -1,8 +1,8 @@
 // classic2.hip -- 2D classic Clawpack unsplit wave-propagation step for gfx950:
 // one fused kernel per step (unsplit.hpp: x- and y-slices of classic/step2.f90
 // with flux2.f90, limiter.f90, philim.f90, the ghost fill as an index map and
-// the CFL max-reduction), plus the device-controlled variant that applies
-// Solver.evolve_to_time's accept/reject and next dt in its last wavefront.
+// the CFL max-reduction), plus the device-controlled variant, with a one-wavefront
+// kernel after it that applies Solver.evolve_to_time's accept/reject and next dt.
 //
 // A fused kernel was measured against a two-launch form (an x-sweep into a work
 // array, then a y-sweep): on 1024^2 Euler FP64 the fused kernel takes 162 us,

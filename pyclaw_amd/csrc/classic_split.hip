@@ -219,6 +219,15 @@ __device__ __forceinline__ long long cell_off(const Geom& g, int i, int s, int p
   return (long long)(i - 1 + g.g) + (long long)(j - 1 + g.g) * g.rs + (long long)(k - 1 + g.g) * g.ss;
 }
 
+// Wavefronts per SIMD a march is compiled for, where that differs from the
+// compiler's choice: FP64 euler_3D sits 4 registers above the 256 of 2 per SIMD
+// and fits them without spills (210x170x190 step 1.07 -> 0.95 ms).  FP32 + Kahan
+// euler_3D (141, 15 spilled at the 128 of 4 per SIMD) loses 4 % there.
+template <class RS>
+struct SplitMarchWaves { static constexpr int value = 1; };
+template <>
+struct SplitMarchWaves<Euler3<double>> { static constexpr int value = 2; };
+
 // A wavefront marches H rows of a 64-column strip of one pencil plane.  The next
 // row is loaded one iteration before its use, the compensation of the row being
 // stored at the top of its iteration.
@@ -232,15 +241,6 @@ __device__ __forceinline__ long long cell_off(const Geom& g, int i, int s, int p
 // split step takes 1.04 instead of 1.33 ms there (FP64; 0.82 with the shared
 // reciprocals) and 4.13 instead of 5.24 ms at 384^3 (FP32 + Kahan; 3.04 with
 // k_xysweep).
-// Wavefronts per SIMD a march is compiled for, where that differs from the
-// compiler's choice: FP64 euler_3D sits 4 registers above the 256 of 2 per SIMD
-// and fits them without spills (210x170x190 step 1.07 -> 0.95 ms).  FP32 + Kahan
-// euler_3D (141, 15 spilled at the 128 of 4 per SIMD) loses 4 % there.
-template <class RS>
-struct SplitMarchWaves { static constexpr int value = 1; };
-template <>
-struct SplitMarchWaves<Euler3<double>> { static constexpr int value = 2; };
-
 template <class RS, typename T, bool KAHAN, int AXIS, bool HALF_IN_SUM>
 __global__ void __launch_bounds__(256)
     __attribute__((amdgpu_waves_per_eu(SplitMarchWaves<RS>::value))) k_march(const SweepArgs<T> a) {

@@ -195,20 +195,6 @@ __device__ __forceinline__ void from_right(const T (&v)[N], T (&o)[N]) {
 template <typename T>
 __device__ __forceinline__ T cfl_term(T acc, T v) { return v > acc ? v : acc; }
 
-// Wave-wide max of a lane's Courant number, then one atomic per wave.  Values
-// that are not >= 0 (a NaN) count as 0, so the result does not depend on which
-// lane held them.  Ordering of non-negative IEEE doubles equals the ordering of
-// their bit patterns.
-__device__ __forceinline__ void wave_atomic_max(double v, unsigned long long* dst) {
-  if (!(v >= 0.0)) v = 0.0;
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    double o = __shfl_xor(v, off, 64);
-    v = o > v ? o : v;
-  }
-  if ((threadIdx.x & 63) == 0 && v > 0.0) atomicMax(dst, (unsigned long long)__double_as_longlong(v));
-}
-
 // Each XCD takes a contiguous range of the blocks (the dispatcher deals them out
 // in turn over 8 XCDs), so that neighbouring blocks meet in one L2.
 __device__ __forceinline__ long long xcd_block() {
@@ -216,8 +202,11 @@ __device__ __forceinline__ long long xcd_block() {
   return (long long)x * per + min(x, rest) + i;
 }
 
-// The same for a workgroup of up to 256 threads: one atomic per workgroup.
-// Every thread of the workgroup calls it (it holds a barrier).
+// Max of a lane's Courant number over a workgroup of up to 256 threads, then one
+// atomic.  Every thread of the workgroup calls it (it holds a barrier).  Values that
+// are not >= 0 (a NaN) count as 0, so the result does not depend on which lane held
+// them.  Ordering of non-negative IEEE doubles equals the ordering of their bit
+// patterns.
 __device__ __forceinline__ void block_atomic_max(double v, unsigned long long* dst) {
   __shared__ double part[256 / 64];
   if (!(v >= 0.0)) v = 0.0;

@@ -88,7 +88,7 @@ struct SharpArgs {
   T* recon;                     //   their full-WENO5 edge values, 2*meqn per interface id
   // device-controlled stage (ctl non-null): it runs while *gate != 0, takes dt
   // from ctl and the pointers named in `res` from the state's two buffers by
-  // ctl->cur; its last wavefront applies phase ctl_phase; with count_bad it
+  // ctl->cur; k_sharp_ctl after it applies phase ctl_phase; with count_bad it
   // counts the stored cells whose fields in pos_mask are not > 0 (or not finite)
   SharpCtl* ctl;
   const int* gate;

@@ -736,10 +736,14 @@ class SharpClawSolver(Solver):
 
     def _captured(self, n):
         """Whether n attempts are launched as a captured graph: a whole chunk.  A
-        rest is launched as it is: an attempt's dozen launches take the host less
-        time than the GPU, and a graph for every rest before an indicator audit
-        (13 sizes for runs of 16 attempts) was captured at about 7 ms each: 16
-        attempts at 2048^2 took 13.2 ms on average instead of 6.5."""
+        rest is launched as it is: an attempt's dozen launches take the host no
+        longer than the GPU, also on small grids, and a graph for every rest
+        before an indicator audit (13 sizes for runs of 16 attempts) was captured
+        at 7 to 20 ms each: 16 attempts at 2048^2 took 13.2 ms on average instead
+        of 6.5.  Runs of 1 / 15 attempts as launched and as a graph's replay, us:
+        FP64 48^2 126 / 1084 and 131 / 1062, 512^2 190 / 2034 and 205 / 2047,
+        2048^2 1276 / 18011 and 1377 / 17874; FP32 with the indicator 48^2 151 /
+        1240 and 151 / 1170, 2048^2 402 / 5282 and 419 / 5263."""
         return self.use_graph and n == self.graph_chunk
 
     def _chunk_sizes(self, nsteps):
