@@ -190,10 +190,10 @@ __device__ __forceinline__ void cfl_y(const UnsplitArgs<T>& a, T& acc, const T (
   if constexpr (CAPA) {
     const T dlo = dy1d<CAPA>(a, Alo), dhi = dy1d<CAPA>(a, Ahi);
 #pragma unroll
-    for (int w = 0; w < MW; w++) acc = dmax(dmax(acc, dhi * s[w]), -(dlo * s[w]));
+    for (int w = 0; w < MW; w++) acc = cfl_term(cfl_term(acc, dhi * s[w]), -(dlo * s[w]));
   } else {
 #pragma unroll
-    for (int w = 0; w < MW; w++) acc = dmax(acc, fabs(s[w]));
+    for (int w = 0; w < MW; w++) acc = cfl_term(acc, T(fabs(s[w])));
   }
 }
 

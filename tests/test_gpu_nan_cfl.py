@@ -57,3 +57,36 @@ def test_nan_cell_courant_numbers_match_oracle():
         K.sharp2_stage(rp, cd, out, cfl, [1, 1], [1, 1], [1, 2], dt, dx, dy, qi)
         torch.cuda.synchronize()
         assert float(cfl.item()) == cref, (cd, float(cfl.item()), cref)
+
+
+@pytest.mark.parametrize("jet,nan", [((1, 4), 7), ((1, 8), 9), ((20, 24), 27), ((30, 36), 39)])
+def test_nan_cell_past_a_jet_along_y(jet, nan, monkeypatch):
+    """The unsplit step's marches run along y: a NaN cell after a jet v = 4 in the same
+    column (and, with ten rows a wavefront, in the same wavefront) leaves the
+    jet's Courant number as it is."""
+    from pyclaw_amd import kernels as K
+    from pyclaw_amd.device import q_from_device, q_to_device
+    monkeypatch.setenv("CLAWHIP_UNSPLIT_ROWS", "11")   # one block of 41 solves
+    mx, my, i = 12, 40, 5
+    v = np.zeros((mx, my))
+    v[i, jet[0]:jet[1]] = 4.0
+    q = np.zeros((4, mx, my), order="F")
+    q[0], q[2], q[3] = 1.0, v, 1.0 / 0.4 + 0.5 * v * v
+    q[:, i, nan - 1] = np.nan
+    dx, dy = 1.0 / mx, 1.0 / my
+    dt = 0.1 * dy
+    for trans in (0, 2):
+        meth = O.method_array(transverse=trans)
+        qbc = O.with_ghosts(q, 2)
+        O.bc2(qbc, 2, [1, 1], [1, 1])
+        ref = qbc.copy(order="F")
+        c = O.step2(O.make_rp(O.EULER, efix=1, gamma=1.4), qbc, ref, 2, dx, dy, dt, meth, [4] * 4)
+        assert c > 0.4   # the jet's: 0.1 (4 + c)
+        qi = q_to_device(q)
+        qo = torch.empty_like(qi)
+        cfl = torch.zeros(1, dtype=torch.float64, device="cuda")
+        K.step2_unsplit(K.make_rp(O.EULER, {"gamma": 1.4}), qi, qo, cfl, [1, 1], [1, 1], [1, 2],
+                        meth, [4] * 4, dx, dy, dt)
+        torch.cuda.synchronize()
+        assert float(cfl.item()) == c
+        assert np.array_equal(q_from_device(qo), O.interior(ref, 2), equal_nan=True)
