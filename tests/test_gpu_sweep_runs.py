@@ -13,13 +13,19 @@ from tests._cases import seeded_state
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("my", [2, 3, 4, 5, 7, 8, 9, 16, 17, 33])
-def test_split3_runs_bit_exact(my):
+EXTRAP = ([1, 1, 1], [1, 1, 1])
+SIDES3 = [([2, 2, 2], [2, 2, 2]), ([3, 3, 3], [3, 3, 3]), ([1, 3, 2], [3, 1, 2]),
+          ([2, 1, 3], [2, 3, 1])]
+
+
+@pytest.mark.parametrize("my,sides", [(my, EXTRAP) for my in (2, 3, 4, 5, 7, 8, 9, 16, 17, 33)]
+                         + [(my, s) for my in (2, 5, 8, 17) for s in SIDES3])
+def test_split3_runs_bit_exact(my, sides):
     from pyclaw_amd import kernels as K
     from pyclaw_amd.device import q_from_device, q_to_device
     mx, mz, ng = 67, my + 2, 2
     print("split3 runs", (mx, my, mz), flush=True)
-    bcl, bcu = [1, 1, 1], [1, 1, 1]
+    bcl, bcu = sides
     q = seeded_state(np.random.default_rng(my), O.EULER3, (mx, my, mz))
     meth = O.method_array(dimensional_split=True)
     dx, dy, dz = 1.0 / mx, 0.9 / my, 1.1 / mz
@@ -40,12 +46,13 @@ def test_split3_runs_bit_exact(my):
     assert float(cfl.item()) == max(cs)
 
 
+@pytest.mark.parametrize("sides", [([1, 1], [1, 1]), ([2, 3], [2, 1])])
 @pytest.mark.parametrize("mx,my", [(3, 2), (64, 2), (61, 3), (200, 37), (5, 130), (130, 1030)])
-def test_split2_runs_bit_exact(mx, my):
+def test_split2_runs_bit_exact(mx, my, sides):
     """Both forms of the 2D y sweep: out of place, and in place on a whole qbc."""
     from pyclaw_amd import kernels as K
     from pyclaw_amd.device import q_from_device, q_to_device
-    ng, bcl, bcu = 2, [1, 1], [1, 1]
+    ng, (bcl, bcu) = 2, sides
     print("split2 runs", (mx, my), flush=True)
     q = seeded_state(np.random.default_rng(mx + my), O.SHALLOW, (mx, my))
     meth = O.method_array(dimensional_split=True)
@@ -107,3 +114,29 @@ def test_split3_fp32_one_pass_xy(mx, my, mz):
     bound = 3 * 50 * 4 * max(cs) * 2.0 ** -24 * np.abs(start).max()
     assert np.abs(out - O.interior(qbc, ng)).max() <= bound
     assert abs(float(cfl.item()) - max(cs)) <= 50 * 2.0 ** -24 * max(cs)
+
+
+@pytest.mark.parametrize("sides", [EXTRAP] + SIDES3)
+@pytest.mark.parametrize("mx,my,mz", [(60, 2, 3), (61, 3, 2), (121, 9, 5), (2, 37, 4), (7, 130, 3)])
+def test_split3_fp32_carries_the_compensation(mx, my, mz, sides):
+    """With dt = 0 the three sweeps of the FP32 + Kahan step change nothing, so the state
+    less its compensation (varying from cell to cell, far above the rounding of the
+    steps) comes out as it went in: each sweep adds -comp to q and keeps what the sum
+    lost, exactly where |q| >= |comp|, within half a unit of comp elsewhere."""
+    from pyclaw_amd import kernels as K
+    from pyclaw_amd.device import q_from_device, q_to_device
+    print("split3 compensation", (mx, my, mz), sides, flush=True)
+    rng = np.random.default_rng(mx + my + mz)
+    q = seeded_state(rng, O.EULER3, (mx, my, mz)).astype(np.float32)
+    comp = rng.uniform(-1e-3, 1e-3, q.shape).astype(np.float32)
+    qi = q_to_device(np.asfortranarray(q.astype(np.float64)), 1)
+    ci = q_to_device(np.asfortranarray(comp.astype(np.float64)), 1)
+    qo, co = torch.empty_like(qi), torch.empty_like(ci)
+    cfl = torch.zeros(1, dtype=torch.float64, device="cuda")
+    K.step3_split(K.make_rp(5, {"gamma": 1.4}), qi, qo, cfl, *sides, [1, 2, 3],
+                  O.method_array(dimensional_split=True), [4] * 3, 0.1, 0.1, 0.1, 0.0,
+                  comp_in=ci, comp_out=co)
+    torch.cuda.synchronize()
+    out = q_from_device(qo.double()) - q_from_device(co.double())
+    before = q.astype(np.float64) - comp.astype(np.float64)
+    assert np.abs(out - before).max() <= 3 * 2.0 ** -24 * np.abs(comp).max()
