@@ -165,7 +165,10 @@ __device__ __forceinline__ T weno_char_side(T hm2, T hm1, T h0, T hp1, T hp2, in
   T a2 = im == 1 ? hm2 : hp2;   // hh(intwo)
   T a1 = im == 1 ? hm1 : hp1;   // hh(inone)
   T b1 = im == 1 ? hp1 : hm1;   // hh(ione)
-  const T eps = weno_eps_char<T>();
+  // FP32 takes the squares at a 16th, so that no reciprocal below leaves the normal
+  // numbers before its quotient does (see quo)
+  constexpr T fourth = sizeof(T) == 4 ? T(0.25) : T(1);
+  const T eps = fourth * weno_eps_char<T>();
   T fim = T(im);
   T t1 = fim * (a2 - a1);
   T t2 = fim * (a1 - h0);
@@ -173,17 +176,18 @@ __device__ __forceinline__ T weno_char_side(T hm2, T hm1, T h0, T hp1, T hp2, in
   T e1 = a2 - T(3) * a1;
   T e2 = a1 + h0;
   T e3 = T(3) * h0 - b1;
-  T tt1 = T(13) * (t1 * t1) + T(3) * (e1 * e1);
-  T tt2 = T(13) * (t2 * t2) + T(3) * (e2 * e2);
-  T tt3 = T(13) * (t3 * t3) + T(3) * (e3 * e3);
+  T tt1 = (T(13) * fourth) * (t1 * t1) + (T(3) * fourth) * (e1 * e1);
+  T tt2 = (T(13) * fourth) * (t2 * t2) + (T(3) * fourth) * (e2 * e2);
+  T tt3 = (T(13) * fourth) * (t3 * t3) + (T(3) * fourth) * (e3 * e3);
   tt1 = (eps + tt1) * (eps + tt1);
   tt2 = (eps + tt2) * (eps + tt2);
   tt3 = (eps + tt3) * (eps + tt3);
   T s1, s3;
   if constexpr (sizeof(T) == 4) {
     // the same weights as d_k / (eps + beta_k)^2: no fourth powers to underflow
-    const T r1 = quo(T(1), tt1), r2 = T(6) / tt2, r3 = T(3) / tt3;
-    const T t0 = quo(T(1), r1 + r2 + r3);   // the sum is at most 10 / eps^2 = 1e37
+    // (1, 6 and 3 over them); the sum is at most 10 / eps^2 = 1e37
+    const T r1 = quo(T(1. / 16.), tt1), r2 = quo(T(6. / 16.), tt2), r3 = quo(T(3. / 16.), tt3);
+    const T t0 = quo(T(1), r1 + r2 + r3);
     s1 = r1 * t0;
     s3 = r3 * t0;
   } else {   // the reference's products of two squares, bit for bit
