@@ -145,8 +145,8 @@ __global__ void __launch_bounds__(256) k_xsweep(const SweepArgs<T> a) {
       typename RS::Roe roe;
       Watch<RS, T> seen;
       seen.see(Q);
-      const bool wide = watched<RS, T>() && (a.rp.wide || !seen.all_tame());
-      rpn_either<RS, 1>(a.rp, wide, QL, Q, AL, A, W, s, am, ap, roe);
+      int way = a.rp.wide ? kPlain : seen.way();
+      rpn_either<RS, 1>(a.rp, way, QL, Q, AL, A, W, s, am, ap, roe);
       T smax = T(0);
       if (lane >= 1 && c >= 1 && c <= mx + 1) {
 #pragma unroll
@@ -311,21 +311,21 @@ __global__ void __launch_bounds__(256)
     load_aux(j0 - 2, Am);
     load_aux(j0 - 1, A0);
     load_aux(j0, A1);
-    // uniform: a value read so far needs the plain division (see Divided)
+    // uniform: as the values read so far need it
     Watch<RS, T> seen;
     seen.see(Qm); seen.see(Q0); seen.see(Q1);
-    bool wide = watched<RS, T>() && (a.rp.wide || !seen.all_tame());
+    int way = a.rp.wide ? kPlain : seen.way();
     T Wt[MW][ME], st[MW], amt[ME], apt[ME], dotl[MW];
     Roe roet;
     {
       T Wp[MW][ME], sp[MW], amp[ME], app[ME];
       Roe roep;
-      rpn_either<RS, IXY>(a.rp, wide, Qm, Q0, Am, A0, Wp, sp, amp, app, roep);
+      rpn_either<RS, IXY>(a.rp, way, Qm, Q0, Am, A0, Wp, sp, amp, app, roep);
       if (j0 - 1 >= 1) {
 #pragma unroll
         for (int w = 0; w < MW; w++) smax = cfl_term(smax, fabs(sp[w]));
       }
-      rpn_either<RS, IXY>(a.rp, wide, Q0, Q1, A0, A1, Wt, st, amt, apt, roet);
+      rpn_either<RS, IXY>(a.rp, way, Q0, Q1, A0, A1, Wt, st, amt, apt, roet);
 #pragma unroll
       for (int w = 0; w < MW; w++) smax = cfl_term(smax, fabs(st[w]));
       wave_dots<ME, MW>(Wp, Wt, dotl);
@@ -339,8 +339,11 @@ __global__ void __launch_bounds__(256)
     for (int t = j0; t <= jend; t++) {
 #pragma unroll
       for (int m = 0; m < ME; m++) Q1[m] = Qn[m];
-      seen.see(Q1);
-      if (watched<RS, T>()) wide = wide || !seen.all_tame();   // to the run's end
+      {
+        Watch<RS, T> row;
+        row.see(Q1);
+        way = max(way, row.way());   // to the run's end
+      }
       if (inplace && t + 2 >= jend) {   // rows jend, jend+1 belong to the next run
 #pragma unroll
         for (int m = 0; m < ME; m++) Qn[m] = t + 2 == jend ? U0[m] : U1[m];
@@ -357,7 +360,7 @@ __global__ void __launch_bounds__(256)
       load_aux(t + 1, A1);
       T Wn[MW][ME], sn[MW], amn[ME], apn[ME], dotn[MW];
       Roe roen;
-      rpn_either<RS, IXY>(a.rp, wide, Q0, Q1, A0, A1, Wn, sn, amn, apn, roen);
+      rpn_either<RS, IXY>(a.rp, way, Q0, Q1, A0, A1, Wn, sn, amn, apn, roen);
       if (t + 1 <= m_ax + 1) {
 #pragma unroll
         for (int w = 0; w < MW; w++) smax = cfl_term(smax, fabs(sn[w]));

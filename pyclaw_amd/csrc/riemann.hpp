@@ -68,18 +68,24 @@ struct RPParams {
 // spent half their cycles on them (1024^2 Euler step 128 -> 119 us, 2048^2 shallow-
 // water WENO5 stage 465 -> 398, 210x170x190 euler_3D step 0.99 -> 0.82 ms).
 // WIDE = true, and every type but double: the plain division and sqrt.  The
-// reference-equal FP64 kernels take it where a state has a value beyond 2^40 or
-// a nonzero one below 2^-320 (Watch; decaying tails reach denormals): a
-// march with several solves a row starts again at that row with the plain division
-// (march_both), the split sweeps go on with it.
-// Why there: numerators hold products of two small values (a velocity times a jump,
-// v d2 in a Roe solve's a3, where the other terms are zero).  A jump of values in
-// [2^-L, 2^U) is 0 or at least 2^-(L+52), an averaged velocity over the sound speed
-// at least 2^-(L+U+53), their product in a sum of such terms at least
-// 2^-(2L+U+157); a parameter (within 2^+-60) takes 30 more.  The classic steps have
-// L = 320: 2^-867.  WENO5 makes edge values as small as eps^2 / M^3 of a zero region
-// beside a jump M < 2^41: L = 362, 2^-951.  Only a product of three small values, where
-// those of two cancel, may lie below: its quotient's last bit can differ.
+// reference-equal FP64 kernels take it where a state leaves the bounds of Watch
+// (decaying tails reach denormals): a march with several solves a row starts again at
+// that row with the plain division (march_both), the split sweeps go on with it.
+// The bounds: densities, depths and energies in (2^-100, 2^100), the other fields zero
+// or in (2^-800, 2^100), parameters within 2^+-60.  Then the averages' numerators, sums
+// of one such field over or times a root, are zero or above 2^-930 with all that can
+// cancel; squares of momenta below 2^-960 are divided, but vanish beside the energy
+// they are taken from; the edge values that WENO5 gives a zero region beside a jump M,
+// eps^2 / M^3, are above 2^-540.  Only the numerator of the Euler solvers' strength a4
+// holds products of two small values (v d2, where the jumps of density, normal momentum
+// and energy are zero).  A jump is zero or above 2^-(L+52) for values in 2^-L .. 2^U, an
+// averaged velocity over the sound speed above 2^-(L+U+53), their product in a sum above
+// 2^-(2L+U+157), with a parameter 2^-(2L+U+187): the Euler solvers are held to the
+// narrower 2^-320 and 2^40 (with WENO5's edges L = 362 and 2^-951).  Only a product of
+// three small values, where those of two cancel, may lie lower: its quotient's last bit
+// can differ.  Between the bounds the split sweeps look for such a jump instead
+// (rpn_either, shear_alone): a blast into gas at rest has such momenta about it (384^3
+// split step 6.1 ms, with the plain division there 6.95).
 
 // a / b: FP32 by the hardware reciprocal, as the build's FP32 division (about 1 ulp),
 // without its scaling of denominators above 2^96 (compare, select and two
@@ -146,22 +152,33 @@ __device__ __forceinline__ T root(T x) {
 template <class RS, typename T>
 constexpr bool watched() { return RS::shares && sizeof(T) == 8 && CLAW_FAST == 0; }
 
-// The magnitudes of the values a lane has met: tame() while all are zero or in
-// (2^-320, 2^40) (not NaN).  Kept as the smallest and largest of the words that
-// hold a value's exponent and leading digits (doubled, which drops the sign; a
-// zero, less one, is the largest), so that watching costs no branch.
+// A wavefront's kind of division: shared reciprocals, the same with a look for the jumps
+// that they may not do for, plain.
+enum { kShared = 0, kLooked = 1, kPlain = 2 };
+
+// A value's exponent and leading digits, doubled, which drops the sign, and less one,
+// which makes a zero the largest.
+__device__ __forceinline__ unsigned small_word(double x) {
+  const unsigned long long b = __builtin_bit_cast(unsigned long long, x);
+  const unsigned low = (unsigned)b;
+  return (((unsigned)(b >> 32) << 1) | (low < 1u ? low : 1u)) - 1u;
+}
+
+// The magnitudes of the values a lane has met: tame() while all are within the bounds
+// above (not NaN).  Kept as the smallest word of the densities, depths and energies,
+// that of the other fields, and the largest (of a zero: 0), so that watching costs no
+// branch.
 template <class RS, typename T>
 struct Watch {
-  unsigned least = ~0u, most = 0u;
+  unsigned least = ~0u, least_other = ~0u, most = 0u;
   template <int ME>
   __device__ __forceinline__ void see(const T (&q)[ME]) {
     if constexpr (watched<RS, T>()) {
 #pragma unroll
       for (int m = 0; m < ME; m++) {
-        const unsigned long long b = __builtin_bit_cast(unsigned long long, q[m]);
-        const unsigned low = (unsigned)b;
-        const unsigned u = ((unsigned)(b >> 32) << 1) | (low < 1u ? low : 1u);
-        least = least < u - 1u ? least : u - 1u;
+        const unsigned w = small_word(q[m]), u = w + 1u;
+        if (m == 0 || m == RS::energy) least = least < w ? least : w;
+        else least_other = least_other < w ? least_other : w;
         most = most > u ? most : u;
       }
     }
@@ -171,7 +188,25 @@ struct Watch {
     return !watched<RS, T>() || __ballot(!tame()) == 0ull;
   }
   __device__ __forceinline__ bool tame() const {
-    return least >= 2u * 0x2bf00000u && most < 2u * 0x42700000u;
+    if constexpr (watched<RS, T>()) return within<RS::numerator>();
+    else return true;
+  }
+  // how the split sweeps divide (rpn_either)
+  __device__ __forceinline__ int way() const {
+    if constexpr (watched<RS, T>()) {
+      if (__builtin_expect(__ballot(!tame()) == 0ull, 1)) return kShared;
+      if (RS::numerator && __ballot(!within<false>()) == 0ull) return kLooked;
+      return kPlain;
+    } else {
+      return kShared;
+    }
+  }
+
+ private:
+  template <bool NARROW>
+  __device__ __forceinline__ bool within() const {
+    return least >= 2u * 0x39b00000u && least_other >= 2u * (NARROW ? 0x2bf00000u : 0x0df00000u) &&
+           most < 2u * (NARROW ? 0x42700000u : 0x46300000u);
   }
 };
 
@@ -236,7 +271,16 @@ template <typename T, int TR>
 struct EulerT {
   static constexpr int meqn = 4 + TR, mwaves = 4 + TR, maux = 0;
   static constexpr bool shares = true;   // shared denominators: rpn and rpt take WIDE
+  static constexpr int energy = 3;
+  static constexpr bool numerator = true;   // shear_alone
   struct Roe { T u, v, enth, u2v2, a, g1a2, euv, a2r; };   // a2r: reciprocal of 2 a (Divided)
+  // The states differ in the transverse momentum but in none of density, normal
+  // momentum and energy: a4's numerator holds products of small values only.
+  template <int IXY>
+  __device__ static __forceinline__ bool shear_alone(const T* qL, const T* qR) {
+    constexpr int mu = IXY == 1 ? 1 : 2, mv = IXY == 1 ? 2 : 1;
+    return qL[0] == qR[0] && qL[mu] == qR[mu] && qL[3] == qR[3] && qL[mv] != qR[mv];
+  }
   // normal flux; the Roe linearisation gives amdq + apdq = flux(qR) - flux(qL)
   template <int IXY>
   __device__ static __forceinline__ void flux(const RPParams<T>& p, const T* q, T (&f)[meqn]) {
@@ -475,7 +519,8 @@ template <typename T> using Euler5 = EulerT<T, 1>;
 template <typename T>
 struct Shallow {
   static constexpr int meqn = 3, mwaves = 3, maux = 0;
-  static constexpr bool shares = true;
+  static constexpr bool shares = true, numerator = false;
+  static constexpr int energy = 0;   // none
   struct Roe { T u, v, a; };
   // normal flux; the Roe linearisation gives amdq + apdq = flux(qR) - flux(qL)
   template <int IXY>
@@ -619,10 +664,18 @@ struct Advection {
 template <typename T>
 struct Euler3 {
   static constexpr int meqn = 5, mwaves = 3, maux = 0;
-  static constexpr bool shares = true;
+  static constexpr bool shares = true, numerator = true;
+  static constexpr int energy = 4;
   // the interface's Roe averages, kept for the transverse splits (u is the
   // normal velocity, v and w the next two in the cycle x -> y -> z)
   struct Roe { T u, v, w, enth, a, g1a2, euv, u2v2w2, a2r; };   // a2r: reciprocal of 2 a (Divided)
+  // as EulerT's
+  template <int IXY>
+  __device__ static __forceinline__ bool shear_alone(const T* qL, const T* qR) {
+    constexpr int mu = IXY, mv = IXY % 3 + 1, mw = (IXY + 1) % 3 + 1;
+    return qL[0] == qR[0] && qL[mu] == qR[mu] && qL[4] == qR[4] &&
+           (qL[mv] != qR[mv] || qL[mw] != qR[mw]);
+  }
   // IXY = 1, 2, 3 selects x, y, z as the normal direction.
   template <int IXY, bool WIDE>
   __device__ static __forceinline__ void rpn(const RPParams<T>& p, const T* qL, const T* qR,
@@ -841,7 +894,8 @@ struct Euler3 {
 template <typename T>
 struct ShallowHLLE {
   static constexpr int meqn = 3, mwaves = 2, maux = 0;
-  static constexpr bool shares = true;
+  static constexpr bool shares = true, numerator = false;
+  static constexpr int energy = 0;   // none
   struct Roe {};
   // normal flux; the HLL waves give amdq + apdq = flux(qR) - flux(qL)
   template <int IXY>
@@ -1152,12 +1206,20 @@ __device__ __forceinline__ void march_both(bool wide, int first, March march) {
 
 // One normal solve with the wavefront's kind of division.
 template <class RS, int IXY, typename T>
-__device__ __forceinline__ void rpn_either(const RPParams<T>& p, bool wide, const T* qL,
+__device__ __forceinline__ void rpn_either(const RPParams<T>& p, int way, const T* qL,
                                            const T* qR, const T* auxL, const T* auxR,
                                            T (&wave)[RS::mwaves][RS::meqn], T (&s)[RS::mwaves],
                                            T (&amdq)[RS::meqn], T (&apdq)[RS::meqn],
                                            typename RS::Roe& roe) {
-  if (watched<RS, T>() && __builtin_expect(wide, 0))
+  bool plain = false;
+  if constexpr (watched<RS, T>()) {
+    plain = way == kPlain;
+    if constexpr (RS::numerator) {
+      if (__builtin_expect(way == kLooked, 0))
+        plain = __ballot(RS::template shear_alone<IXY>(qL, qR)) != 0ull;
+    }
+  }
+  if (__builtin_expect(plain, 0))
     rpn_call<RS, IXY, true>(p, qL, qR, auxL, auxR, wave, s, amdq, apdq, roe);
   else
     rpn_call<RS, IXY, false>(p, qL, qR, auxL, auxR, wave, s, amdq, apdq, roe);

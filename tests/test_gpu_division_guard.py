@@ -1,7 +1,7 @@
 """Where the FP64 solves' shared reciprocals give way to the plain division
 (riemann.hpp Watch, march_both): products of two small values among the numerators,
-a march that meets the first such value in any of its rows, values above the upper
-bound, parameters out of range.  Bit for bit against the oracle."""
+states that are small as a whole, a march that meets the first value out of bounds in
+any of its rows, parameters out of range.  Bit for bit against the oracle."""
 import numpy as np
 import pytest
 import torch
@@ -82,8 +82,9 @@ def _shear(kind, shape, exponents, rho, rng):
     return np.asfortranarray(q)
 
 
-# squares around the smallest numbers, around 2^-960 and between
-@pytest.mark.parametrize("exponents", [(-162.5, -152.0), (-155.0, -142.0), (-125.0, -94.0)])
+# squares around the smallest numbers, around 2^-960, around 2^-800 and above
+@pytest.mark.parametrize("exponents", [(-162.5, -152.0), (-155.0, -142.0), (-125.0, -117.0),
+                                       (-115.0, -94.0)])
 @pytest.mark.parametrize("rho", [1.0, 1.37])
 @pytest.mark.parametrize("kind", SOLVERS)
 def test_products_of_small_values(kind, rho, exponents):
@@ -96,7 +97,20 @@ def test_products_of_small_values(kind, rho, exponents):
             _equal(_sharp2(kind, q, cd))
 
 
-@pytest.mark.parametrize("exponents", [(-162.5, -152.0), (-155.0, -142.0)])
+@pytest.mark.parametrize("power", [-98, -101, -320, -505, -520])
+@pytest.mark.parametrize("kind", SOLVERS)
+def test_all_fields_small(kind, power):
+    """A state scaled to about 2^power: squares of its momenta over its densities are of its
+    energies' size."""
+    q = np.asfortranarray(2.0 ** power * seeded_state(np.random.default_rng(kind), kind, (66, 23)))
+    grav = 2.0 ** min(-power, 55)
+    for split in (False, True):
+        _equal(_classic2(kind, q, split, grav, 0.05))
+    if kind != O.EULER5:
+        _equal(_sharp2(kind, q, 0, grav, 0.05))
+
+
+@pytest.mark.parametrize("exponents", [(-162.5, -152.0), (-155.0, -142.0), (-125.0, -117.0)])
 def test_products_of_small_values_3d(exponents):
     from pyclaw_amd import kernels as K
     from pyclaw_amd.device import q_from_device, q_to_device
@@ -136,24 +150,29 @@ def test_small_edge_values_beside_a_zero_region(kind, scale):
 
 
 def _one_row(kind, shape, row, what, rng):
-    """An ordinary state but for one row, in half of the columns: its momenta below the
-    lower bound (2^-320 = 4.7e-97), around it or near the smallest numbers; its cells
-    scaled beyond the upper bound (2^40) or around it."""
+    """An ordinary state but for one row, in half of the columns: its momenta below their
+    lower bound (2^-800 = 1.5e-241), around it, around the Euler solvers' (2^-320 =
+    4.7e-97) or near the smallest numbers; its cells scaled beyond the upper bound
+    (2^100), around it, around the Euler solvers' (2^40), or around the lower bound of
+    densities, depths and energies (2^-100)."""
     q = seeded_state(rng, kind, shape)
     if kind in (O.EULER, O.EULER5):   # milder noise keeps edge pressures positive
         mean = seeded_state(np.random.default_rng(0), kind, (1, 1)).mean(axis=(1, 2))
         q = np.asfortranarray(0.85 * mean[:, None, None] + 0.15 * q)
     at = slice(0, shape[0] // 2)
-    if what in ("large", "upper"):
-        q[:, at, row] *= 2.0 ** (205 if what == "large" else 40)
+    powers = {"large": 205, "upper": 100, "middle": 40, "thin": -100}
+    if what in powers:
+        q[:, at, row] *= 2.0 ** powers[what]
     else:
-        size = {"small": 1e-200, "denormal": 1e-315,
-                "lower": 10.0 ** rng.uniform(-98.0, -94.0, q[1:3, at, row].shape)}[what]
+        size = {"small": 1e-250, "denormal": 1e-315,
+                "lower": 10.0 ** rng.uniform(-243.0, -239.0, q[1:3, at, row].shape),
+                "narrow": 10.0 ** rng.uniform(-98.0, -94.0, q[1:3, at, row].shape)}[what]
         q[1:3, at, row] *= size
     return q
 
 
-@pytest.mark.parametrize("what", ["small", "lower", "denormal", "large", "upper"])
+@pytest.mark.parametrize("what", ["small", "lower", "narrow", "denormal", "large", "upper",
+                                  "middle", "thin"])
 @pytest.mark.parametrize("kind", SOLVERS)
 def test_first_such_row_anywhere_in_a_march(kind, what, monkeypatch):
     """Four wavefronts of nine rows each (one block of 35), and marches of nine rows in the

@@ -1,6 +1,6 @@
 """The reference-equal FP64 solves share reciprocals between quotients while a
-wavefront's values lie in (2^-320, 2^40) or are zero, and divide plainly
-otherwise (riemann.hpp Divided).  States whose tails decay through the lower bound
+wavefront's values lie within bounds, and divide plainly otherwise (riemann.hpp
+Divided, Watch).  States whose tails decay through the lower bound of momenta, 2^-800,
 to denormals and zeros, in half of the columns of every row, are stepped bit for bit
 as the oracle does, by every march that chooses (the choice in mid-march and the upper
 bound: test_gpu_division_guard.py).  Acoustics divides plainly whatever the values."""
@@ -14,9 +14,9 @@ from tests.test_gpu_sharp import PD, _orp
 
 pytestmark = pytest.mark.gpu
 
-# decimal exponents of the values' magnitudes: around 2^-320 (4.7e-97), around 2^-700,
+# decimal exponents of the values' magnitudes: around 2^-800 (1.5e-241), around 2^-700,
 # down to the smallest denormal, around 2^200 (the linear solver only)
-RANGES = {"bound": (-99.0, -94.0), "edge": (-213.0, -209.0), "denormal": (-323.5, -190.0),
+RANGES = {"bound": (-243.0, -239.0), "edge": (-213.0, -209.0), "denormal": (-323.5, -190.0),
           "large": (59.0, 61.5)}
 
 
