@@ -83,9 +83,11 @@ struct RPParams {
 // 2^-(2L+U+157), with a parameter 2^-(2L+U+187): the Euler solvers are held to the
 // narrower 2^-320 and 2^40 (with WENO5's edges L = 362 and 2^-951).  Only a product of
 // three small values, where those of two cancel, may lie lower: its quotient's last bit
-// can differ.  Between the bounds the split sweeps look for such a jump instead
-// (rpn_either, shear_alone): a blast into gas at rest has such momenta about it (384^3
-// split step 6.1 ms, with the plain division there 6.95).
+// can differ.  Between the bounds the split sweeps and the unsplit 3D step look for
+// such a jump instead (shear_alone): a blast into gas at rest has such momenta about it
+// (384^3 split step 6.1 ms, with the plain division there 6.95).  In the unsplit 2D
+// march the look cost 1.1 % of every step (1024^2 Euler), for the first hundred steps of
+// a blast (125 after 146 us; then its tails are below either bound): left out.
 
 // a / b: FP32 by the hardware reciprocal, as the build's FP32 division (about 1 ulp),
 // without its scaling of denominators above 2^96 (compare, select and two

@@ -285,8 +285,11 @@ __global__ void __launch_bounds__(256) k_flux3(const Step3Args<double> a) {
     family(std::integral_constant<int, 1>(), cmam, cpam, cmap, cpap, cmcq, cpcq, bmam, bpam,
            bmap, bpap, bmcq, bpcq, dt1);
     };
-    // uniform over the wavefront (see Divided)
-    if (__builtin_expect(!a.rp.wide && seen.all_tame(), 1)) slice(std::false_type());
+    // uniform over the wavefront (see Divided, rpn_either)
+    const int way = a.rp.wide ? kPlain : seen.way();
+    if (__builtin_expect(way == kShared, 1) ||
+        (way == kLooked && __ballot(RS::template shear_alone<DIR>(QL, Q)) == 0ull))
+      slice(std::false_type());
     else slice(std::true_type());
   }
   block_atomic_max(cfl_wave, a.cfl_bits);
