@@ -280,6 +280,10 @@ int launch_unsplit(const clawhip_rp& rp, int dtype, const void* q_in, const Geom
   if (aux.p) return CLAWHIP_E_ARG;
   switch (rp.kind) {
     case CLAWHIP_RP_ACOUSTICS:
+      if (stiff(rp))
+        return dispatch_unsplit<StiffAcoustics>(dtype, rp, q_in, gin, q_out, gout, comp_in,
+                                                comp_out, lo, hi, refl, ng, method, mthlim, dx,
+                                                dy, dt, cfl_bits, stream);
       return dispatch_unsplit<Acoustics>(dtype, rp, q_in, gin, q_out, gout, comp_in, comp_out, lo, hi, refl,
                                          ng, method, mthlim, dx, dy, dt, cfl_bits, stream);
     case CLAWHIP_RP_EULER:
@@ -308,6 +312,9 @@ int launch_unsplit_ctl(const clawhip_rp& rp, int dtype, const Geom& g, const int
                        hipStream_t stream) {
   switch (rp.kind) {
     case CLAWHIP_RP_ACOUSTICS:
+      if (stiff(rp))
+        return dispatch_unsplit_ctl<StiffAcoustics>(dtype, rp, g, lo, hi, refl, ng, method,
+                                                    mthlim, ctl, bufs, nsteps, stream);
       return dispatch_unsplit_ctl<Acoustics>(dtype, rp, g, lo, hi, refl, ng, method, mthlim, ctl,
                                              bufs, nsteps, stream);
     case CLAWHIP_RP_EULER:

@@ -899,6 +899,10 @@ int launch_split2(const clawhip_rp& rp, int dtype, const void* q_in, const Geom&
   }
   switch (rp.kind) {
     case CLAWHIP_RP_ACOUSTICS:
+      if (stiff(rp))
+        return dispatch_split2<StiffAcoustics>(dtype, rp, q_in, gin, q_out, gout, comp_in,
+                                               comp_out, work, cwork, lo, hi, refl, ng, method,
+                                               mthlim, dx, dy, dt, aux, cfl, s);
       return dispatch_split2<Acoustics>(dtype, rp, q_in, gin, q_out, gout, comp_in, comp_out,
                                         work, cwork, lo, hi, refl, ng, method, mthlim, dx, dy,
                                         dt, aux, cfl, s);

@@ -215,7 +215,10 @@ int ensemble_run(const clawhip_rp& rp, int dtype, const void* table_dev, const l
   const EnsHeader* h = (const EnsHeader*)table_dev;
   const EnsMember* m = (const EnsMember*)((const char*)table_dev + ens_members_offset());
   switch (rp.kind) {
-    case CLAWHIP_RP_ACOUSTICS: ens_dispatch<Acoustics>(dtype, h, m, waves, nsteps, s); break;
+    case CLAWHIP_RP_ACOUSTICS:
+      if (stiff(rp)) ens_dispatch<StiffAcoustics>(dtype, h, m, waves, nsteps, s);
+      else ens_dispatch<Acoustics>(dtype, h, m, waves, nsteps, s);
+      break;
     case CLAWHIP_RP_EULER: ens_dispatch<Euler>(dtype, h, m, waves, nsteps, s); break;
     case CLAWHIP_RP_SHALLOW: ens_dispatch<Shallow>(dtype, h, m, waves, nsteps, s); break;
     case CLAWHIP_RP_ADVECTION: ens_dispatch<Advection>(dtype, h, m, waves, nsteps, s); break;

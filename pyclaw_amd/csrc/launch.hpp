@@ -40,6 +40,9 @@ inline long long resident_waves(const void* kernel, int per_simd_cap) {
 
 namespace claw {
 
+// The acoustics solver's denominator 2 zz leaves what FP32's quo does for.
+inline bool stiff(const clawhip_rp& r) { return !(r.zz <= 0x1p125 && r.zz >= -0x1p125); }
+
 template <typename T>
 inline RPParams<T> to_params(const clawhip_rp& r) {
   RPParams<T> p;

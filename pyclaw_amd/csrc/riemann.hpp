@@ -95,9 +95,9 @@ struct RPParams {
 // So only for |a| <= 1 (such a quotient is flushed either way) and for denominators
 // that stay below by what they are: roots and their sums (at most 2^66), and depths (one
 // above 2^126 has overflowed g h^2 in the fluxes, and its velocity, at most 4, is lost
-// against sqrt(g h)).  Written a / b everywhere else (acoustics' impedance among them:
-// 3 % of a 1600^2 FP32 step); limit_waves tests its denominators (wave norms above
-// 2^63).  2048^2 flagged SharpClaw march 85 -> 80 us, 1024^2 Euler step 64 -> 62,
+// against sqrt(g h)).  Written a / b everywhere else; limit_waves tests its
+// denominators (wave norms above 2^63), the launchers the acoustics solver's constant
+// one (stiff).  2048^2 flagged SharpClaw march 85 -> 80 us, 1024^2 Euler step 64 -> 62,
 // ensemble step 2 %.
 template <typename T>
 __device__ __forceinline__ T quo(T a, T b) {
@@ -218,8 +218,11 @@ template <typename T>
 __device__ __forceinline__ T dmin(T a, T b) { return a < b ? a : b; }
 
 // ---------------------------------------------------------------- acoustics
-template <typename T>
-struct Acoustics {
+// STIFF: an impedance zz whose double is beyond 2^126, where quo does not do (FP32).
+// Kernels of their own, as the scaled quotients by the constant take 3 % of a 1600^2
+// FP32 step.
+template <typename T, bool STIFF>
+struct AcousticsT {
   static constexpr int meqn = 3, mwaves = 2, maux = 0;
   // divides plainly: its divisions are few, and watching the values for shared
   // reciprocals costs a 256^2 step 5 % where it gains 4 % at 4096^2
@@ -233,8 +236,9 @@ struct Acoustics {
     const T zz = p.zz, cc = p.cc;
     T delta1 = qR[0] - qL[0];
     T delta2 = qR[mu] - qL[mu];
-    T a1 = (-delta1 + zz * delta2) / (T(2) * zz);
-    T a2 = (delta1 + zz * delta2) / (T(2) * zz);
+    const Divided<T, true, STIFF> z2(T(2) * zz);
+    T a1 = (-delta1 + zz * delta2) / z2;
+    T a2 = (delta1 + zz * delta2) / z2;
     wave[0][0] = -a1 * zz; wave[0][mu] = a1; wave[0][mv] = T(0); s[0] = -cc;
     wave[1][0] = a2 * zz; wave[1][mu] = a2; wave[1][mv] = T(0); s[1] = cc;
 #pragma unroll
@@ -248,8 +252,9 @@ struct Acoustics {
                                              T (&bm)[meqn], T (&bp)[meqn]) {
     constexpr int mu = IXY == 1 ? 1 : 2, mv = IXY == 1 ? 2 : 1;
     const T zz = p.zz, cc = p.cc;
-    T a1 = (-asdq[0] + zz * asdq[mv]) / (T(2) * zz);
-    T a2 = (asdq[0] + zz * asdq[mv]) / (T(2) * zz);
+    const Divided<T, true, STIFF> z2(T(2) * zz);
+    T a1 = (-asdq[0] + zz * asdq[mv]) / z2;
+    T a2 = (asdq[0] + zz * asdq[mv]) / z2;
     bm[0] = cc * a1 * zz; bm[mu] = T(0); bm[mv] = -cc * a1;
     bp[0] = cc * a2 * zz; bp[mu] = T(0); bp[mv] = cc * a2;
   }
@@ -262,6 +267,9 @@ struct Acoustics {
     f[mv] = T(0);
   }
 };
+
+template <typename T> using Acoustics = AcousticsT<T, false>;
+template <typename T> using StiffAcoustics = AcousticsT<T, sizeof(T) == 4>;
 
 // ---------------------------------------------------------------- 2D Euler
 // TR = 0: euler_4wave_2D.  TR = 1: euler_5wave_2D, the same with a passive tracer

@@ -1309,7 +1309,9 @@ int launch_sharp_stage(const clawhip_rp& rp, int dtype, int char_decomp, const G
                 // not finish on the device once, cause not shown, and no later form has run
     case CLAWHIP_RP_EULER5: return dispatch_stage<Euler5, false>(ARGS);
 #endif
-    case CLAWHIP_RP_ACOUSTICS: return dispatch_stage<Acoustics, false>(ARGS);
+    case CLAWHIP_RP_ACOUSTICS:
+      return stiff(rp) ? dispatch_stage<StiffAcoustics, false>(ARGS)
+                       : dispatch_stage<Acoustics, false>(ARGS);
     case CLAWHIP_RP_ADVECTION: return dispatch_stage<Advection, false>(ARGS);
   }
 #undef ARGS
@@ -1343,7 +1345,7 @@ int launch_sharp_ssp33_run(const clawhip_rp& rp, int dtype, int char_decomp, con
 #if CLAW_FAST   // as in launch_sharp_stage
     case CLAWHIP_RP_EULER5: return RUN(Euler5, false);
 #endif
-    case CLAWHIP_RP_ACOUSTICS: return RUN(Acoustics, false);
+    case CLAWHIP_RP_ACOUSTICS: return stiff(rp) ? RUN(StiffAcoustics, false) : RUN(Acoustics, false);
     case CLAWHIP_RP_ADVECTION: return RUN(Advection, false);
   }
 #undef RUN

@@ -109,3 +109,32 @@ def test_weno_weights_of_large_jumps(factor):
     # differences of fluxes g h^2 / 2, of some 20 roundings each
     flux = 0.5 * q[0].max() ** 2
     assert np.abs(got - ref).max() <= 20 * 2.0 ** -24 * flux * dt / dx
+
+
+@pytest.mark.parametrize("form", ["unsplit", "split"])
+@pytest.mark.parametrize("power", [120, 124, 125])
+def test_stiff_acoustics(form, power):
+    """Density and bulk modulus scaled by 2^power scale the impedance and the pressures, and
+    leave the velocities: first-order steps (the squared norms of such waves have no FP32
+    value) of an impedance of 2^(power + 1), whose double is the denominator."""
+    from pyclaw_amd import kernels as K
+    from pyclaw_amd.device import q_from_device, q_to_device
+    mx, my, bc = 67, 21, [1, 2]
+    q = np.random.default_rng(5).uniform(-0.2, 0.2, (3, mx, my)).astype(np.float32)
+    d, dt = [1.0 / mx, 1.0 / my], 0.002
+    outs = []
+    for scale in (1.0, 2.0 ** power):
+        rp = K.make_rp(O.ACOUSTICS, dict(rho=scale, bulk=4.0 * scale, cc=2.0, zz=2.0 * scale))
+        qi = q_to_device(np.asfortranarray(q * np.array([scale, 1.0, 1.0])[:, None, None]), 1)
+        qo, co = torch.empty_like(qi), torch.empty_like(qi)
+        cfl = torch.zeros(1, dtype=torch.float64, device="cuda")
+        meth = O.method_array(order=1, dimensional_split=True) if form == "split" else \
+            O.method_array(order=1, transverse=1)
+        (K.step2_split if form == "split" else K.step2_unsplit)(
+            rp, qi, qo, cfl, bc, bc, [1, 2], meth, [0, 0], *d, dt,
+            comp_in=torch.zeros_like(qi), comp_out=co)
+        torch.cuda.synchronize()
+        outs.append((q_from_device(qo) - q_from_device(co)) / np.array([scale, 1.0, 1.0])[:, None, None])
+    assert np.isfinite(outs[1]).all()
+    # powers of two scale exactly but for a reciprocal scaled on its way (1 ulp)
+    assert np.abs(outs[1] - outs[0]).max() <= 50 * 2.0 ** -23 * np.abs(q).max()
